@@ -18,21 +18,35 @@
 namespace csm {
 namespace {
 
+// The groups' run lookups are independent: issued kNlfIlp at a time, so an entry of up to that many
+// groups costs one round trip.
+constexpr uint32_t kNlfIlp = 4;
+
 __device__ __forceinline__ bool nlf_pass(const DevGraph& g, const NlfEntry& e, const NlfGroup* groups, uint32_t v, int mode) {
-    for (uint32_t k = e.g0; k < e.g1; k++) {
-        const NlfGroup gr = groups[k];
-        uint32_t lo, hi;
-        base_range(g, gr.dir, v, gr.slot, lo, hi);
-        uint32_t deg = hi - lo;
-        if (mode == 0) {
-            const uint4 s = g.delta[gr.dir].seg[v];
-            if (s.y) {
-                uint32_t dlo, dhi;
-                slot_range(g.delta[gr.dir].ins, s.x, s.x + s.y, gr.slot, g.id_bits, dlo, dhi);
-                deg += dhi - dlo;
-            }
+    for (uint32_t k0 = e.g0; k0 < e.g1; k0 += kNlfIlp) {
+        uint32_t lo[kNlfIlp], hi[kNlfIlp];
+#pragma unroll
+        for (uint32_t k = 0; k < kNlfIlp; k++) {
+            lo[k] = hi[k] = 0;
+            if (k0 + k >= e.g1) continue;
+            const NlfGroup gr = groups[k0 + k];
+            base_range(g, gr.dir, v, gr.slot, lo[k], hi[k]);
         }
-        if (deg < gr.count) return false;
+#pragma unroll
+        for (uint32_t k = 0; k < kNlfIlp; k++) {
+            if (k0 + k >= e.g1) continue;
+            const NlfGroup gr = groups[k0 + k];
+            uint32_t deg = hi[k] - lo[k];
+            if (mode == 0 && deg < gr.count) {  // the pending insertions only add
+                const uint4 s = g.delta[gr.dir].seg[v];
+                if (s.y) {
+                    uint32_t dlo, dhi;
+                    slot_range(g.delta[gr.dir].ins, s.x, s.x + s.y, gr.slot, g.id_bits, dlo, dhi);
+                    deg += dhi - dlo;
+                }
+            }
+            if (deg < gr.count) return false;
+        }
     }
     return true;
 }
@@ -56,15 +70,17 @@ __global__ void __launch_bounds__(256) k_nlf_full(DevGraph g, const NlfEntry* en
     }
 }
 
-__global__ void k_nlf_touched(DevGraph g, const NlfEntry* entries, uint32_t n_entries, const NlfGroup* groups,
-                              const uint32_t* touched, const uint32_t* n_touched, int mode) {
-    const uint32_t T = *n_touched;
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < T; i += gridDim.x * blockDim.x) {
-        const uint32_t v = touched[i];
-        const uint32_t vr = g.vrank[v];
-        for (uint32_t e = 0; e < n_entries; e++) {
-            const NlfEntry en = entries[e];
-            if (en.vrank != vr || vr == kNoVertex) continue;
+// One block row per entry (a query vertex): its label's touched vertices, one per thread.  Latency
+// bound: a dependent chain vertex -> directory rows -> delta segment per (vertex, entry) pair of
+// equal label.
+__global__ void __launch_bounds__(256) k_nlf_touched(DevGraph g, const NlfEntry* entries, uint32_t n_entries, const NlfGroup* groups,
+                                                     const uint32_t* by_label, const uint32_t* label_off, int mode) {
+    for (uint32_t e = blockIdx.y; e < n_entries; e += gridDim.y) {
+        const NlfEntry en = entries[e];
+        if (en.vrank == kNoVertex) continue;
+        const uint32_t first = label_off[en.vrank], T = label_off[en.vrank + 1] - first;
+        for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < T; i += gridDim.x * blockDim.x) {
+            const uint32_t v = by_label[first + i];
             const bool pass = nlf_pass(g, en, groups, v, mode);
             const uint32_t bit = 1u << (v & 31);
             if (pass) atomicOr(&en.bitmap[v >> 5], bit);
@@ -556,9 +572,12 @@ void nlf_full(const DevGraph& g, const NlfEntry* entries, uint32_t n_entries, co
     k_nlf_full<<<grid_for(nw, 4, 16384), 256, 0, s>>>(g, entries, n_entries, groups);
 }
 
-void nlf_touched(const DevGraph& g, const NlfEntry* entries, uint32_t n_entries, const NlfGroup* groups, const uint32_t* touched,
-                 const uint32_t* n_touched, uint32_t max_touched, int mode, hipStream_t s) {
-    k_nlf_touched<<<grid_for(max_touched, 256, 4096), 256, 0, s>>>(g, entries, n_entries, groups, touched, n_touched, mode);
+void nlf_touched(const DevGraph& g, const NlfEntry* entries, uint32_t n_entries, const NlfGroup* groups, const BatchScratch& w,
+                 uint32_t max_touched, int mode, hipStream_t s) {
+    if (!n_entries) return;
+    const dim3 grid(static_cast<uint32_t>(grid_for(max_touched, 256, static_cast<int>(std::max<uint32_t>(16, 4096 / n_entries)))),
+                    std::min<uint32_t>(n_entries, 65535));
+    k_nlf_touched<<<grid, 256, 0, s>>>(g, entries, n_entries, groups, w.by_label, w.label_off, mode);
 }
 
 void relation_summary(const DevGraph& g, uint32_t dir, uint32_t slot, uint32_t vrank_u, const uint32_t* cand_u,

@@ -87,9 +87,10 @@ struct NlfEntry {
 
 void nlf_full(const DevGraph& g, const NlfEntry* entries, uint32_t n_entries, const NlfGroup* groups, hipStream_t s);
 // mode 0: upper bound with the pending insertions (only sets bits); mode 1: exact on the base
-// adjacency (sets and clears bits).  Runs over the touched vertices of direction `dir`.
-void nlf_touched(const DevGraph& g, const NlfEntry* entries, uint32_t n_entries, const NlfGroup* groups,
-                 const uint32_t* touched, const uint32_t* n_touched, uint32_t max_touched, int mode, hipStream_t s);
+// adjacency (sets and clears bits).  Runs over the batch's touched vertices of one direction, grouped
+// by label (after batch_bucket).
+void nlf_touched(const DevGraph& g, const NlfEntry* entries, uint32_t n_entries, const NlfGroup* groups, const BatchScratch& w,
+                 uint32_t max_touched, int mode, hipStream_t s);
 // Cardinality and number of non-empty sources of the relation u->w restricted to candidates
 // (statisticIndex, indexing.cu:265-301).  out[0] += card, out[1] += #sources.
 void relation_summary(const DevGraph& g, uint32_t dir, uint32_t slot, uint32_t vrank_u, const uint32_t* cand_u,

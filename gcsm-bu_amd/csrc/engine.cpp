@@ -1877,7 +1877,7 @@ std::string Engine::run_resident(uint64_t lo, uint64_t n, const uint32_t* hsrc, 
     }
     for (int d = 0; d < ndirs_; d++) {
         batch_bucket(g_, max_arcs, bs_[d], s_);
-        nlf_touched(g_, d_entries_, n_entries_, d_groups_, bs_[d].touched, bs_[d].n_touched, max_arcs, 0, s_);
+        nlf_touched(g_, d_entries_, n_entries_, d_groups_, bs_[d], max_arcs, 0, s_);
     }
     fill_u32(reinterpret_cast<uint32_t*>(results_), 0u, qs_.size() * 8, s_);
     const auto t1 = std::chrono::steady_clock::now();
@@ -1914,7 +1914,7 @@ std::string Engine::run_resident(uint64_t lo, uint64_t n, const uint32_t* hsrc, 
         prof_end(prof_main_, s_, kKApply);
     }
     for (int d = 0; d < ndirs_; d++)
-        nlf_touched(g_, d_entries_, n_entries_, d_groups_, bs_[d].touched, bs_[d].n_touched, max_arcs, 1, s_);
+        nlf_touched(g_, d_entries_, n_entries_, d_groups_, bs_[d], max_arcs, 1, s_);
     for (int d = 0; d < ndirs_; d++) batch_cleanup(g_, d, max_arcs, bs_[d], s_);
     std::vector<unsigned long long> res(qs_.size() * 4);
     CSM_HIP(hipMemcpyAsync(res.data(), results_, res.size() * 8, hipMemcpyDeviceToHost, s_));

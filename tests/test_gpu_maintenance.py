@@ -1,0 +1,80 @@
+"""GPU tests of the batch maintenance kernels against plain Python over the updated edge set."""
+import random
+from collections import Counter
+
+import pytest
+
+import util
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def lib():
+    util.ensure_built()
+    return util.ffi()
+
+
+def write_graph(path, labels, edges, head=""):
+    with open(path, "w") as f:
+        f.write(head + "".join(f"v {v} {x}\n" for v, x in enumerate(labels)))
+        f.write("".join(f"e {a} {b} {x}\n" for a, b, x in edges))
+
+
+def random_edges(rng, n, m, elabels, directed, hub=0):
+    """m distinct edges over n vertices; the first `hub` vertices take part in half of them."""
+    seen = {}
+    while len(seen) < m:
+        a, b = rng.randrange(hub) if hub and rng.random() < 0.5 else rng.randrange(n), rng.randrange(n)
+        if a == b or (a, b) in seen or (not directed and (b, a) in seen):
+            continue
+        seen[a, b] = rng.randrange(elabels)
+    return [(a, b, x) for (a, b), x in seen.items()]
+
+
+def groups_of(nv, edges, labels, directed):
+    """Per vertex: number of neighbours by (direction, edge label, neighbour label)."""
+    got = [Counter() for _ in range(nv)]
+    for a, b, x in edges:
+        got[a][0, x, labels[b]] += 1
+        got[b][1 if directed else 0, x, labels[a]] += 1
+    return got
+
+
+# a star's centre has one group per leaf label: fewer, as many and more than the run lookups the
+# candidate kernel issues together (4)
+@pytest.mark.parametrize("leaves,directed,batch", [(1, False, 1), (4, False, 63), (5, False, 257), (9, False, 700), (4, True, 65), (6, True, 400)])
+def test_candidates_after_batches(lib, tmp_path, leaves, directed, batch):
+    rng = random.Random(leaves * 1000 + batch)
+    n, nl, el = 300, 5, 2
+    labels = [rng.randrange(nl) for _ in range(n)]
+    edges = random_edges(rng, n, 2600, el, directed)
+    rng.shuffle(edges)
+    held, start = edges[:batch], edges[batch:]
+    gone = start[:batch // 2]
+    write_graph(tmp_path / "data.graph", labels, start)
+    # label nl has no query vertex; one query holds a label the data graph lacks
+    star = [rng.randrange(nl - 1) for _ in range(leaves + 1)]
+    queries = [(star, [(0, k, rng.randrange(el)) if k % 2 or not directed else (k, 0, rng.randrange(el)) for k in range(1, leaves + 1)]),
+               ([0, 1, 2], [(0, 1, 0), (1, 2, 1)]), ([0, nl + 3], [(0, 1, 0)])]
+    with open(tmp_path / "update.stream", "w") as f:
+        f.write("".join(f"e {a} {b} {x}\n" for a, b, x in held) + "".join(f"-e {a} {b} {x}\n" for a, b, x in gone))
+    with lib.Session(device=0, directed=directed, ring_bytes=64 << 20, cp_list_bytes=32 << 20) as s:
+        s.load_graph(str(tmp_path / "data.graph"))
+        ids = []
+        for k, (labs, es) in enumerate(queries):
+            write_graph(tmp_path / f"q{k}.graph", labs, es, "t # 0\n")
+            ids.append(s.add_query(str(tmp_path / f"q{k}.graph")))
+        nb = s.open_updates(str(tmp_path / "update.stream"), len(held) + len(gone))
+        s.build()
+        for q in ids:
+            s.plan(q)
+        for b in range(nb):
+            s.apply_batch(b)
+        now = groups_of(n, [e for e in start if e not in set(gone)] + held, labels, directed)
+        for q, (labs, es) in zip(ids, queries):
+            need = groups_of(len(labs), es, labs, directed)
+            for u, x in enumerate(labs):
+                want = [v for v in range(n) if labels[v] == x and all(now[v][k] >= c for k, c in need[u].items())]
+                words = s.candidates(q, u)
+                assert [v for v in range(n) if words[v >> 5] >> (v & 31) & 1] == want, (q, u)
