@@ -434,29 +434,6 @@ __device__ __forceinline__ uint32_t record_runs(const DevGraph& g, const StepDes
     return best;
 }
 
-// Block-wide exclusive scan of one value per thread over T threads (s_wave holds T / 64 words);
-// returns the exclusive prefix and the block total.
-template <uint32_t T>
-__device__ __forceinline__ unsigned long long block_scan(unsigned long long v, unsigned long long* s_wave, unsigned long long& total) {
-    const uint32_t lane = lane_id(), wv = threadIdx.x >> 6;
-    unsigned long long x = v;
-    for (uint32_t o = 1; o < 64; o <<= 1) {
-        const unsigned long long y = __shfl_up(x, o, 64);
-        if (lane >= o) x += y;
-    }
-    if (lane == 63) s_wave[wv] = x;
-    __syncthreads();
-    unsigned long long before = 0;
-    total = 0;
-    for (uint32_t k = 0; k < T / 64; k++) {
-        const unsigned long long t = s_wave[k];
-        if (k < wv) before += t;
-        total += t;
-    }
-    __syncthreads();  // s_wave may be rewritten by the caller's next scan
-    return before + x - v;
-}
-
 constexpr uint32_t kSmallThreads = 1024;
 // Multi-block level preparation: 256-thread blocks (small enough to find room beside the other
 // lanes' kernels), two records per thread.

@@ -5,7 +5,7 @@
 //   batch build      the batch's arcs as a per-vertex sorted delta (replaces BuildTries /
 //                    BuildTriesFromEdgeList, match_gpu.cu:302-322, 2296-2344: CUB radix sort + RLE +
 //                    scan into a CSR).  Counting sort by source into per-vertex segments, then a
-//                    wave-level sort of each segment.
+//                    sort of each segment; admission is decided on the way.
 //   apply deletions  delete-compact of every touched list (extension; the reference is
 //                    insertion-only).
 //   apply insertions merge-insert of every touched list, relocating to a larger arena block when
@@ -22,58 +22,43 @@ constexpr int kScanItems = 8;
 constexpr uint32_t kScanTile = kScanThreads * kScanItems;
 
 template <typename T>
-__device__ T block_exclusive_scan(T v, T* sh, T& total) {
-    const int t = threadIdx.x;
-    sh[t] = v;
-    __syncthreads();
-    for (int o = 1; o < kScanThreads; o <<= 1) {
-        T x = t >= o ? sh[t - o] : T(0);
-        __syncthreads();
-        sh[t] += x;
-        __syncthreads();
-    }
-    total = sh[kScanThreads - 1];
-    const T incl = sh[t];
-    __syncthreads();
-    return incl - v;
-}
-
-template <typename T>
 __global__ void __launch_bounds__(kScanThreads) k_scan_tile_sums(const T* in, const uint32_t* n_dev, uint32_t n_max, T* sums) {
-    __shared__ T sh[kScanThreads];
+    __shared__ unsigned long long sh[kScanThreads / 64];
     const uint32_t n = n_dev ? min(*n_dev, n_max) : n_max;
     const uint32_t base = blockIdx.x * kScanTile;
     if (base >= n && blockIdx.x != 0) { if (threadIdx.x == 0) sums[blockIdx.x] = T(0); return; }
-    T acc = 0;
+    unsigned long long acc = 0, total;
     for (int k = 0; k < kScanItems; k++) {
         const uint32_t i = base + k * kScanThreads + threadIdx.x;
         if (i < n) acc += in[i];
     }
-    T total;
-    block_exclusive_scan<T>(acc, sh, total);
-    if (threadIdx.x == 0) sums[blockIdx.x] = total;
+    block_scan<kScanThreads>(acc, sh, total);
+    if (threadIdx.x == 0) sums[blockIdx.x] = static_cast<T>(total);
 }
 
+// Thread t of a tile owns its kScanItems consecutive elements: one block scan of the thread sums
+// (a scan per row of kScanThreads elements took 10 us for one tile, all of it barriers).
 template <typename T>
 __global__ void __launch_bounds__(kScanThreads) k_scan_tiles(const T* in, T* out, const uint32_t* n_dev, uint32_t n_max,
                                                               const T* tile_offsets, bool write_total) {
-    __shared__ T sh[kScanThreads];
-    __shared__ T carry;
+    __shared__ unsigned long long sh[kScanThreads / 64];
     const uint32_t n = n_dev ? min(*n_dev, n_max) : n_max;
     const uint32_t base = blockIdx.x * kScanTile;
     if (base > n) return;
-    if (threadIdx.x == 0) carry = tile_offsets ? tile_offsets[blockIdx.x] : T(0);
-    __syncthreads();
+    const unsigned long long carry = tile_offsets ? tile_offsets[blockIdx.x] : T(0);
+    const uint32_t i0 = base + threadIdx.x * kScanItems;
+    T v[kScanItems];
+    unsigned long long sum = 0, total;
+#pragma unroll
     for (int k = 0; k < kScanItems; k++) {
-        const uint32_t i = base + k * kScanThreads + threadIdx.x;
-        const T v = i < n ? in[i] : T(0);
-        T total;
-        const T ex = block_exclusive_scan<T>(v, sh, total);
-        if (i < n) out[i] = carry + ex;
-        if (write_total && i == n) out[n] = carry + ex;  // ex == sum of in[0..n) here
-        __syncthreads();
-        if (threadIdx.x == 0) carry += total;
-        __syncthreads();
+        v[k] = i0 + k < n ? in[i0 + k] : T(0);
+        sum += v[k];
+    }
+    unsigned long long ex = carry + block_scan<kScanThreads>(sum, sh, total);
+#pragma unroll
+    for (int k = 0; k < kScanItems; k++) {
+        if (i0 + k < n || (write_total && i0 + k == n)) out[i0 + k] = static_cast<T>(ex);  // at n: the sum of in[0..n)
+        ex += v[k];
     }
 }
 
@@ -116,71 +101,168 @@ template void scan_exclusive<unsigned long long>(const unsigned long long*, unsi
 // directed -> (src, key_to_dst) in direction 0 and (dst, key_to_src) in direction 1.
 namespace {
 
-__device__ __forceinline__ bool arc_of(const BatchInput& b, uint32_t k, int dirsel, int which, uint32_t& v, uint32_t& key) {
-    // which: 0 = source-side arc, 1 = destination-side arc
-    if (dirsel == 1 && which == 1) return false;  // directed, out direction: only source arcs
-    if (dirsel == 2 && which == 0) return false;  // directed, in direction: only destination arcs
-    if (which == 0) { v = b.src[k]; key = b.key_fwd[k]; }
-    else { v = b.dst[k]; key = b.key_bwd[k]; }
-    return true;
-}
-
-__global__ void k_batch_count(BatchInput b, uint32_t lo, uint32_t n, int dirsel, BatchScratch w) {
-    const uint32_t tid = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t stride = gridDim.x * blockDim.x;
-    for (uint32_t i = tid; i < 2 * n; i += stride) {
-        const uint32_t k = lo + (i >> 1);
-        uint32_t v, key;
-        if (!arc_of(b, k, dirsel, i & 1, v, key)) continue;
-        uint32_t* cnt = b.op[k] ? w.cnt_del : w.cnt_ins;
-        atomicAdd(&cnt[v], 1u);
-        if (atomicExch(&w.tflag[v], 1u) == 0u) {
-            const uint32_t p = atomicAdd(w.n_touched, 1u);
-            w.touched[p] = v;
+// Zeroes what a batch counts into: touched, segment and label counters of each direction, results.
+__global__ void __launch_bounds__(256) k_batch_begin(BatchScratch w0, BatchScratch w1, uint32_t dirs, uint32_t labels, uint32_t* results,
+                                                     uint32_t nresults) {
+    const uint32_t i0 = blockIdx.x * blockDim.x + threadIdx.x, stride = gridDim.x * blockDim.x;
+    for (uint32_t d = 0; d < dirs; d++) {
+        const BatchScratch& w = d ? w1 : w0;
+        if (i0 == 0) {
+            *w.n_touched = 0;
+            *w.n_big = 0;
+            *w.cursor = 0;
         }
+        for (uint32_t i = i0; i < labels; i += stride) w.label_cur[i] = 0;
     }
+    for (uint32_t i = i0; i < nresults; i += stride) results[i] = 0;
 }
 
-__global__ void k_batch_gather_counts(BatchScratch w) {
-    const uint32_t T = *w.n_touched;
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < T; i += gridDim.x * blockDim.x) {
-        const uint32_t v = w.touched[i];
-        w.tmp_ins[i] = w.cnt_ins[v];
-        w.tmp_del[i] = w.cnt_del[v];
-    }
-}
+// Per arc: its rank among its vertex's insertions or deletions (w.rank, by arrival) from one packed
+// 64-bit counter per vertex, whose first visitor lists the vertex.  One thread per edge; a block
+// collects its new vertices in LDS and reserves their places with one device atomic per tile (atomics
+// on one address serialise).
+constexpr uint32_t kCountEdges = 2;  // edges per thread of a tile
+constexpr uint32_t kCountTile = 256 * kCountEdges;
 
-__global__ void k_batch_write_segments(BatchScratch w, DevDelta d) {
-    const uint32_t T = *w.n_touched;
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < T; i += gridDim.x * blockDim.x) {
-        const uint32_t v = w.touched[i];
-        d.seg[v] = make_uint4(w.off_ins[i], w.cnt_ins[v], w.off_del[i], w.cnt_del[v]);
-        w.cnt_ins[v] = 0;
-        w.cnt_del[v] = 0;
-    }
-}
-
-__global__ void k_batch_scatter(BatchInput b, uint32_t lo, uint32_t n, int dirsel, BatchScratch w, DevDelta d, uint32_t* err) {
-    const uint32_t tid = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t stride = gridDim.x * blockDim.x;
-    for (uint32_t i = tid; i < 2 * n; i += stride) {
-        const uint32_t k = lo + (i >> 1);
-        uint32_t v, key;
-        if (!arc_of(b, k, dirsel, i & 1, v, key)) continue;
-        const uint4 s = d.seg[v];
-        if (b.op[k]) {
-            const uint32_t p = atomicAdd(&w.cnt_del[v], 1u);
-            if (p < s.w) d.del[s.z + p] = key; else atomicOr(err, kErrPrecondition);
-        } else {
-            const uint32_t p = atomicAdd(&w.cnt_ins[v], 1u);
-            if (p < s.y) d.ins[s.x + p] = key; else atomicOr(err, kErrPrecondition);
+__global__ void __launch_bounds__(256) k_batch_count(BatchInput b, uint32_t lo, uint32_t n, int dirsel, BatchScratch w) {
+    __shared__ uint32_t s_list[2 * kCountTile], s_n, s_base;
+    for (uint32_t tile = blockIdx.x * kCountTile; tile < n; tile += gridDim.x * kCountTile) {  // block-uniform
+        if (threadIdx.x == 0) s_n = 0;
+        __syncthreads();
+        uint32_t v[2 * kCountEdges];
+        unsigned long long old[2 * kCountEdges];
+#pragma unroll
+        for (uint32_t e = 0; e < kCountEdges; e++) {
+            const uint32_t k = tile + e * 256 + threadIdx.x;
+#pragma unroll
+            for (uint32_t side = 0; side < 2; side++) {
+                old[2 * e + side] = 1;  // not a first visitor
+                // directed: direction 0 takes the source arcs (dirsel 1), direction 1 the others (dirsel 2)
+                if (k >= n || dirsel == (side ? 1 : 2)) continue;
+                const bool del = b.op[lo + k];
+                v[2 * e + side] = side ? b.dst[lo + k] : b.src[lo + k];
+                old[2 * e + side] = atomicAdd(&w.cnt[v[2 * e + side]], del ? 1ull << 32 : 1ull);
+                w.rank[2 * k + side] = static_cast<uint32_t>(del ? old[2 * e + side] >> 32 : old[2 * e + side]);
+            }
         }
+#pragma unroll
+        for (uint32_t e = 0; e < 2 * kCountEdges; e++)
+            if (!old[e]) s_list[atomicAdd(&s_n, 1u)] = v[e];
+        __syncthreads();
+        if (threadIdx.x == 0) s_base = s_n ? atomicAdd(w.n_touched, s_n) : 0u;
+        __syncthreads();
+        for (uint32_t i = threadIdx.x; i < s_n; i += 256) w.touched[s_base + i] = s_list[i];
+        __syncthreads();
     }
+}
+
+// Delta segments of the touched vertices.  Any disjoint placement will do, so a block scans its
+// tile's counts and reserves its share of both arrays with one atomic on the packed cursor: one
+// launch instead of a gather, two device-wide scans and a write (eight).
+constexpr uint32_t kSegItems = 4;
+__global__ void __launch_bounds__(256) k_batch_segments(BatchScratch w, DevDelta d) {
+    __shared__ unsigned long long sh[4], s_base;
+    const uint32_t T = *w.n_touched;
+    for (uint32_t tile = blockIdx.x * 256 * kSegItems; tile < T; tile += gridDim.x * 256 * kSegItems) {  // block-uniform
+        uint32_t v[kSegItems];
+        unsigned long long c[kSegItems], sum = 0, total;
+#pragma unroll
+        for (uint32_t j = 0; j < kSegItems; j++) {
+            const uint32_t i = tile + j * 256 + threadIdx.x;
+            v[j] = i < T ? w.touched[i] : kNoVertex;
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < kSegItems; j++) {
+            c[j] = v[j] != kNoVertex ? w.cnt[v[j]] : 0ull;
+            sum += c[j];  // both halves stay under 2^32: a batch has fewer arcs
+        }
+        unsigned long long at = block_scan<256>(sum, sh, total);
+        if (threadIdx.x == 0) s_base = atomicAdd(w.cursor, total);
+        __syncthreads();
+        at += s_base;
+#pragma unroll
+        for (uint32_t j = 0; j < kSegItems; j++) {
+            if (v[j] != kNoVertex)
+                d.seg[v[j]] = make_uint4(static_cast<uint32_t>(at), static_cast<uint32_t>(c[j]), static_cast<uint32_t>(at >> 32),
+                                         static_cast<uint32_t>(c[j] >> 32));
+            at += c[j];
+        }
+        __syncthreads();  // s_base is rewritten
+    }
+}
+
+// Whether `key` is in v's base list of direction dir.
+__device__ __forceinline__ bool base_contains(const DevGraph& g, int dir, uint32_t v, uint32_t key) {
+    uint32_t lo, hi;
+    if (g.sdir[dir] && g.id_bits < 32) {
+        base_range(g, dir, v, key >> g.id_bits, lo, hi);
+    } else {
+        const uint2 a = g.dir[dir].adj[v];
+        lo = a.x;
+        hi = a.x + a.y;
+    }
+    return contains_u32(g.arena, lo, hi, key);
+}
+
+// Every arc's key to its place in the delta, and the preconditions of the update semantics per arc:
+// an inserted arc must not be in the list (this also catches a delete and re-insert of one arc in the
+// same batch), a deleted arc must be.  An undirected graph holds both arcs of an edge or neither:
+// the source's list answers for both.  adm[1] |= a violation.
+__global__ void __launch_bounds__(256) k_batch_scatter(DevGraph g, BatchInput b, uint32_t lo, uint32_t n, int dirsel, int dir, BatchScratch w,
+                                                       unsigned long long* adm) {
+    const DevDelta d = g.delta[dir];
+    bool bad = false;
+    for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
+        const bool del = b.op[lo + k];
+        uint32_t* const out = del ? d.del : d.ins;
+        const uint32_t sv = b.src[lo + k], dv = b.dst[lo + k], kf = b.key_fwd[lo + k], kb = b.key_bwd[lo + k];
+        if (dirsel != 2) {
+            const uint4 s = d.seg[sv];
+            out[(del ? s.z : s.x) + w.rank[2 * k]] = kf;
+        }
+        if (dirsel != 1) {
+            const uint4 s = d.seg[dv];
+            out[(del ? s.z : s.x) + w.rank[2 * k + 1]] = kb;
+        }
+        bad = bad || (dirsel == 2 ? base_contains(g, dir, dv, kb) : base_contains(g, dir, sv, kf)) != del;
+    }
+    if (__ballot(bad) != 0 && lane_id() == 0) atomicOr(reinterpret_cast<uint32_t*>(&adm[1]), 1u);
 }
 
 // Sorting network with every comparator ascending ("mirror" first step per stage), so elements
-// past n behave as +infinity padding and are never touched: valid for any n <= N = 2^k.
-__device__ void wave_sort_small(uint32_t* a, uint32_t n) {
+// past n behave as +infinity padding and are never touched: valid for any n <= N = 2^k.  The sorts
+// return whether a key occurs twice (in some lane).
+constexpr uint32_t kSortLane = 8;
+__device__ __forceinline__ bool lane_sort(uint32_t* a, uint32_t n) {
+    // n <= kSortLane, one segment per lane: odd-even merge network in registers
+    uint32_t v[kSortLane];
+#pragma unroll
+    for (uint32_t i = 0; i < kSortLane; i++) v[i] = i < n ? a[i] : 0xFFFFFFFFu;
+#pragma unroll
+    for (uint32_t k = 2; k <= kSortLane; k <<= 1) {
+#pragma unroll
+        for (uint32_t j = k >> 1; j > 0; j >>= 1) {
+#pragma unroll
+            for (uint32_t i = 0; i < kSortLane; i++) {
+                const uint32_t p = (j == (k >> 1)) ? (i ^ (k - 1)) : (i ^ j);
+                if (p > i) {
+                    const uint32_t x = v[i], y = v[p];
+                    v[i] = min(x, y);
+                    v[p] = max(x, y);
+                }
+            }
+        }
+    }
+    bool twice = false;
+#pragma unroll
+    for (uint32_t i = 0; i < kSortLane; i++) {
+        if (i < n) a[i] = v[i];
+        if (i > 0 && i < n && v[i] == v[i - 1]) twice = true;
+    }
+    return twice;
+}
+
+__device__ bool wave_sort_small(uint32_t* a, uint32_t n) {
     // n <= 64: one element per lane, exchanges through shuffles.
     const uint32_t lane = lane_id();
     uint32_t v = lane < n ? a[lane] : 0xFFFFFFFFu;
@@ -192,9 +274,11 @@ __device__ void wave_sort_small(uint32_t* a, uint32_t n) {
         }
     }
     if (lane < n) a[lane] = v;
+    const uint32_t before = __shfl_up(v, 1, 64);
+    return lane > 0 && lane < n && before == v;
 }
 
-__device__ void wave_sort_lds(uint32_t* g, uint32_t n, uint32_t* sh) {
+__device__ bool wave_sort_lds(uint32_t* g, uint32_t n, uint32_t* sh) {
     // n <= kSortLdsWave: staged through this wave's LDS slice.
     const uint32_t lane = lane_id();
     for (uint32_t i = lane; i < n; i += 64) sh[i] = g[i];
@@ -213,56 +297,117 @@ __device__ void wave_sort_lds(uint32_t* g, uint32_t n, uint32_t* sh) {
             wave_sync();
         }
     }
-    for (uint32_t i = lane; i < n; i += 64) g[i] = sh[i];
+    bool twice = false;
+    for (uint32_t i = lane; i < n; i += 64) {
+        g[i] = sh[i];
+        if (i > 0 && sh[i] == sh[i - 1]) twice = true;
+    }
     wave_sync();
+    return twice;
 }
 
 constexpr uint32_t kSortWaves = 4;
-constexpr uint32_t kSortLdsWave = 2048;
 
-__global__ void __launch_bounds__(kSortWaves * 64) k_batch_segsort(BatchScratch w, DevDelta d) {
+// Sorts the segments and finishes the admission: a key twice in a segment breaks a precondition (an
+// undirected edge given as both (a, b) and (b, a) lands in a's segment twice), and adm[6 + c] +=
+// the relocations into blocks of size class c under k_apply_insertions' rule.  A wave takes 64
+// touched vertices, a lane each: most segments hold a few keys and are sorted in the lane's
+// registers; the longer ones are then sorted by the whole wave in turn, the longest left to
+// k_batch_segsort_big.  The vertices of a wave are a group count apart in the list: hubs are touched
+// first, and 64 neighbours of the list's start held 64 long segments for one wave (500,000 edges:
+// 625 us).  (A wave per vertex spent its time in the dependent loads of one vertex after the other.)
+__global__ void __launch_bounds__(kSortWaves * 64) k_batch_segsort(DevGraph g, int dir, BatchScratch w, unsigned long long* adm) {
     __shared__ uint32_t sh[kSortWaves][kSortLdsWave];
-    const uint32_t wid = threadIdx.x >> 6;
+    __shared__ uint32_t cls_n[kFreeClasses];  // relocations of this block by size class
+    if (threadIdx.x < kFreeClasses) cls_n[threadIdx.x] = 0;
+    __syncthreads();
+    const DevDelta d = g.delta[dir];
+    const DevAdj A = g.dir[dir];
+    const uint32_t wid = threadIdx.x >> 6, lane = lane_id();
     const uint32_t T = *w.n_touched;
-    for (uint32_t i = blockIdx.x * kSortWaves + wid; i < T; i += gridDim.x * kSortWaves) {
-        const uint32_t v = w.touched[i];
-        const uint4 s = d.seg[v];
-        for (int which = 0; which < 2; which++) {
-            uint32_t* base = which == 0 ? d.ins + s.x : d.del + s.z;
-            const uint32_t len = which == 0 ? s.y : s.w;
-            if (len <= 1) continue;
-            if (len <= 64) wave_sort_small(base, len);
-            else if (len <= kSortLdsWave) wave_sort_lds(base, len, sh[wid]);
-            else if (lane_id() == 0) {
-                const uint32_t p = atomicAdd(w.n_big, 1u);
-                if (p < kMaxBigSegments) { w.big_ptr[p] = static_cast<uint32_t>(base - (which == 0 ? d.ins : d.del)); w.big_len[p] = len | (which ? 0x80000000u : 0u); }
+    bool bad = false;
+    const uint32_t groups = (T + 63) / 64;
+    for (uint32_t gi = blockIdx.x * kSortWaves + wid; gi < groups; gi += gridDim.x * kSortWaves) {
+        uint4 s = make_uint4(0, 0, 0, 0);
+        const uint32_t i = lane * groups + gi;
+        if (i < T) {
+            const uint32_t v = w.touched[i];
+            s = d.seg[v];
+            const uint2 a = A.adj[v];
+            const uint32_t cap = A.cap[v];
+            const uint32_t nd = a.y - s.w + s.y;
+            if (s.w <= a.y && s.y && nd > cap) {
+                uint32_t p2 = 1;
+                while (p2 < nd) p2 <<= 1;
+                atomicAdd(&cls_n[31u - __clz(max(kMinNbrSize, 2u * p2))], 1u);
             }
+        }
+#pragma unroll
+        for (int which = 0; which < 2; which++) {
+            uint32_t* const keys = which == 0 ? d.ins : d.del;
+            const uint32_t off = which == 0 ? s.x : s.z, len = which == 0 ? s.y : s.w;
+            if (len > 1 && len <= kSortLane) bad = lane_sort(keys + off, len) || bad;
+            for (uint64_t m = __ballot(len > kSortLane); m; m &= m - 1) {
+                const int l = __ffsll(static_cast<long long>(m)) - 1;
+                const uint32_t o = uniform(__shfl(off, l, 64)), n = uniform(__shfl(len, l, 64));
+                if (n <= 64) bad = wave_sort_small(keys + o, n) || bad;
+                else if (n <= kSortLdsWave) bad = wave_sort_lds(keys + o, n, sh[wid]) || bad;
+                else if (lane == 0) {
+                    const uint32_t p = atomicAdd(w.n_big, 1u);
+                    if (p < w.max_big) { w.big_ptr[p] = o; w.big_len[p] = n | (which ? 0x80000000u : 0u); }
+                }
+            }
+        }
+    }
+    if (__ballot(bad) != 0 && lane == 0) atomicOr(reinterpret_cast<uint32_t*>(&adm[1]), 1u);
+    __syncthreads();
+    if (threadIdx.x < kFreeClasses && cls_n[threadIdx.x]) atomicAdd(&adm[6 + threadIdx.x], static_cast<unsigned long long>(cls_n[threadIdx.x]));
+}
+
+// Segments longer than one wave's LDS slice: one block each, the bitonic network in LDS, or in
+// global memory when they do not fit there.
+constexpr uint32_t kSortLdsBlock = 8192;
+__device__ __forceinline__ void block_sort(uint32_t* a, uint32_t n) {
+    uint32_t N = 1;
+    while (N < n) N <<= 1;
+    for (uint32_t k = 2; k <= N; k <<= 1) {
+        for (uint32_t j = k >> 1; j > 0; j >>= 1) {
+            for (uint32_t i = threadIdx.x; i < N; i += blockDim.x) {
+                const uint32_t p = (j == (k >> 1)) ? (i ^ (k - 1)) : (i ^ j);
+                if (p > i && p < n) {
+                    const uint32_t x = a[i], y = a[p];
+                    if (y < x) { a[i] = y; a[p] = x; }
+                }
+            }
+            __syncthreads();
         }
     }
 }
 
-// Segments longer than one wave's LDS slice: one block each, bitonic network in global memory.
-__global__ void __launch_bounds__(1024) k_batch_segsort_big(BatchScratch w, DevDelta d, uint32_t* err) {
-    const uint32_t nb = min(*w.n_big, kMaxBigSegments);
-    if (*w.n_big > kMaxBigSegments && threadIdx.x == 0 && blockIdx.x == 0) atomicOr(err, kErrSegmentTooLong);
+__global__ void __launch_bounds__(1024) k_batch_segsort_big(BatchScratch w, DevDelta d, uint32_t* err, unsigned long long* adm) {
+    __shared__ uint32_t sh[kSortLdsBlock];
+    const uint32_t nb = min(*w.n_big, w.max_big);
+    if (*w.n_big > w.max_big && threadIdx.x == 0 && blockIdx.x == 0) atomicOr(err, kErrSegmentTooLong);
     for (uint32_t s = blockIdx.x; s < nb; s += gridDim.x) {
         const uint32_t raw = w.big_len[s];
         const uint32_t n = raw & 0x7FFFFFFFu;
         uint32_t* a = ((raw >> 31) ? d.del : d.ins) + w.big_ptr[s];
-        uint32_t N = 1;
-        while (N < n) N <<= 1;
-        for (uint32_t k = 2; k <= N; k <<= 1) {
-            for (uint32_t j = k >> 1; j > 0; j >>= 1) {
-                for (uint32_t i = threadIdx.x; i < N; i += blockDim.x) {
-                    const uint32_t p = (j == (k >> 1)) ? (i ^ (k - 1)) : (i ^ j);
-                    if (p > i && p < n) {
-                        const uint32_t x = a[i], y = a[p];
-                        if (y < x) { a[i] = y; a[p] = x; }
-                    }
-                }
-                __syncthreads();
+        bool twice = false;
+        if (n <= kSortLdsBlock) {
+            for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) sh[i] = a[i];
+            __syncthreads();
+            block_sort(sh, n);
+            for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) {
+                a[i] = sh[i];
+                if (i > 0 && sh[i] == sh[i - 1]) twice = true;
             }
+            __syncthreads();  // sh is rewritten by the next segment
+        } else {
+            block_sort(a, n);
+            for (uint32_t i = threadIdx.x; i < n; i += blockDim.x)
+                if (i > 0 && a[i] == a[i - 1]) twice = true;
         }
+        if (twice) atomicOr(reinterpret_cast<uint32_t*>(&adm[1]), 1u);
     }
 }
 
@@ -409,69 +554,26 @@ __global__ void k_free_merge_counts(DevGraph g) {
     g.fl_pend_n[c] = 0;
 }
 
-// Admission of a built batch before anything changes, one wave per touched vertex: the list space
-// its insertions will take under k_apply_insertions' relocation rule (adm[0]) and whether the batch
-// breaks a precondition of the update semantics (adm[1]): an inserted arc that is already in the
-// list (this also catches a delete and re-insert of one arc in the same batch), a deleted arc that
-// is not in the list, or the same arc twice in the batch (equal neighbouring keys in the sorted
-// segments: an undirected edge given as both (a, b) and (b, a) lands in a's segment twice).
-__global__ void __launch_bounds__(256) k_admit(DevGraph g, int dir, BatchScratch w, unsigned long long* adm) {
-    __shared__ uint32_t cls_n[kFreeClasses];  // relocations of this block by size class
-    if (threadIdx.x < kFreeClasses) cls_n[threadIdx.x] = 0;
-    __syncthreads();
-    const uint32_t T = *w.n_touched;
-    const DevAdj A = g.dir[dir];
-    const DevDelta D = g.delta[dir];
-    const uint32_t lane = lane_id();
-    const uint32_t wpb = blockDim.x >> 6;
-    bool bad = false;
-    for (uint32_t i = blockIdx.x * wpb + (threadIdx.x >> 6); i < T; i += gridDim.x * wpb) {
-        const uint32_t v = w.touched[i];
-        const uint4 s = D.seg[v];
-        const uint2 a = A.adj[v];
-        for (uint32_t j = lane; j < s.y; j += 64) {
-            const uint32_t k = D.ins[s.x + j];
-            if (j > 0 && D.ins[s.x + j - 1] == k) bad = true;
-            if (contains_u32(g.arena, a.x, a.x + a.y, k)) bad = true;
-        }
-        for (uint32_t j = lane; j < s.w; j += 64) {
-            const uint32_t k = D.del[s.z + j];
-            if (j > 0 && D.del[s.z + j - 1] == k) bad = true;
-            if (!contains_u32(g.arena, a.x, a.x + a.y, k)) bad = true;
-        }
-        if (lane == 0 && s.w <= a.y) {
-            const uint32_t nd = a.y - s.w + s.y;
-            if (s.y && nd > A.cap[v]) {
-                uint32_t p2 = 1;
-                while (p2 < nd) p2 <<= 1;
-                atomicAdd(&cls_n[31u - __clz(max(kMinNbrSize, 2u * p2))], 1u);
-            }
-        }
-    }
-    const bool any_bad = __ballot(bad) != 0;
-    if (lane == 0 && any_bad) atomicOr(reinterpret_cast<uint32_t*>(&adm[1]), 1u);
-    __syncthreads();
-    if (threadIdx.x < kFreeClasses && cls_n[threadIdx.x]) atomicAdd(&adm[6 + threadIdx.x], static_cast<unsigned long long>(cls_n[threadIdx.x]));
-}
-
-// adm[2..5] = {need, bad, arena top, error bits} for the host, need = the words of the relocations
-// that the free blocks of their classes cannot serve; adm[0..1] and the class counts adm[6..37]
-// cleared for the next batch.
-__global__ void k_admit_finish(DevGraph g, unsigned long long* adm) {
-    if (threadIdx.x != 0) return;
+// The built batch's verdict for the host: out[0..3] = {need, bad, arena top, error bits}, need = the
+// words of the relocations that the free blocks of their classes cannot serve; the flag and the
+// class counts adm[6..37] are cleared for the next batch.  One wave, a lane per class.
+__global__ void __launch_bounds__(64) k_admit_finish(DevGraph g, unsigned long long* adm, unsigned long long* out) {
+    const uint32_t c = threadIdx.x;
     unsigned long long need = 0;
-    for (uint32_t c = 0; c < kFreeClasses; c++) {
+    if (c < kFreeClasses) {
         const unsigned long long n = adm[6 + c];
         const unsigned long long avail = g.fl_cls[c].y ? static_cast<unsigned long long>(max(g.fl_top[c], 0)) : 0ull;
-        if (n > avail) need += (n - avail) << c;
+        if (n > avail) need = (n - avail) << c;
         adm[6 + c] = 0;
     }
-    adm[2] = need;
-    adm[3] = adm[1];
-    adm[4] = *g.arena_top;
-    adm[5] = *g.err;
-    adm[0] = 0;
-    adm[1] = 0;
+    need = wave_sum_u64(need);
+    if (c == 0) {
+        out[0] = need;
+        out[1] = adm[1];
+        out[2] = *g.arena_top;
+        out[3] = *g.err;
+        adm[1] = 0;
+    }
 }
 
 __global__ void k_batch_cleanup(BatchScratch w, DevDelta d) {
@@ -479,9 +581,7 @@ __global__ void k_batch_cleanup(BatchScratch w, DevDelta d) {
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < T; i += gridDim.x * blockDim.x) {
         const uint32_t v = w.touched[i];
         d.seg[v] = make_uint4(0, 0, 0, 0);
-        w.tflag[v] = 0;
-        w.cnt_ins[v] = 0;
-        w.cnt_del[v] = 0;
+        w.cnt[v] = 0;
     }
 }
 
@@ -559,33 +659,28 @@ __global__ void __launch_bounds__(256) k_bucket_scatter(DevGraph g, BatchScratch
     }
 }
 
-__global__ void k_reset_counters(BatchScratch w) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) { *w.n_touched = 0; *w.n_big = 0; }
-}
-
 }  // namespace
 
+void batch_begin(const BatchScratch* w, int dirs, uint32_t nvl, uint32_t* results, uint32_t nresults, hipStream_t s) {
+    const uint32_t most = std::max(nvl + 1, nresults);
+    k_batch_begin<<<std::min<uint32_t>(256, (most + 255) / 256), 256, 0, s>>>(w[0], w[dirs - 1], static_cast<uint32_t>(dirs), nvl + 1, results, nresults);
+}
+
 // Builds the delta of batch edges [lo, lo + n) for one direction.  n_touched ends up on the
-// device; max_arcs bounds every grid.
-void batch_build(const DevGraph& g, int dir, int dirsel, const BatchInput& b, uint32_t lo, uint32_t n,
-                 const BatchScratch& w, hipStream_t s) {
+// device; the number of arcs bounds every grid.
+void batch_build(const DevGraph& g, int dir, int dirsel, const BatchInput& b, uint32_t lo, uint32_t n, const BatchScratch& w,
+                 unsigned long long* adm, hipStream_t s) {
     const uint32_t max_arcs = 2 * n;
-    const int grid = static_cast<int>(std::min<uint32_t>(4096, (max_arcs + 255) / 256 + 1));
-    k_reset_counters<<<1, 64, 0, s>>>(w);
-    k_batch_count<<<grid, 256, 0, s>>>(b, lo, n, dirsel, w);
-    k_batch_gather_counts<<<grid, 256, 0, s>>>(w);
-    scan_exclusive<uint32_t>(w.tmp_ins, w.off_ins, w.n_touched, max_arcs, false, w.scan_tmp, s);
-    scan_exclusive<uint32_t>(w.tmp_del, w.off_del, w.n_touched, max_arcs, false, w.scan_tmp, s);
-    k_batch_write_segments<<<grid, 256, 0, s>>>(w, g.delta[dir]);
-    k_batch_scatter<<<grid, 256, 0, s>>>(b, lo, n, dirsel, w, g.delta[dir], g.err);
-    const int sgrid = static_cast<int>(std::min<uint32_t>(2048, (max_arcs + kSortWaves - 1) / kSortWaves + 1));
-    k_batch_segsort<<<sgrid, kSortWaves * 64, 0, s>>>(w, g.delta[dir]);
-    k_batch_segsort_big<<<64, 1024, 0, s>>>(w, g.delta[dir], g.err);
+    auto grid = [](uint32_t items, uint32_t per, uint32_t cap) { return std::min<uint32_t>(cap, (items + per - 1) / per); };
+    k_batch_count<<<grid(n, kCountTile, 2048), 256, 0, s>>>(b, lo, n, dirsel, w);
+    k_batch_segments<<<grid(max_arcs, 256 * kSegItems, 1024), 256, 0, s>>>(w, g.delta[dir]);
+    k_batch_scatter<<<grid(n, 256, 4096), 256, 0, s>>>(g, b, lo, n, dirsel, dir, w, adm);
+    k_batch_segsort<<<grid(max_arcs, kSortWaves * 64, 2048), kSortWaves * 64, 0, s>>>(g, dir, w, adm);
+    if (max_arcs > kSortLdsWave) k_batch_segsort_big<<<grid(max_arcs, kSortLdsWave, 256), 1024, 0, s>>>(w, g.delta[dir], g.err, adm);
 }
 
 void batch_bucket(const DevGraph& g, uint32_t max_touched, const BatchScratch& w, hipStream_t s) {
     const int grid = static_cast<int>(std::min<uint32_t>(2048, (max_touched + 255) / 256 + 1));
-    fill_u32(w.label_cur, 0u, g.nvl + 1, s);
     k_bucket_count<<<grid, 256, 0, s>>>(g, w);
     scan_exclusive<uint32_t>(w.label_cur, w.label_off, nullptr, g.nvl, true, w.label_tmp, s);
     copy_u32(w.label_off, w.label_cur, g.nvl, s);  // the scatter's cursors
@@ -610,12 +705,9 @@ void batch_apply_insertions(const DevGraph& g, int dir, uint32_t max_touched, co
     k_apply_insertions<<<grid, 256, 0, s>>>(g, dir, w, bytes);
 }
 
-void batch_admit(const DevGraph& g, int dir, uint32_t max_touched, const BatchScratch& w, unsigned long long* adm, hipStream_t s) {
-    const int grid = static_cast<int>(std::min<uint32_t>(8192, (max_touched + 3) / 4 + 1));
-    k_admit<<<grid, 256, 0, s>>>(g, dir, w, adm);
+void batch_admit_finish(const DevGraph& g, unsigned long long* adm, unsigned long long* out, hipStream_t s) {
+    k_admit_finish<<<1, 64, 0, s>>>(g, adm, out);
 }
-
-void batch_admit_finish(const DevGraph& g, unsigned long long* adm, hipStream_t s) { k_admit_finish<<<1, 64, 0, s>>>(g, adm); }
 
 void free_blocks_merge(const DevGraph& g, hipStream_t s) {
     k_free_merge<<<dim3(64, kFreeClasses), 256, 0, s>>>(g);

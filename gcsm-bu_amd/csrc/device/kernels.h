@@ -11,7 +11,7 @@
 
 namespace csm {
 
-constexpr uint32_t kMaxBigSegments = 4096;
+constexpr uint32_t kSortLdsWave = 512;  // longest delta segment one wave sorts
 
 // The whole update stream, resident in HBM: edge k is src[k] -- dst[k] with precomputed keys.
 struct BatchInput {
@@ -23,20 +23,16 @@ struct BatchInput {
 };
 
 struct BatchScratch {
-    uint32_t* cnt_ins;   // [dv]
-    uint32_t* cnt_del;   // [dv]
-    uint32_t* tflag;     // [dv]
+    unsigned long long* cnt;  // [dv] the vertex's arcs in the batch: insertions | deletions << 32 (zero between batches)
     uint32_t* touched;   // [max_arcs]
     uint32_t* n_touched; // [1]
-    uint32_t* tmp_ins;   // [max_arcs + 1]
-    uint32_t* tmp_del;
-    uint32_t* off_ins;
-    uint32_t* off_del;
+    unsigned long long* cursor;  // [1] delta words handed out: insertions | deletions << 32
+    uint32_t* rank;      // [max_arcs] per arc, its rank among its vertex's insertions or deletions
     uint32_t* ins_pos;   // [max_arcs]
-    uint32_t* scan_tmp;  // scan_scratch_elems(max_arcs)
-    uint32_t* n_big;     // [1]
-    uint32_t* big_ptr;   // [kMaxBigSegments]
+    uint32_t* n_big;     // [1] segments longer than kSortLdsWave
+    uint32_t* big_ptr;   // [max_big]
     uint32_t* big_len;
+    uint32_t max_big;
     // the touched vertices grouped by label rank (batch_bucket): rank r's at by_label[label_off[r] ..
     // label_off[r + 1])
     uint32_t* by_label;  // [max_arcs]
@@ -49,16 +45,17 @@ template <typename T>
 void scan_exclusive(const T* in, T* out, const uint32_t* n_dev, uint32_t n_max, bool write_total, T* scratch, hipStream_t s);
 uint64_t scan_scratch_elems(uint32_t n_max);
 
-void batch_build(const DevGraph& g, int dir, int dirsel, const BatchInput& b, uint32_t lo, uint32_t n,
-                 const BatchScratch& w, hipStream_t s);
+// Clears the counters of both directions' scratch and the results; comes before the batch's batch_build.
+void batch_begin(const BatchScratch* w, int dirs, uint32_t nvl, uint32_t* results, uint32_t nresults, hipStream_t s);
+// Builds the delta and decides admission on the way: adm[6 + c] += the insertions' relocations into
+// blocks of size class c, adm[1] |= a precondition violation (all zero before the first batch).
+void batch_build(const DevGraph& g, int dir, int dirsel, const BatchInput& b, uint32_t lo, uint32_t n, const BatchScratch& w,
+                 unsigned long long* adm, hipStream_t s);
 // Groups the built batch's touched vertices by label rank (w.by_label, w.label_off).
 void batch_bucket(const DevGraph& g, uint32_t max_touched, const BatchScratch& w, hipStream_t s);
-// Admission of the built batch (per direction, then finish once): adm[6 + c] += the insertions'
-// relocations into blocks of size class c, adm[1] |= a precondition violation; finish moves
-// {need, bad, arena top, error bits} to adm[2..5], need = words the free blocks cannot serve, and
-// clears adm[0..1] and adm[6..37] (all zero before the first batch).
-void batch_admit(const DevGraph& g, int dir, uint32_t max_touched, const BatchScratch& w, unsigned long long* adm, hipStream_t s);
-void batch_admit_finish(const DevGraph& g, unsigned long long* adm, hipStream_t s);
+// After every direction's batch_build: {need, bad, arena top, error bits} to out (pinned host memory),
+// need = words the free blocks cannot serve; clears adm.
+void batch_admit_finish(const DevGraph& g, unsigned long long* adm, unsigned long long* out, hipStream_t s);
 // The blocks freed by a batch's relocations become available (after its insertions are applied).
 void free_blocks_merge(const DevGraph& g, hipStream_t s);
 // Recomputes label-slot directory rows of direction dir: every vertex when list is null, else

@@ -234,9 +234,9 @@ std::string Engine::build() {
     for (int d = 0; d < ndirs_; d++) {
         add(dv_ * 8ull); add(dv_ * 4ull);                       // adj, cap
         add(dv_ * 16ull); add(max_arcs * 4); add(max_arcs * 4); // delta seg, ins, del
-        add(dv_ * 12ull);                                       // cnt_ins, cnt_del, tflag
-        add(max_arcs * 4); add(16); add(4 * (max_arcs + 1) * 4); add(max_arcs * 4);
-        add(scan_scratch_elems(static_cast<uint32_t>(max_arcs)) * 4); add(16); add(2 * kMaxBigSegments * 4);
+        add(dv_ * 8ull);                                        // cnt
+        add(max_arcs * 4); add(16); add(max_arcs * 4); add(max_arcs * 4);  // touched, counters, rank, ins_pos
+        add((max_arcs / kSortLdsWave + 1) * 4); add((max_arcs / kSortLdsWave + 1) * 4);  // long segments
         add(max_arcs * 4); add(2 * (nvl_ + 1) * 4ull); add(scan_scratch_elems(nvl_ + 1) * 4);  // label buckets
     }
     add(stream_.size() * 17ull + 2 * max_batch_ * 17ull);      // stream + two live-batch slots
@@ -359,24 +359,18 @@ std::string Engine::build() {
             g_.delta[d].del = pool_.take<uint32_t>(max_arcs);
             CSM_HIP(hipMemsetAsync(g_.delta[d].seg, 0, dv_ * 16ull, s_));
             BatchScratch& w = bs_[d];
-            w.cnt_ins = pool_.take<uint32_t>(dv_);
-            w.cnt_del = pool_.take<uint32_t>(dv_);
-            w.tflag = pool_.take<uint32_t>(dv_);
-            CSM_HIP(hipMemsetAsync(w.cnt_ins, 0, dv_ * 4ull, s_));
-            CSM_HIP(hipMemsetAsync(w.cnt_del, 0, dv_ * 4ull, s_));
-            CSM_HIP(hipMemsetAsync(w.tflag, 0, dv_ * 4ull, s_));
+            w.cnt = pool_.take<unsigned long long>(dv_);
+            CSM_HIP(hipMemsetAsync(w.cnt, 0, dv_ * 8ull, s_));
             w.touched = pool_.take<uint32_t>(max_arcs);
             w.n_touched = pool_.take<uint32_t>(4);
             w.n_big = w.n_touched + 1;
+            w.cursor = reinterpret_cast<unsigned long long*>(w.n_touched + 2);
             CSM_HIP(hipMemsetAsync(w.n_touched, 0, 16, s_));
-            w.tmp_ins = pool_.take<uint32_t>(max_arcs + 1);
-            w.tmp_del = pool_.take<uint32_t>(max_arcs + 1);
-            w.off_ins = pool_.take<uint32_t>(max_arcs + 1);
-            w.off_del = pool_.take<uint32_t>(max_arcs + 1);
+            w.rank = pool_.take<uint32_t>(max_arcs);
             w.ins_pos = pool_.take<uint32_t>(max_arcs);
-            w.scan_tmp = pool_.take<uint32_t>(scan_scratch_elems(static_cast<uint32_t>(max_arcs)));
-            w.big_ptr = pool_.take<uint32_t>(kMaxBigSegments);
-            w.big_len = pool_.take<uint32_t>(kMaxBigSegments);
+            w.max_big = static_cast<uint32_t>(max_arcs / kSortLdsWave + 1);
+            w.big_ptr = pool_.take<uint32_t>(w.max_big);
+            w.big_len = pool_.take<uint32_t>(w.max_big);
             w.by_label = pool_.take<uint32_t>(max_arcs);
             w.label_off = pool_.take<uint32_t>(nvl_ + 1);
             w.label_cur = pool_.take<uint32_t>(nvl_ + 1);
@@ -1845,12 +1839,13 @@ std::string Engine::run_resident(uint64_t lo, uint64_t n, const uint32_t* hsrc, 
     const uint32_t max_arcs = static_cast<uint32_t>(2 * n);
     if (n == 0) { out.assign(qs_.size(), QueryResult{}); return ""; }
     prof_begin(prof_main_, s_, kKBatchBuild);
-    for (int d = 0; d < ndirs_; d++) batch_build(g_, d, ndirs_ == 1 ? 0 : d + 1, bin_, static_cast<uint32_t>(lo), static_cast<uint32_t>(n), bs_[d], s_);
-    // admission before anything changes: list space of the insertions, deletions of missing arcs
-    for (int d = 0; d < ndirs_; d++) batch_admit(g_, d, max_arcs, bs_[d], adm_, s_);
-    batch_admit_finish(g_, adm_, s_);
+    batch_begin(bs_, ndirs_, nvl_, reinterpret_cast<uint32_t*>(results_), static_cast<uint32_t>(qs_.size() * 8), s_);
+    // the deltas, with admission decided on the way, before anything changes: list space of the
+    // insertions, insertions of arcs that exist, deletions of missing arcs
+    for (int d = 0; d < ndirs_; d++)
+        batch_build(g_, d, ndirs_ == 1 ? 0 : d + 1, bin_, static_cast<uint32_t>(lo), static_cast<uint32_t>(n), bs_[d], adm_, s_);
+    batch_admit_finish(g_, adm_, reinterpret_cast<unsigned long long*>(h_pinned_), s_);
     prof_end(prof_main_, s_, kKBatchBuild);
-    CSM_HIP(hipMemcpyAsync(h_pinned_, adm_ + 2, 32, hipMemcpyDeviceToHost, s_));
     CSM_HIP(hipStreamSynchronize(s_));
     unsigned long long a[4];
     std::memcpy(a, h_pinned_, 32);
@@ -1879,7 +1874,6 @@ std::string Engine::run_resident(uint64_t lo, uint64_t n, const uint32_t* hsrc, 
         batch_bucket(g_, max_arcs, bs_[d], s_);
         nlf_touched(g_, d_entries_, n_entries_, d_groups_, bs_[d], max_arcs, 0, s_);
     }
-    fill_u32(reinterpret_cast<uint32_t*>(results_), 0u, qs_.size() * 8, s_);
     const auto t1 = std::chrono::steady_clock::now();
     double match_ms = 0;
     if (info.deletes) {

@@ -2,6 +2,7 @@
 import random
 from collections import Counter
 
+import numpy as np
 import pytest
 
 import util
@@ -78,3 +79,58 @@ def test_candidates_after_batches(lib, tmp_path, leaves, directed, batch):
                 want = [v for v in range(n) if labels[v] == x and all(now[v][k] >= c for k, c in need[u].items())]
                 words = s.candidates(q, u)
                 assert [v for v in range(n) if words[v >> 5] >> (v & 31) & 1] == want, (q, u)
+
+
+def run_batch(s, edges, gone):
+    rows = np.array([(a, b, 0) for a, b in edges], dtype=np.uint32).reshape(-1, 3)
+    s.apply_edges(np.ascontiguousarray(rows[:, 0]), np.ascontiguousarray(rows[:, 1]), np.ascontiguousarray(rows[:, 2]),
+                  np.array(gone, dtype=np.uint8))
+
+
+# delta segments around the limits of a lane's registers (8), a wave (64), a wave's LDS slice (512) and
+# a block's LDS (8192), with the other segments of the batch short
+@pytest.mark.parametrize("arcs", [1, 8, 9, 64, 65, 512, 513, 8192, 8193])
+@pytest.mark.parametrize("directed", [False, True])
+def test_delta_segments(lib, tmp_path, arcs, directed):
+    rng = random.Random(arcs)
+    n = arcs + 400
+    hub = rng.randrange(n)
+    spokes = rng.sample([v for v in range(n) if v != hub], arcs)
+    ring = [(v, (v + 1) % n) for v in range(0, n - 1, 2) if hub not in (v, v + 1)]  # one arc per vertex, deleted and put back
+    star = [(hub, v) if rng.random() < 0.5 else (v, hub) for v in spokes]
+    write_graph(tmp_path / "data.graph", [0] * n, [(a, b, 0) for a, b in ring])
+    write_graph(tmp_path / "q.graph", [0, 0], [(0, 1, 0)], "t # 0\n")
+    with lib.Session(device=0, directed=directed, max_batch_edges=2 * n, ring_bytes=64 << 20, cp_list_bytes=32 << 20) as s:
+        s.load_graph(str(tmp_path / "data.graph"))
+        q = s.add_query(str(tmp_path / "q.graph"))
+        s.build()
+        s.plan(q)
+
+        def lists(edges):
+            out, inn = [[] for _ in range(n)], [[] for _ in range(n)]
+            for a, b in edges:
+                out[a].append(b)
+                (inn if directed else out)[b].append(a)
+            return [sorted(x) for x in out], [sorted(x) for x in inn]
+
+        def check(edges):
+            out, inn = lists(edges)
+            for v in [hub] + rng.sample(range(n), 60):
+                assert list(s.adjacency(v)) == out[v], v
+                if directed:
+                    assert list(s.adjacency(v, 1)) == inn[v], v
+
+        twice = star + [star[-1]]  # the same arc twice, in the hub's segment
+        for bad in (twice, twice if directed else star + [star[0][::-1]], star + [ring[0]]):
+            with pytest.raises(lib.CsmError):
+                run_batch(s, bad, [0] * len(bad))
+        with pytest.raises(lib.CsmError):
+            run_batch(s, star, [1] * len(star))
+        check(ring)
+        both = star + ring
+        rng.shuffle(both)
+        fresh = set(star)
+        run_batch(s, both, [0 if e in fresh else 1 for e in both])
+        check(star)
+        run_batch(s, both, [1 if e in fresh else 0 for e in both])
+        check(ring)
