@@ -83,8 +83,8 @@ def test_candidates_after_batches(lib, tmp_path, leaves, directed, batch):
 
 def run_batch(s, edges, gone):
     rows = np.array([(a, b, 0) for a, b in edges], dtype=np.uint32).reshape(-1, 3)
-    s.apply_edges(np.ascontiguousarray(rows[:, 0]), np.ascontiguousarray(rows[:, 1]), np.ascontiguousarray(rows[:, 2]),
-                  np.array(gone, dtype=np.uint8))
+    return s.apply_edges(np.ascontiguousarray(rows[:, 0]), np.ascontiguousarray(rows[:, 1]), np.ascontiguousarray(rows[:, 2]),
+                         np.array(gone, dtype=np.uint8))[0]
 
 
 # delta segments around the limits of a lane's registers (8), a wave (64), a wave's LDS slice (512) and
@@ -130,7 +130,11 @@ def test_delta_segments(lib, tmp_path, arcs, directed):
         both = star + ring
         rng.shuffle(both)
         fresh = set(star)
-        run_batch(s, both, [0 if e in fresh else 1 for e in both])
+        # the query is one edge: its embeddings are the anchors, the hub's all in one run
+        way = 1 if directed else 2
+        got = run_batch(s, both, [0 if e in fresh else 1 for e in both])
+        assert tuple(got[0])[:2] == (way * len(star), way * len(ring))
         check(star)
-        run_batch(s, both, [1 if e in fresh else 0 for e in both])
+        got = run_batch(s, both, [1 if e in fresh else 0 for e in both])
+        assert tuple(got[0])[:2] == (way * len(ring), way * len(star))
         check(ring)
