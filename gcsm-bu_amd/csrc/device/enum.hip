@@ -936,7 +936,9 @@ __global__ void k_init_from_pairs(const uint32_t* pairs, const uint32_t* n_pairs
 // Pairs (v, x) with v in the start list, x in the view run of v along a->b and x in filter(b).
 // The runs of a wave's G start vertices are flattened (a wave prefix of their lengths, one element
 // per lane per round, its vertex found by a search of the prefix in LDS), and the wave reserves
-// its survivors' output once per round: most start vertices have a run of a few elements.
+// its survivors' output once per round of kInitIlp elements a lane, whose loads are in flight
+// together: most start vertices have a run of a few elements.
+constexpr uint32_t kInitIlp = 4;
 __device__ __forceinline__ void init_set_body(const DevGraph& g, const InitJob& J) {
     __shared__ uint32_t s_pre[4][65];
     __shared__ RunView s_run[4][64];
@@ -964,29 +966,42 @@ __device__ __forceinline__ void init_set_body(const DevGraph& g, const InitJob& 
         s_v[wv][lane] = v;
         if (lane == 63) s_pre[wv][64] = T;
         wave_sync();
-        for (uint32_t e0 = 0; e0 < T; e0 += 64) {  // wave-uniform trip count
-            const uint32_t e = e0 + lane;
-            bool ok = false;
-            uint32_t sv = 0, x = 0;
-            if (e < T) {
-                const uint32_t k = owner_of(s_pre[wv], e);
-                const RunView rr = s_run[wv][k];
-                sv = s_v[wv][k];
-                const uint32_t key = run_elem(g, dl, rr, s_nb[wv][k], e - s_pre[wv][k]);
-                x = key & g.id_mask;
-                ok = x != sv && bit_test(J.filter_b, x) && run_elem_live(dl, rr, J.view, key);
+        for (uint32_t e0 = 0; e0 < T; e0 += 64 * kInitIlp) {  // wave-uniform trip count
+            uint32_t k[kInitIlp], key[kInitIlp], sv[kInitIlp];
+            bool ok[kInitIlp];
+            uint64_t m[kInitIlp];
+            uint32_t c = 0;
+#pragma unroll
+            for (uint32_t u = 0; u < kInitIlp; u++) {
+                const uint32_t e = e0 + 64 * u + lane;
+                ok[u] = e < T;
+                k[u] = ok[u] ? owner_of(s_pre[wv], e) : 0u;
+                sv[u] = s_v[wv][k[u]];
+                key[u] = ok[u] ? run_elem(g, dl, s_run[wv][k[u]], s_nb[wv][k[u]], e - s_pre[wv][k[u]]) : 0u;
             }
-            const uint64_t m = __ballot(ok);
-            if (!m) continue;
+#pragma unroll
+            for (uint32_t u = 0; u < kInitIlp; u++) {
+                const uint32_t x = key[u] & g.id_mask;
+                ok[u] = ok[u] && x != sv[u] && bit_test(J.filter_b, x);
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < kInitIlp; u++) {
+                ok[u] = ok[u] && run_elem_live(dl, s_run[wv][k[u]], J.view, key[u]);
+                m[u] = __ballot(ok[u]);
+                c += static_cast<uint32_t>(__popcll(m[u]));
+            }
+            if (!c) continue;  // wave-uniform
             uint32_t o = 0;
-            if (lane == 0) o = atomicAdd(J.out_count, static_cast<uint32_t>(__popcll(m)));
-            o = __shfl(o, 0, 64);
-            if (static_cast<uint64_t>(o) + __popcll(m) > J.out_cap) {
+            if (lane == 0) o = atomicAdd(J.out_count, c);
+            o = uniform(__shfl(o, 0, 64));
+            if (static_cast<uint64_t>(o) + c > J.out_cap) {
                 if (lane == 0) atomicOr(J.overflow, 1u);
-            } else if (ok) {
-                const uint64_t p = o + lanes_below(m);
-                J.out[2 * p] = sv;
-                J.out[2 * p + 1] = x;
+                continue;
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < kInitIlp; u++) {
+                if (ok[u]) reinterpret_cast<uint2*>(J.out)[o + lanes_below(m[u])] = make_uint2(sv[u], key[u] & g.id_mask);
+                o += static_cast<uint32_t>(__popcll(m[u]));
             }
         }
         wave_sync();  // the LDS rows are rewritten by the next items

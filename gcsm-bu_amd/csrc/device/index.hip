@@ -146,8 +146,8 @@ struct Rel4 {
 // Expands `total` frontier items: item(i, j, x) gives item i's job and frontier vertex, rel(j) the
 // job's expansion relation, target(j, cand, bitmap) its candidate bitmap and output bitmap.  Every
 // element y of an item's run that is a candidate and live in the view is offered to the output
-// bitmap (atomic test-and-set); emit(fresh, y, j) is called by the whole wave once per element
-// group.  Returns this lane's algorithmic bytes.
+// bitmap (atomic test-and-set); emit(fresh, y, j) is called by the whole wave once per round with its
+// kFlatIlp elements per lane.  Returns this lane's algorithmic bytes.
 template <class Item, class Rel, class Target, class Emit>
 __device__ __forceinline__ uint64_t expand_flat(const DevGraph& g, FlatLds& lds, uint32_t total, Item item, Rel rel, Target target,
                                                 Emit emit) {
@@ -212,12 +212,9 @@ __device__ __forceinline__ uint64_t expand_flat(const DevGraph& g, FlatLds& lds,
                 // else offered by another visitor
                 fresh[u] = ok[u] && !(atomicOr(const_cast<uint32_t*>(lds.bm[wv][kk[u]]) + (y[u] >> 5), bit) & bit);
             }
+            emit(fresh, y, jj);
 #pragma unroll
-            for (uint32_t u = 0; u < kFlatIlp; u++) {
-                if (e0 + 64 * u >= T) break;  // wave-uniform
-                emit(fresh[u], y[u], jj[u]);
-                bytes += fresh[u] ? 4u : 0u;
-            }
+            for (uint32_t u = 0; u < kFlatIlp; u++) bytes += fresh[u] ? 4u : 0u;
         }
         wave_sync();  // the LDS rows are rewritten by the next items
     }
@@ -301,15 +298,28 @@ __device__ __forceinline__ uint64_t check_flat(const DevGraph& g, FlatLds& lds, 
     return bytes;
 }
 
-// Appends the wave's flagged vertices to list[*len ...] with one reservation (entries past cap are
-// dropped; the caller sizes cap for every vertex).
-__device__ __forceinline__ void append_fresh(bool fresh, uint32_t y, uint32_t* list, uint32_t* len, uint32_t cap) {
-    const uint64_t m = __ballot(fresh);
-    if (!m) return;
+// Appends the wave's flagged vertices (N per lane) to list[*len ...] with one reservation (entries past
+// cap are dropped; the caller sizes cap for every vertex).  One device atomic per round: atomics on
+// one cache line serialise at about 9 ns, and each is a round trip for its wave.
+template <uint32_t N>
+__device__ __forceinline__ void append_fresh(const bool* fresh, const uint32_t* y, uint32_t* list, uint32_t* len, uint32_t cap) {
+    uint64_t m[N];
+    uint32_t n = 0;
+#pragma unroll
+    for (uint32_t u = 0; u < N; u++) {
+        m[u] = __ballot(fresh[u]);
+        n += static_cast<uint32_t>(__popcll(m[u]));
+    }
+    if (!n) return;
     uint32_t p = 0;
-    if (lane_id() == 0) p = atomicAdd(len, static_cast<uint32_t>(__popcll(m)));
-    p = static_cast<uint32_t>(__shfl(static_cast<int>(p), 0, 64)) + lanes_below(m);
-    if (fresh && p < cap) list[p] = y;
+    if (lane_id() == 0) p = atomicAdd(len, n);
+    p = uniform(__shfl(static_cast<int>(p), 0, 64));
+#pragma unroll
+    for (uint32_t u = 0; u < N; u++) {
+        const uint32_t q = p + lanes_below(m[u]);
+        if (fresh[u] && q < cap) list[q] = y[u];
+        p += static_cast<uint32_t>(__popcll(m[u]));
+    }
 }
 
 // Anchors of one step: the batch arcs (v, x) of its slot with v a candidate of u0 among its label's
@@ -449,7 +459,7 @@ __global__ void __launch_bounds__(256) k_local_expand(DevGraph g, uint32_t phase
         g, lds, F, [&](uint32_t i, uint32_t& j, uint32_t& x) { j = 0; x = frontier[i]; },
         [&](uint32_t) { return Rel4{phase, view, dir, slot}; },
         [&](uint32_t, const uint32_t*& c, uint32_t*& bm) { c = cand_u; bm = out.bitmap; },
-        [&](bool fresh, uint32_t y, uint32_t) { append_fresh(fresh, y, out.list, out.len, out.cap); });
+        [&](const bool* fresh, const uint32_t* y, const uint32_t*) { append_fresh<kFlatIlp>(fresh, y, out.list, out.len, out.cap); });
     add_bytes(nbytes, bytes);
 }
 
@@ -467,7 +477,7 @@ __global__ void __launch_bounds__(256) k_local_queue(DevGraph g, uint32_t phase,
         g, lds, F, [&](uint32_t i, uint32_t& j, uint32_t& x) { j = 0; x = frontier[i]; },
         [&](uint32_t) { return Rel4{phase, view, dir, slot}; },
         [&](uint32_t, const uint32_t*& c, uint32_t*& bm) { c = cand_u; bm = bitmap; },
-        [&](bool fresh, uint32_t y, uint32_t) { append_fresh(fresh, y, queue, queue_len, 0xFFFFFFFFu); });
+        [&](const bool* fresh, const uint32_t* y, const uint32_t*) { append_fresh<kFlatIlp>(fresh, y, queue, queue_len, 0xFFFFFFFFu); });
     add_bytes(nbytes, bytes);
 }
 
@@ -479,7 +489,8 @@ __global__ void __launch_bounds__(256) k_local_check(DevGraph g, uint32_t phase,
         g, lds, n, [&](uint32_t i, uint32_t& j, uint32_t& y, uint32_t& nf) { j = 0; y = queue[i]; nf = fl.n; },
         [&](uint32_t, uint32_t k) { return fl.f[k]; }, [&](uint32_t) { return phase; },
         [&](bool active, bool pass, uint32_t y, uint32_t) {
-            append_fresh(active && pass, y, out.list, out.len, out.cap);
+            const bool kept = active && pass;
+            append_fresh<1>(&kept, &y, out.list, out.len, out.cap);
             if (active && !pass) atomicAnd(&out.bitmap[y >> 5], ~(1u << (y & 31)));
         });
     add_bytes(nbytes, bytes);
@@ -529,29 +540,38 @@ __device__ __forceinline__ uint32_t job_of(const uint32_t* off, uint32_t njobs, 
     return lo;
 }
 
-// Appends the flagged lanes' vertices to their jobs' queues (to_queue) or output lists: one
-// reservation when every flagged lane belongs to the same job, else one atomic per lane.
-__device__ __forceinline__ void append_jobs(bool flag, uint32_t y, uint32_t j, const LocalJob* jobs, bool to_queue) {
-    const uint64_t m = __ballot(flag);
+// Appends the flagged vertices (N per lane) to their jobs' queues (to_queue) or output lists: one
+// reservation when every flagged vertex belongs to the same job, else one atomic each.
+template <uint32_t N>
+__device__ __forceinline__ void append_jobs(const bool* flag, const uint32_t* y, const uint32_t* j, const LocalJob* jobs, bool to_queue) {
+    bool any = false;
+    uint32_t mine = 0;
+#pragma unroll
+    for (uint32_t u = 0; u < N; u++) {
+        if (flag[u]) mine = j[u];
+        any = any || flag[u];
+    }
+    const uint64_t m = __ballot(any);
     if (!m) return;
-    const uint32_t first = static_cast<uint32_t>(__ffsll(static_cast<long long>(m)) - 1);
-    const uint32_t j0 = static_cast<uint32_t>(__shfl(static_cast<int>(j), first, 64));
-    if (__ballot(flag && j != j0) == 0) {
+    const uint32_t j0 = uniform(__shfl(static_cast<int>(mine), __ffsll(static_cast<long long>(m)) - 1, 64));
+    bool other = false;
+#pragma unroll
+    for (uint32_t u = 0; u < N; u++) other = other || (flag[u] && j[u] != j0);
+    if (__ballot(other) == 0) {
         const LocalJob& J = jobs[j0];
-        uint32_t* list = to_queue ? J.queue : J.out.list;
-        uint32_t* len = to_queue ? J.queue_len : J.out.len;
-        const uint32_t cap = to_queue ? 0xFFFFFFFFu : J.out.cap;
-        uint32_t p = 0;
-        if (lane_id() == first) p = atomicAdd(len, static_cast<uint32_t>(__popcll(m)));
-        p = static_cast<uint32_t>(__shfl(static_cast<int>(p), first, 64)) + lanes_below(m);
-        if (flag && p < cap) list[p] = y;
-    } else if (flag) {
-        const LocalJob& J = jobs[j];
+        if (to_queue) append_fresh<N>(flag, y, J.queue, J.queue_len, 0xFFFFFFFFu);
+        else append_fresh<N>(flag, y, J.out.list, J.out.len, J.out.cap);
+        return;
+    }
+#pragma unroll
+    for (uint32_t u = 0; u < N; u++) {
+        if (!flag[u]) continue;
+        const LocalJob& J = jobs[j[u]];
         if (to_queue) {
-            J.queue[atomicAdd(J.queue_len, 1u)] = y;
+            J.queue[atomicAdd(J.queue_len, 1u)] = y[u];
         } else {
             const uint32_t p = atomicAdd(J.out.len, 1u);
-            if (p < J.out.cap) J.out.list[p] = y;
+            if (p < J.out.cap) J.out.list[p] = y[u];
         }
     }
 }
@@ -571,7 +591,7 @@ __global__ void __launch_bounds__(256, 8) k_local_queue_multi(DevGraph g, const 
         },
         [&](uint32_t j) { return Rel4{jobs[j].phase, jobs[j].view, jobs[j].dir, jobs[j].slot}; },
         [&](uint32_t j, const uint32_t*& c, uint32_t*& bm) { c = jobs[j].cand_u; bm = jobs[j].out.bitmap; },
-        [&](bool fresh, uint32_t y, uint32_t j) { append_jobs(fresh, y, j, jobs, true); });
+        [&](const bool* fresh, const uint32_t* y, const uint32_t* j) { append_jobs<kFlatIlp>(fresh, y, j, jobs, true); });
     add_bytes(nbytes, bytes);
 }
 
@@ -588,7 +608,8 @@ __global__ void __launch_bounds__(256, 7) k_local_check_multi(DevGraph g, const 
         },
         [&](uint32_t j, uint32_t k) { return jobs[j].fl.f[k]; }, [&](uint32_t j) { return jobs[j].phase; },
         [&](bool active, bool pass, uint32_t y, uint32_t j) {
-            append_jobs(active && pass, y, j, jobs, false);
+            const bool kept = active && pass;
+            append_jobs<1>(&kept, &y, &j, jobs, false);
             if (active && !pass) atomicAnd(&jobs[j].out.bitmap[y >> 5], ~(1u << (y & 31)));
         });
     add_bytes(nbytes, bytes);
