@@ -26,63 +26,38 @@
 namespace csm {
 namespace {
 
-constexpr uint32_t kWaves = 4;  // waves per block
+constexpr uint32_t kWaves = 2;  // waves per block of the depth-first kernel (their LDS stacks stay under 64 KB at 16 depths)
 
-// Per-wave DFS state in LDS.  Behind it (dynamic LDS, per wave): `rows` candidate buffers of 64
-// words, one per depth d0 .. end_depth-2.
-struct WaveHdr {
-    unsigned long long ph[kMaxQV + 1];  // ph[d] = sum_{j<d} pair_hash(order[j], f[j])
-    RunView run[kMaxQE];
-    uint32_t f[kMaxQV];
-    uint32_t cur[kMaxQV], tot[kMaxQV], nb[kMaxQV], bcnt[kMaxQV], bpos[kMaxQV];
+// Per-wave state of the depth-first search in LDS.  The wave searches batches of up to 64 partial
+// results: frame j extends its rows (partial results of depth d0 + j, at most one per lane) by the
+// vertex of that depth.  Behind the header (dynamic LDS, per wave): the current frame's matched
+// vertices, one row of 64 words per position below end_depth, then one child buffer per frame that
+// is followed by another.
+constexpr uint32_t kDfsIlp = 2;                       // candidates a lane tests together
+constexpr uint32_t kDfsBuf = 64 + 64 * kDfsIlp;       // a round finds fewer than 64 rows waiting
+constexpr uint32_t kDfsRuns = 4;                      // entries whose runs are kept per row; the others are looked up per candidate
+struct DfsHdr {
+    unsigned long long ph[64];   // prefix hash of the row
+    uint4 runs[kDfsRuns][64];    // view runs of the row's backward entries
+    uint32_t pre[64];            // exclusive prefix of the rows' generating lengths
+    uint32_t gen[64];            // generating entry of the row (the shortest of the kept runs)
+    uint32_t skip[64];           // first generated element (a record cut into chunks)
+    uint32_t rec[64];            // record of each row of frame 0
+    uint32_t chunk[64], chunks[64];
+    uint32_t rows[kMaxQV], waiting[kMaxQV], cur[kMaxQV], tot[kMaxQV];
+};
+struct DfsBuf {
+    uint32_t cand[kDfsBuf];   // vertex matched at the frame's depth
+    uint8_t parent[kDfsBuf];  // row of the frame it extends
 };
 
-__host__ __device__ constexpr uint32_t wave_lds_bytes(uint32_t rows) {
-    return static_cast<uint32_t>((sizeof(WaveHdr) + rows * 256u + 15u) & ~15u);
+__host__ __device__ constexpr uint32_t wave_lds_bytes(uint32_t d0, uint32_t end_depth) {
+    const uint32_t bufs = end_depth > d0 + 1 ? end_depth - 1 - d0 : 0u;
+    return static_cast<uint32_t>((sizeof(DfsHdr) + (end_depth - 1) * 256u + bufs * sizeof(DfsBuf) + 15u) & ~15u);
 }
 
 __device__ __forceinline__ const uint32_t* entry_delta(const DevGraph& g, const StepDesc& d, const BackEntry& e) {
     return phase_delta(g, e.dir, d.phase);
-}
-
-// Computes the view runs of every backward entry of `depth` and resets its frame.
-// Algorithmic bytes of a frame: every view run of the depth's backward lists read once.
-__device__ __forceinline__ void setup_frame(const DevGraph& g, const StepDesc& d, WaveHdr& W, uint32_t depth, uint32_t lane,
-                                            unsigned long long& bytes, bool count_bytes) {
-    const uint32_t e0 = d.boff[depth], e1 = d.boff[depth + 1];
-    if (lane < e1 - e0) {
-        const BackEntry e = d.be[e0 + lane];
-        W.run[e0 + lane] = make_run(g, d.phase, e.view, e.dir, W.f[e.pos], e.slot);
-    }
-    wave_sync();
-    const uint32_t p = d.pivot[depth];
-    if (lane == 0) {
-        if (count_bytes)
-            for (uint32_t e = e0; e < e1; e++) bytes += 4ull * ((W.run[e].hi - W.run[e].lo) + (W.run[e].dhi - W.run[e].dlo));
-        const RunView r = W.run[p];
-        W.nb[depth] = run_base_len(r, d.be[p].view);
-        W.tot[depth] = run_seq_len(r, d.be[p].view);
-        W.cur[depth] = 0;
-        W.bcnt[depth] = 0;
-        W.bpos[depth] = 0;
-    }
-    wave_sync();
-}
-
-__device__ __forceinline__ bool test_candidate(const DevGraph& g, const StepDesc& d, const WaveHdr& W, uint32_t depth, uint32_t key) {
-    const uint32_t c = key & g.id_mask;
-    if (!bit_test(d.filter[depth], c)) return false;
-    for (uint32_t im = d.inj[depth]; im; im &= im - 1)
-        if (W.f[__ffs(im) - 1] == c) return false;
-    const uint32_t p = d.pivot[depth];
-    const BackEntry pe = d.be[p];
-    if (!run_elem_live(entry_delta(g, d, pe), W.run[p], pe.view, key)) return false;
-    for (uint32_t e = d.boff[depth]; e < d.boff[depth + 1]; e++) {
-        if (e == p) continue;
-        const BackEntry be = d.be[e];
-        if (!view_contains(g, d.phase, be.view, be.dir, be.slot, W.f[be.pos], (be.slot << g.id_bits) | c)) return false;
-    }
-    return true;
 }
 
 // Last record r with off[r] <= item, given off[0] <= item < off[n]: a 64-ary search in which every
@@ -101,13 +76,16 @@ __device__ __forceinline__ uint32_t find_record(const unsigned long long* off, u
 
 // ---- Range donation (work stealing) of the depth-first kernel --------------------------------
 // Each wave owns one word per launch: the candidate range [cur, end) of its current record's first
-// depth still to be explored, packed as version (16 bits) | cur (24) | end (24), with the record's
-// index in a second array.  The owner takes its next 64-candidate round by moving cur up; a wave
+// frame still to be explored, packed as version (16 bits) | cur (24) | end (24), with the item
+// group's index in a second array.  The owner takes its next 64-candidate round by moving cur up; a wave
 // out of work takes the upper half of another wave's range by moving that wave's end down to the
 // midpoint.  Both are compare-and-swaps on the one word, so the rounds taken and the halves
-// donated never overlap.  The version changes whenever the owner publishes a new record, so a
-// thief's swap fails if the record index it read belongs to another record.  Ranges only shrink,
-// so every wave's search ends.  (The reference's disabled design: gamma_enumeration.cu:209-357.)
+// donated never overlap.  The owner publishes only when its range is used up, and then another
+// version, so a thief's swap fails if the group index it read belongs to another range.  Ranges only
+// shrink, so every wave's search ends.  All of it is relaxed: the two words are the only data the
+// waves exchange, and the agent-scope acquire and release that ordered them before (an L1
+// invalidation per probe, an L2 write-back per publication) took more than half of the kernel's time.
+// (The reference's disabled design: gamma_enumeration.cu:209-357.)
 constexpr uint32_t kRangeBits = 24;
 constexpr uint32_t kRangeMask = (1u << kRangeBits) - 1;
 constexpr uint32_t kStealRounds = 8;  // victim probes of 64 waves each before a wave gives up
@@ -139,7 +117,7 @@ __device__ __forceinline__ bool steal_range(unsigned long long* donate, const ui
                                             uint32_t lane, uint32_t& rec, uint32_t& lo, uint32_t& hi) {
     for (uint32_t a = 0; a < kStealRounds; a++) {
         const uint32_t v = (gw + 1 + a * 64 + lane * (1 + a)) % total_waves;
-        const unsigned long long w = v != gw ? __hip_atomic_load(donate + v, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT) : 0ull;
+        const unsigned long long w = v != gw ? __hip_atomic_load(donate + v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0ull;
         const uint32_t cur = range_cur(w), end = range_end(w);
         const uint32_t rem = end > cur ? end - cur : 0u;
         uint32_t key = rem << 6 | lane;  // rem < 2^24: fits
@@ -163,192 +141,6 @@ __device__ __forceinline__ bool steal_range(unsigned long long* donate, const ui
     return false;
 }
 
-template <int kMode>
-__global__ void __launch_bounds__(kWaves * 64) k_extend(DevGraph g, StepDesc d, uint32_t d0, uint32_t end_depth, Ring r, MatchOut out,
-                                                         const unsigned long long* split, unsigned long long* work, int schedule,
-                                                         unsigned long long* donate, uint32_t* donate_rec) {
-    extern __shared__ __align__(16) unsigned char lds_raw[];
-    const uint32_t rows = end_depth > d0 + 1 ? end_depth - 1 - d0 : 0u;
-    unsigned char* wave_base = lds_raw + (threadIdx.x >> 6) * wave_lds_bytes(rows);
-    WaveHdr& W = *reinterpret_cast<WaveHdr*>(wave_base);
-    uint32_t* const buf = reinterpret_cast<uint32_t*>(wave_base + sizeof(WaveHdr));  // row (depth - d0)
-    const uint32_t lane = lane_id();
-    const uint32_t nrec = min(*r.in_count, r.in_max);
-    const unsigned long long nitems = split ? split[nrec] : nrec;
-    const uint32_t total_waves = gridDim.x * kWaves;
-    const uint32_t gw = blockIdx.x * kWaves + (threadIdx.x >> 6);
-    unsigned long long my_cnt = 0, my_hash = 0, my_bytes = 0;
-
-    const bool donating = schedule == 2;
-    uint32_t version = 0;
-    unsigned long long item;
-    if (schedule == 0) item = gw;
-    else {
-        unsigned long long t = 0;
-        if (lane == 0) t = atomicAdd(work, 1ull);
-        item = __shfl(t, 0, 64);
-    }
-    for (;;) {
-        // the next item of the launch, else (donating) a range taken from another wave
-        uint32_t rec_idx, chunk = 0, s_lo = 0, s_hi = 0;
-        bool stolen = false;
-        if (item < nitems) {
-            rec_idx = static_cast<uint32_t>(item);
-            if (split) {
-                rec_idx = find_record(split, nrec, item, lane);
-                chunk = static_cast<uint32_t>(item - split[rec_idx]);
-            }
-        } else if (donating && steal_range(donate, donate_rec, total_waves, gw, lane, rec_idx, s_lo, s_hi)) {
-            stolen = true;
-        } else {
-            break;
-        }
-        if (kMode == kWriteAtEnd && uniform(__hip_atomic_load(r.overflow, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) break;
-        if (lane < d0) W.f[lane] = r.in[static_cast<uint64_t>(rec_idx) * d0 + lane];
-        wave_sync();
-        if (lane == 0) {
-            unsigned long long h = 0;
-            W.ph[0] = 0;
-            for (uint32_t j = 0; j < d0; j++) { h += pair_hash(d.order[j], W.f[j]); W.ph[j + 1] = h; }
-        }
-        wave_sync();
-        uint32_t depth = d0;
-        setup_frame(g, d, W, depth, lane, my_bytes, !stolen && chunk == 0);
-        if (split && !stolen) {
-            if (lane == 0) {
-                const uint32_t k = static_cast<uint32_t>(split[rec_idx + 1] - split[rec_idx]);  // chunks of the record
-                const uint32_t width = ((W.tot[d0] + k - 1) / k + 63u) & ~63u;
-                W.cur[d0] = chunk * width;
-                W.tot[d0] = min(W.tot[d0], chunk * width + width);
-            }
-            wave_sync();
-        }
-        // donating: publish the item's first-depth range and take its first round from the word
-        // (a range past 2^24 candidates stays the wave's own)
-        bool published = false;
-        if (donating) {
-            uint32_t lo = stolen ? s_lo : W.cur[d0], hi = stolen ? s_hi : W.tot[d0];
-            published = hi <= kRangeMask;
-            if (published) {
-                version = (version + 1) & 0xFFFFu;
-                uint32_t t = 0, t_end = 0, ok = 0;
-                if (lane == 0) {
-                    __hip_atomic_store(donate_rec + gw, rec_idx, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    __hip_atomic_store(donate + gw,
-                                       static_cast<unsigned long long>(version) << (2 * kRangeBits) |
-                                           static_cast<unsigned long long>(lo) << kRangeBits | hi,
-                                       __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-                    ok = claim_round(donate + gw, t, t_end) ? 1u : 0u;
-                    W.cur[d0] = ok ? t : 0u;
-                    W.tot[d0] = ok ? t_end : 0u;
-                }
-            } else if (stolen && lane == 0) {
-                W.cur[d0] = lo;
-                W.tot[d0] = hi;
-            }
-            wave_sync();
-        }
-        while (true) {
-            if (W.bpos[depth] < W.bcnt[depth]) {
-                const uint32_t c = buf[(depth - d0) * 64u + W.bpos[depth]];
-                wave_sync();
-                if (lane == 0) {
-                    W.bpos[depth] += 1;
-                    W.f[depth] = c;
-                    W.ph[depth + 1] = W.ph[depth] + pair_hash(d.order[depth], c);
-                }
-                wave_sync();
-                depth += 1;
-                setup_frame(g, d, W, depth, lane, my_bytes, true);
-                continue;
-            }
-            if (W.cur[depth] >= W.tot[depth]) {
-                if (depth == d0) {
-                    if (!published) break;
-                    uint32_t ok = 0;
-                    if (lane == 0) {
-                        uint32_t t = 0, t_end = 0;
-                        ok = claim_round(donate + gw, t, t_end) ? 1u : 0u;
-                        if (ok) {
-                            W.cur[d0] = t;
-                            W.tot[d0] = t_end;
-                        }
-                    }
-                    if (!__shfl(ok, 0, 64)) break;
-                    wave_sync();
-                    continue;
-                }
-                depth -= 1;
-                continue;
-            }
-            const uint32_t t = W.cur[depth] + lane;
-            const bool valid = t < W.tot[depth];
-            const uint32_t p = d.pivot[depth];
-            const uint32_t key = valid ? run_elem(g, entry_delta(g, d, d.be[p]), W.run[p], W.nb[depth], t) : 0u;
-            const bool ok = valid && test_candidate(g, d, W, depth, key);
-            const uint32_t c = key & g.id_mask;
-            const uint64_t m = __ballot(ok);
-            wave_sync();
-            if (lane == 0) { W.cur[depth] += 64; my_bytes += 4ull * static_cast<uint32_t>(__popcll(m)); }
-            if (depth + 1 == end_depth) {
-                if (kMode == kCountAtEnd) {
-                    if (ok) {
-                        my_cnt += 1;
-                        my_hash += embedding_hash(W.ph[depth] + pair_hash(d.order[depth], c));
-                    }
-                } else if (m) {
-                    const uint32_t np = static_cast<uint32_t>(__popcll(m));
-                    uint32_t base = 0;
-                    if (lane == 0) base = atomicAdd(r.out_count, np);
-                    base = __shfl(base, 0, 64);
-                    if (static_cast<uint64_t>(base) + np > r.out_cap) {
-                        if (lane == 0) atomicOr(r.overflow, 1u);
-                    } else if (ok) {
-                        uint32_t* o = r.out + static_cast<uint64_t>(base + lanes_below(m)) * end_depth;
-                        for (uint32_t j = 0; j < depth; j++) o[j] = W.f[j];
-                        o[depth] = c;
-                    }
-                }
-            } else {
-                if (ok) buf[(depth - d0) * 64u + lanes_below(m)] = c;
-                if (lane == 0) { W.bcnt[depth] = static_cast<uint32_t>(__popcll(m)); W.bpos[depth] = 0; }
-            }
-            wave_sync();
-        }
-        if (stolen) continue;  // the launch's items are used up: steal again
-        if (schedule == 0) item += total_waves;
-        else {
-            unsigned long long t2 = 0;
-            if (lane == 0) t2 = atomicAdd(work, 1ull);
-            item = __shfl(t2, 0, 64);
-        }
-    }
-    if (kMode == kCountAtEnd) {  // one pair of device atomics per block
-        __shared__ unsigned long long s_cnt[kWaves], s_hash[kWaves];
-        my_cnt = wave_sum_u64(my_cnt);
-        my_hash = wave_sum_u64(my_hash);
-        if (lane == 0) { s_cnt[threadIdx.x >> 6] = my_cnt; s_hash[threadIdx.x >> 6] = my_hash; }
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            unsigned long long c = 0, h = 0;
-            for (uint32_t w = 0; w < kWaves; w++) { c += s_cnt[w]; h += s_hash[w]; }
-            if (c) { atomicAdd(out.count, c); atomicAdd(out.hash, h); }
-        }
-    }
-    if (out.bytes && lane == 0 && my_bytes) atomicAdd(out.bytes, my_bytes);
-}
-
-// ---- One level, flattened over the whole level ------------------------------------------------
-// k_level_len: per record, the view runs of all backward entries of depth d0 (entry order, stored
-// at runs[i * E ..], E = entries of the depth) and the entry whose view sequence is the shortest:
-// that one generates the record's candidates, the others are probed (the candidate set is their
-// intersection whichever entry generates it).  Its length goes to len[i] and, when counting, the
-// record's prefix hash to ph[i].  After an exclusive scan, k_level_flat gives one thread per
-// candidate of the whole level: thread t finds its record by binary search over the offsets, so
-// skewed records spread over the grid, and probes the precomputed runs (no directory or delta
-// segment lookups per candidate).
-// Algorithmic bytes (as the DFS kernel's frames): every view run of the depth's backward lists
-// read once per record, plus 4 per passing candidate (counted by k_level_flat).
 // Membership of key[j] in the sorted a[lo[j], hi[j]) for the active j, N searches advancing in
 // lock-step (each round issues all N loads before using any).  A present key is always probed: a
 // lower-bound search probes the position it ends on unless that position is hi.
@@ -387,6 +179,386 @@ __device__ __forceinline__ void contains_many(const uint32_t* a, const uint32_t*
     }
 }
 
+// Matched vertices, prefix hashes, backward runs and generating lengths of the rows of frame j; the
+// frame's candidates are the rows' generating runs one after another.  Returns their number.
+__device__ __forceinline__ uint32_t dfs_rows(const DevGraph& g, const StepDesc& d, uint32_t d0, uint32_t j, uint32_t rows, const uint32_t* in,
+                                             DfsHdr& H, uint32_t* f, const DfsBuf* buf, uint32_t lane, unsigned long long& bytes,
+                                             bool count_bytes) {
+    const uint32_t depth = d0 + j, e0 = d.boff[depth], ne = d.boff[depth + 1] - e0;
+    uint32_t len = 0, skip = 0;
+    if (lane < rows) {
+        unsigned long long h = 0;
+        uint32_t r = lane;
+        for (uint32_t p = depth; p-- > d0;) {
+            const uint32_t v = buf[p - d0].cand[r];
+            f[p * 64 + lane] = v;
+            h += pair_hash(d.order[p], v);
+            r = buf[p - d0].parent[r];
+        }
+        const uint32_t* rec = in + static_cast<uint64_t>(H.rec[r]) * d0;
+        for (uint32_t p = 0; p < d0; p++) {
+            const uint32_t v = rec[p];
+            f[p * 64 + lane] = v;
+            h += pair_hash(d.order[p], v);
+        }
+        H.ph[lane] = h;
+        RunView rv[kDfsRuns];
+#pragma unroll
+        for (uint32_t e = 0; e < kDfsRuns; e++) {
+            if (e >= ne) break;
+            const BackEntry be = d.be[e0 + e];
+            rv[e] = make_run(g, d.phase, be.view, be.dir, f[be.pos * 64 + lane], be.slot);
+        }
+        uint32_t best = 0xFFFFFFFFu, gen = 0;
+#pragma unroll
+        for (uint32_t e = 0; e < kDfsRuns; e++) {
+            if (e >= ne) break;
+            H.runs[e][lane] = make_uint4(rv[e].lo, rv[e].hi, rv[e].dlo, rv[e].dhi);
+            const uint32_t l = run_seq_len(rv[e], d.be[e0 + e].view);
+            if (l < best) {
+                best = l;
+                gen = e;
+            }
+            if (count_bytes && (j || H.chunk[lane] == 0)) bytes += 4ull * ((rv[e].hi - rv[e].lo) + (rv[e].dhi - rv[e].dlo));
+        }
+        H.gen[lane] = gen;
+        len = best;
+        if (j == 0 && H.chunks[lane] > 1) {  // the record's candidates are cut into whole 64-candidate chunks
+            const uint32_t width = ((best + H.chunks[lane] - 1) / H.chunks[lane] + 63u) & ~63u;
+            skip = min(best, H.chunk[lane] * width);
+            len = min(best - skip, width);
+        }
+    }
+    uint32_t total;
+    const uint32_t pre = wave_prefix(len, total);
+    H.pre[lane] = pre;
+    H.skip[lane] = skip;
+    wave_sync();
+    return uniform(total);
+}
+
+// Depth-first search from the records at depth d0.  The search is latency-bound, and one partial
+// result at a time left most lanes without a candidate (a run has a few elements), so a wave holds a
+// stack of batches instead: a frame's rows are the partial results found by the frame above it, its
+// candidates are flattened over the lanes, and the rows found wait until there are 64 of them or
+// the frame is used up.  A returned-to frame looks its rows up again rather than keeping 64 runs per
+// depth in LDS.  Items (records, or chunks of records) are taken in groups of up to 64, sized so
+// that the grid has a few groups per resident wave.
+constexpr uint32_t kDfsGroupWaves = 2048;
+constexpr int kDfsGridWaves = 2048;
+template <int kMode>
+__global__ void __launch_bounds__(kWaves * 64) k_extend(DevGraph g, StepDesc d, uint32_t d0, uint32_t end_depth, Ring r, MatchOut out,
+                                                         const unsigned long long* split, unsigned long long* work, int schedule,
+                                                         unsigned long long* donate, uint32_t* donate_rec) {
+    extern __shared__ __align__(16) unsigned char lds_raw[];
+    unsigned char* const wave_base = lds_raw + (threadIdx.x >> 6) * wave_lds_bytes(d0, end_depth);
+    DfsHdr& H = *reinterpret_cast<DfsHdr*>(wave_base);
+    uint32_t* const f = reinterpret_cast<uint32_t*>(wave_base + sizeof(DfsHdr));  // f[position * 64 + row]
+    DfsBuf* const buf = reinterpret_cast<DfsBuf*>(wave_base + sizeof(DfsHdr) + (end_depth - 1) * 256u);
+    const uint32_t lane = lane_id();
+    const uint32_t nrec = min(*r.in_count, r.in_max);
+    const unsigned long long nitems = split ? split[nrec] : nrec;
+    const uint32_t total_waves = gridDim.x * kWaves;
+    const uint32_t gw = blockIdx.x * kWaves + (threadIdx.x >> 6);
+    const uint32_t G = static_cast<uint32_t>(min(64ull, max(1ull, nitems / kDfsGroupWaves)));
+    const unsigned long long ngroups = (nitems + G - 1) / G;
+    const uint32_t last = end_depth - 1 - d0;  // the frame whose candidates complete
+    unsigned long long my_cnt = 0, my_hash = 0, my_bytes = 0;
+
+    const bool donating = schedule == 2;
+    uint32_t version = 0;
+    unsigned long long group;
+    if (schedule == 0) group = gw;
+    else {
+        unsigned long long t = 0;
+        if (lane == 0) t = atomicAdd(work, 1ull);
+        group = __shfl(t, 0, 64);
+    }
+    for (;;) {
+        // the next group of the launch, else (donating) a range taken from another wave
+        uint32_t grp, s_lo = 0, s_hi = 0;
+        bool stolen = false;
+        if (group < ngroups) {
+            grp = static_cast<uint32_t>(group);
+        } else if (donating && steal_range(donate, donate_rec, total_waves, gw, lane, grp, s_lo, s_hi)) {
+            stolen = true;
+        } else {
+            break;
+        }
+        if (kMode == kWriteAtEnd && uniform(__hip_atomic_load(r.overflow, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) break;
+        // frame 0: the group's items, one per lane
+        const unsigned long long item = static_cast<unsigned long long>(grp) * G + lane;
+        const uint32_t rows0 = static_cast<uint32_t>(min(static_cast<unsigned long long>(G), nitems - static_cast<unsigned long long>(grp) * G));
+        if (lane < rows0) {
+            uint32_t rec = static_cast<uint32_t>(item), chunk = 0, chunks = 1;
+            if (split) {  // last record with split[rec] <= item
+                uint32_t lo = 0, hi = nrec;
+                while (hi - lo > 1) {
+                    const uint32_t mid = (lo + hi) >> 1;
+                    if (split[mid] <= item) lo = mid;
+                    else hi = mid;
+                }
+                rec = lo;
+                chunk = static_cast<uint32_t>(item - split[rec]);
+                chunks = static_cast<uint32_t>(split[rec + 1] - split[rec]);
+            }
+            H.rec[lane] = rec;
+            H.chunk[lane] = chunk;
+            H.chunks[lane] = chunks;
+        }
+        wave_sync();
+        uint32_t j = 0, built = 0;
+        const uint32_t total0 = dfs_rows(g, d, d0, 0, rows0, r.in, H, f, buf, lane, my_bytes, !stolen && out.bytes);
+        // donating: publish the group's frame 0 candidates and take the first round from the word
+        // (a range past 2^24 candidates stays the wave's own)
+        uint32_t cur0 = stolen ? s_lo : 0u, end0 = stolen ? s_hi : total0;
+        const bool published = donating && end0 <= kRangeMask;
+        if (published) {
+            version = (version + 1) & 0xFFFFu;
+            uint32_t t = 0, t_end = 0;
+            if (lane == 0) {
+                __hip_atomic_store(donate_rec + gw, grp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __builtin_amdgcn_s_waitcnt(0);  // the group's store is done before the range's is issued
+                asm volatile("" ::: "memory");
+                __hip_atomic_store(donate + gw,
+                                   static_cast<unsigned long long>(version) << (2 * kRangeBits) |
+                                       static_cast<unsigned long long>(cur0) << kRangeBits | end0,
+                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (!claim_round(donate + gw, t, t_end)) t = t_end = 0;
+            }
+            cur0 = __shfl(t, 0, 64);
+            end0 = __shfl(t_end, 0, 64);
+        }
+        if (lane == 0) {
+            H.rows[0] = rows0;
+            H.waiting[0] = 0;
+            H.cur[0] = cur0;
+            H.tot[0] = end0;
+        }
+        wave_sync();
+        for (;;) {
+            uint32_t cur = uniform(H.cur[j]), tot = uniform(H.tot[j]);
+            if (j == 0 && cur >= tot && published) {  // frame 0's next round from the published range
+                uint32_t t = 0, t_end = 0;
+                if (lane == 0 && !claim_round(donate + gw, t, t_end)) t = t_end = 0;
+                cur = uniform(__shfl(t, 0, 64));
+                tot = uniform(__shfl(t_end, 0, 64));
+                if (lane == 0) {
+                    H.cur[0] = cur;
+                    H.tot[0] = tot;
+                }
+                wave_sync();
+            }
+            const uint32_t waiting = j < last ? uniform(H.waiting[j]) : 0u;
+            if (waiting >= 64 || (cur >= tot && waiting)) {  // descend with a batch
+                const uint32_t rows = min(64u, waiting);
+                j += 1;
+                const uint32_t t = dfs_rows(g, d, d0, j, rows, r.in, H, f, buf, lane, my_bytes, out.bytes != nullptr);
+                built = j;
+                if (lane == 0) {
+                    H.rows[j] = rows;
+                    H.waiting[j] = 0;
+                    H.cur[j] = 0;
+                    H.tot[j] = t;
+                }
+                wave_sync();
+                continue;
+            }
+            if (cur >= tot) {
+                if (j == 0) break;
+                // back to the frame above: the rows just searched leave its buffer
+                const uint32_t done = uniform(H.rows[j]);
+                j -= 1;
+                const uint32_t left = uniform(H.waiting[j]) - done;  // fewer than 64 * kDfsIlp
+                uint32_t mv[kDfsIlp];
+                uint8_t mp[kDfsIlp];
+#pragma unroll
+                for (uint32_t u = 0; u < kDfsIlp; u++) {
+                    const uint32_t x = lane + 64 * u;
+                    mv[u] = x < left ? buf[j].cand[done + x] : 0u;
+                    mp[u] = x < left ? buf[j].parent[done + x] : 0u;
+                }
+                wave_sync();
+#pragma unroll
+                for (uint32_t u = 0; u < kDfsIlp; u++) {
+                    const uint32_t x = lane + 64 * u;
+                    if (x < left) {
+                        buf[j].cand[x] = mv[u];
+                        buf[j].parent[x] = mp[u];
+                    }
+                }
+                if (lane == 0) H.waiting[j] = left;
+                wave_sync();
+                continue;
+            }
+            if (built != j) {
+                dfs_rows(g, d, d0, j, uniform(H.rows[j]), r.in, H, f, buf, lane, my_bytes, false);
+                built = j;
+            }
+            // one round of frame j's candidates
+            const uint32_t depth = d0 + j, e0 = d.boff[depth], ne = d.boff[depth + 1] - e0;
+            uint32_t k[kDfsIlp], key[kDfsIlp], c[kDfsIlp], gen[kDfsIlp];
+            bool ok[kDfsIlp];
+#pragma unroll
+            for (uint32_t u = 0; u < kDfsIlp; u++) {
+                const uint32_t e = cur + 64 * u + lane;
+                ok[u] = e < tot;
+                k[u] = 0;
+#pragma unroll
+                for (uint32_t st = 32; st; st >>= 1)
+                    if (H.pre[k[u] + st] <= e) k[u] += st;  // rows past the last hold the total
+                gen[u] = H.gen[k[u]];
+                key[u] = 0;
+                if (ok[u]) {
+                    const uint4 x = H.runs[gen[u]][k[u]];
+                    const BackEntry be = d.be[e0 + gen[u]];
+                    const RunView rv{x.x, x.y, x.z, x.w};
+                    key[u] = run_elem(g, entry_delta(g, d, be), rv, run_base_len(rv, be.view), H.skip[k[u]] + (e - H.pre[k[u]]));
+                }
+                c[u] = key[u] & g.id_mask;
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < kDfsIlp; u++) ok[u] = ok[u] && bit_test(d.filter[depth], c[u]);
+            for (uint32_t im = d.inj[depth]; im; im &= im - 1) {
+                const uint32_t q = static_cast<uint32_t>(__ffs(im)) - 1;
+#pragma unroll
+                for (uint32_t u = 0; u < kDfsIlp; u++) ok[u] = ok[u] && f[q * 64 + k[u]] != c[u];
+            }
+            for (uint32_t e = 0; e < ne; e++) {  // every entry's view; the generating entry's base run holds the candidate by construction
+                const BackEntry be = d.be[e0 + e];
+                const uint32_t hi_bits = be.slot << g.id_bits;
+                uint32_t pk[kDfsIlp];
+                bool act[kDfsIlp];
+#pragma unroll
+                for (uint32_t u = 0; u < kDfsIlp; u++) {
+                    pk[u] = hi_bits | c[u];
+                    act[u] = ok[u] && (gen[u] != e || be.view == kViewBaseMinusDelta);
+                }
+                if (e < kDfsRuns) {
+                    uint32_t lo[kDfsIlp], hi[kDfsIlp];
+                    bool sb[kDfsIlp], inb[kDfsIlp], ind[kDfsIlp], need[kDfsIlp];
+#pragma unroll
+                    for (uint32_t u = 0; u < kDfsIlp; u++) {
+                        const uint4 x = H.runs[e][k[u]];
+                        lo[u] = x.x;
+                        hi[u] = x.y;
+                        sb[u] = act[u] && be.view != kViewDelta && gen[u] != e;
+                        inb[u] = false;
+                    }
+                    contains_many<kDfsIlp>(g.arena, lo, hi, pk, sb, inb);
+#pragma unroll
+                    for (uint32_t u = 0; u < kDfsIlp; u++) {
+                        inb[u] = inb[u] || gen[u] == e;
+                        const uint4 x = H.runs[e][k[u]];
+                        lo[u] = x.z;
+                        hi[u] = x.w;
+                        need[u] = act[u] && (be.view == kViewDelta || (be.view == kViewBasePlusDelta ? !inb[u] : be.view == kViewBaseMinusDelta && inb[u]));
+                        ind[u] = false;
+                    }
+                    if (be.view != kViewBase) contains_many<kDfsIlp>(entry_delta(g, d, be), lo, hi, pk, need, ind);
+#pragma unroll
+                    for (uint32_t u = 0; u < kDfsIlp; u++) {
+                        if (!act[u]) continue;
+                        switch (be.view) {
+                            case kViewBase: ok[u] = inb[u]; break;
+                            case kViewBasePlusDelta: ok[u] = inb[u] || ind[u]; break;
+                            case kViewDelta: ok[u] = ind[u]; break;
+                            default: ok[u] = inb[u] && !ind[u]; break;
+                        }
+                    }
+                } else {
+#pragma unroll
+                    for (uint32_t u = 0; u < kDfsIlp; u++)
+                        if (act[u]) ok[u] = view_contains(g, d.phase, be.view, be.dir, be.slot, f[be.pos * 64 + k[u]], pk[u]);
+                }
+            }
+            uint64_t m[kDfsIlp];
+            uint32_t found = 0;
+#pragma unroll
+            for (uint32_t u = 0; u < kDfsIlp; u++) {
+                m[u] = __ballot(ok[u]);
+                found += static_cast<uint32_t>(__popcll(m[u]));
+            }
+            if (lane == 0) {
+                H.cur[j] = cur + 64 * kDfsIlp;
+                my_bytes += 4ull * found;
+            }
+            if (j < last) {
+                uint32_t at = waiting;
+#pragma unroll
+                for (uint32_t u = 0; u < kDfsIlp; u++) {
+                    if (ok[u]) {
+                        const uint32_t x = at + lanes_below(m[u]);
+                        buf[j].cand[x] = c[u];
+                        buf[j].parent[x] = static_cast<uint8_t>(k[u]);
+                    }
+                    at += static_cast<uint32_t>(__popcll(m[u]));
+                }
+                if (lane == 0) H.waiting[j] = at;
+            } else if (kMode == kCountAtEnd) {
+#pragma unroll
+                for (uint32_t u = 0; u < kDfsIlp; u++)
+                    if (ok[u]) {
+                        my_cnt += 1;
+                        my_hash += embedding_hash(H.ph[k[u]] + pair_hash(d.order[depth], c[u]));
+                    }
+            } else if (found) {
+                uint32_t base = 0;
+                if (lane == 0) base = atomicAdd(r.out_count, found);
+                base = __shfl(base, 0, 64);
+                if (static_cast<uint64_t>(base) + found > r.out_cap) {
+                    if (lane == 0) atomicOr(r.overflow, 1u);
+                } else {
+#pragma unroll
+                    for (uint32_t u = 0; u < kDfsIlp; u++) {
+                        if (ok[u]) {
+                            uint32_t* o = r.out + static_cast<uint64_t>(base + lanes_below(m[u])) * end_depth;
+                            for (uint32_t p = 0; p < depth; p++) o[p] = f[p * 64 + k[u]];
+                            o[depth] = c[u];
+                        }
+                        base += static_cast<uint32_t>(__popcll(m[u]));
+                    }
+                }
+            }
+            wave_sync();
+        }
+        if (stolen) continue;  // the launch's items are used up: steal again
+        if (schedule == 0) group += total_waves;
+        else {
+            unsigned long long t2 = 0;
+            if (lane == 0) t2 = atomicAdd(work, 1ull);
+            group = __shfl(t2, 0, 64);
+        }
+    }
+    if (kMode == kCountAtEnd) {  // one pair of device atomics per block
+        __shared__ unsigned long long s_cnt[kWaves], s_hash[kWaves];
+        my_cnt = wave_sum_u64(my_cnt);
+        my_hash = wave_sum_u64(my_hash);
+        if (lane == 0) { s_cnt[threadIdx.x >> 6] = my_cnt; s_hash[threadIdx.x >> 6] = my_hash; }
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            unsigned long long c = 0, h = 0;
+            for (uint32_t w = 0; w < kWaves; w++) { c += s_cnt[w]; h += s_hash[w]; }
+            if (c) { atomicAdd(out.count, c); atomicAdd(out.hash, h); }
+        }
+    }
+    if (out.bytes) {
+        my_bytes = wave_sum_u64(my_bytes);
+        if (lane == 0 && my_bytes) atomicAdd(out.bytes, my_bytes);
+    }
+}
+
+// ---- One level, flattened over the whole level ------------------------------------------------
+// k_level_len: per record, the view runs of all backward entries of depth d0 (entry order, stored
+// at runs[i * E ..], E = entries of the depth) and the entry whose view sequence is the shortest:
+// that one generates the record's candidates, the others are probed (the candidate set is their
+// intersection whichever entry generates it).  Its length goes to len[i] and, when counting, the
+// record's prefix hash to ph[i].  After an exclusive scan, k_level_flat gives one thread per
+// candidate of the whole level: thread t finds its record by binary search over the offsets, so
+// skewed records spread over the grid, and probes the precomputed runs (no directory or delta
+// segment lookups per candidate).
+// Algorithmic bytes (as the DFS kernel's frames): every view run of the depth's backward lists
+// read once per record, plus 4 per passing candidate (counted by k_level_flat).
 constexpr uint32_t kRunsUnroll = 4;  // entries whose lookups are all issued before the first store
 
 __device__ __forceinline__ uint32_t record_runs(const DevGraph& g, const StepDesc& d, uint32_t d0, const uint32_t* f, uint4* runs,
@@ -1245,13 +1417,13 @@ void bitmap_to_list(const uint32_t* bitmap, uint32_t dv, uint32_t* list, uint32_
 
 void extend(const DevGraph& g, const StepDesc& d, uint32_t d0, uint32_t end_depth, int mode, Ring r, MatchOut out,
             const unsigned long long* split, unsigned long long* work_counter, int schedule, int blocks, Donation dn, hipStream_t s) {
-    // Persistent grid: `blocks` (2048 by default: enough waves to fill 256 CUs several times over),
-    // never more than records (a split launch has at least as many items as records with candidates;
-    // a donating launch keeps the full grid, its waves share the heavy records' ranges).
-    blocks = std::min<int>(blocks, static_cast<int>(kMaxDfsBlocks));
+    // Persistent grid: 4 * `blocks` waves, at most the kDfsGridWaves that are resident when two launches
+    // share the chip (waves that start when the items are used up only contend for them), never
+    // more than records (a split launch has at least as many items as records with candidates; a
+    // donating launch keeps the full grid, its waves share the heavy records' ranges).
+    blocks = std::min<int>(std::min<int>(blocks, static_cast<int>(kMaxDfsBlocks)) * 4, kDfsGridWaves) / static_cast<int>(kWaves);
     const int grid = split || schedule == 2 ? blocks : grid_for(r.in_max, kWaves, blocks);
-    const uint32_t rows = end_depth > d0 + 1 ? end_depth - 1 - d0 : 0u;
-    const size_t lds = static_cast<size_t>(kWaves) * wave_lds_bytes(rows);
+    const size_t lds = static_cast<size_t>(kWaves) * wave_lds_bytes(d0, end_depth);
     if (schedule == 2) fill_u32(reinterpret_cast<uint32_t*>(dn.range), 0u, 2ull * grid * kWaves, s);  // every word: nothing to take
     if (mode == kCountAtEnd)
         k_extend<kCountAtEnd><<<grid, kWaves * 64, lds, s>>>(g, d, d0, end_depth, r, out, split, work_counter, schedule, dn.range, dn.rec);

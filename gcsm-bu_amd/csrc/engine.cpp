@@ -929,13 +929,26 @@ std::string Engine::enumerate_rest(Lane& w, QState& qs, uint32_t i, uint32_t ph,
         default: {  // DFS, with or without work stealing (match_gpu.cu:1721-1914)
             const uint32_t t = tail_from(2);
             if (qs.tech.cartesian_product && t < q.n && t > 2 && cpi[t] == kCpTreeProduct) {
-                // depth-first down to the tail, written for the Cartesian product
-                bool ok;
-                uint32_t n_out;
-                uint32_t* out = ring + top;
-                std::string err = extend_to(w, d, ring, count, 2, t, out, (w.ring_words - top) / t, ok, n_out);
-                if (!err.empty()) return err;
-                if (ok) return n_out ? finish_records(w, qs, d, i, t, n_out, out, res_slot) : "";
+                // depth-first down to the tail, written for the Cartesian product; levels of few
+                // records go breadth-first, which gives the depth-first waves enough to start from
+                const uint32_t* rec = ring;
+                uint32_t depth = 2;
+                uint64_t free_at = top;
+                while (depth < t) {
+                    const uint32_t end = depth + 1 < t && count < kDfsMinRecords ? depth + 1 : t;
+                    bool ok;
+                    uint32_t n_out;
+                    uint32_t* out = ring + free_at;
+                    std::string err = extend_to(w, d, rec, count, depth, end, out, (w.ring_words - free_at) / end, ok, n_out);
+                    if (!err.empty()) return err;
+                    if (!ok) break;
+                    if (!n_out) return "";
+                    rec = out;
+                    count = n_out;
+                    depth = end;
+                    free_at += static_cast<uint64_t>(n_out) * end;
+                }
+                return finish_records(w, qs, d, i, depth, count, rec, res_slot);
             }
             return finish_records(w, qs, d, i, 2, count, ring, res_slot);
         }
@@ -1163,9 +1176,10 @@ std::string Engine::finish_records(Lane& w, QState& qs, const StepDesc& d, uint3
     // setting allows, breadth-first levels run first (records stay on the lane's ring: the words
     // above `rec`'s records are free, as every caller leaves its records at the top).
     const uint32_t rows = d.n - 1 - depth;
-    if (!any_depth && rows > opt_.stack_depth && rec >= w.ring && rec < w.ring + w.ring_words) {
+    const bool few = rows > 1 && count < kDfsMinRecords;  // one level first (search returns here with its records)
+    if (!any_depth && (rows > opt_.stack_depth || few) && rec >= w.ring && rec < w.ring + w.ring_words) {
         const uint64_t top = static_cast<uint64_t>(rec - w.ring) + static_cast<uint64_t>(count) * depth;
-        return search(w, qs, d, i, rec, count, depth, top, d.n - 1 - opt_.stack_depth, res_slot);
+        return search(w, qs, d, i, rec, count, depth, top, rows > opt_.stack_depth ? d.n - 1 - opt_.stack_depth : depth + 1, res_slot);
     }
     store_words(rec_count, Words{7, {count, 0, 0, 0, 0, 0, 0}}, w.s);  // [3]: count, [8..9]: work counter
     out.bytes = bytes_ptr(kKExtendCount);

@@ -67,6 +67,9 @@ struct EngineOptions {
 
 constexpr uint64_t kMaxSlotDirectoryBytes = 4ull << 30;
 constexpr uint32_t kSplitMaxRecords = 1u << 14;  // root splitting only below this many records
+// A depth-first search starts from at least this many records where its depths allow: levels of fewer
+// go breadth-first, so that a heavy subtree is not one wave's alone.
+constexpr uint32_t kDfsMinRecords = 2048;
 constexpr uint32_t kMaxLanes = 64;
 // Per-entry view runs a lane's level scratch holds, in records' worth of cp_max_records: levels
 // whose depth has more backward entries than this take fewer records per call.
