@@ -180,9 +180,12 @@ __device__ __forceinline__ void contains_many(const uint32_t* a, const uint32_t*
 }
 
 // Matched vertices, prefix hashes, backward runs and generating lengths of the rows of frame j; the
-// frame's candidates are the rows' generating runs one after another.  Returns their number.
+// frame's candidates are the rows' generating runs one after another.  Returns their number.  The
+// rows of frame 0 are records `stride` words apart; with kRanged, row r takes the elements
+// [chunk[r], chunks[r]) of its run instead of a whole chunk of it.
+template <bool kRanged>
 __device__ __forceinline__ uint32_t dfs_rows(const DevGraph& g, const StepDesc& d, uint32_t d0, uint32_t j, uint32_t rows, const uint32_t* in,
-                                             DfsHdr& H, uint32_t* f, const DfsBuf* buf, uint32_t lane, unsigned long long& bytes,
+                                             uint32_t stride, DfsHdr& H, uint32_t* f, const DfsBuf* buf, uint32_t lane, unsigned long long& bytes,
                                              bool count_bytes) {
     const uint32_t depth = d0 + j, e0 = d.boff[depth], ne = d.boff[depth + 1] - e0;
     uint32_t len = 0, skip = 0;
@@ -195,7 +198,7 @@ __device__ __forceinline__ uint32_t dfs_rows(const DevGraph& g, const StepDesc& 
             h += pair_hash(d.order[p], v);
             r = buf[p - d0].parent[r];
         }
-        const uint32_t* rec = in + static_cast<uint64_t>(H.rec[r]) * d0;
+        const uint32_t* rec = in + static_cast<uint64_t>(H.rec[r]) * stride;
         for (uint32_t p = 0; p < d0; p++) {
             const uint32_t v = rec[p];
             f[p * 64 + lane] = v;
@@ -223,7 +226,12 @@ __device__ __forceinline__ uint32_t dfs_rows(const DevGraph& g, const StepDesc& 
         }
         H.gen[lane] = gen;
         len = best;
-        if (j == 0 && H.chunks[lane] > 1) {  // the record's candidates are cut into whole 64-candidate chunks
+        if (kRanged) {
+            if (j == 0) {
+                skip = min(best, H.chunk[lane]);
+                len = min(best, H.chunks[lane]) - skip;
+            }
+        } else if (j == 0 && H.chunks[lane] > 1) {  // the record's candidates are cut into whole 64-candidate chunks
             const uint32_t width = ((best + H.chunks[lane] - 1) / H.chunks[lane] + 63u) & ~63u;
             skip = min(best, H.chunk[lane] * width);
             len = min(best - skip, width);
@@ -235,6 +243,112 @@ __device__ __forceinline__ uint32_t dfs_rows(const DevGraph& g, const StepDesc& 
     H.skip[lane] = skip;
     wave_sync();
     return uniform(total);
+}
+
+// One round of a frame's candidates, flattened elements cur + 64 u + lane below tot: their row k, vertex
+// c, and whether it extends the row (candidate bitmap, injectivity, every backward entry's view).
+__device__ __forceinline__ void dfs_round(const DevGraph& g, const StepDesc& d, uint32_t depth, uint32_t cur, uint32_t tot, const DfsHdr& H,
+                                          const uint32_t* f, uint32_t lane, uint32_t* k, uint32_t* c, bool* ok) {
+    const uint32_t e0 = d.boff[depth], ne = d.boff[depth + 1] - e0;
+    uint32_t key[kDfsIlp], gen[kDfsIlp];
+#pragma unroll
+    for (uint32_t u = 0; u < kDfsIlp; u++) {
+        const uint32_t e = cur + 64 * u + lane;
+        ok[u] = e < tot;
+        k[u] = 0;
+#pragma unroll
+        for (uint32_t st = 32; st; st >>= 1)
+            if (H.pre[k[u] + st] <= e) k[u] += st;  // rows past the last hold the total
+        gen[u] = H.gen[k[u]];
+        key[u] = 0;
+        if (ok[u]) {
+            const uint4 x = H.runs[gen[u]][k[u]];
+            const BackEntry be = d.be[e0 + gen[u]];
+            const RunView rv{x.x, x.y, x.z, x.w};
+            key[u] = run_elem(g, entry_delta(g, d, be), rv, run_base_len(rv, be.view), H.skip[k[u]] + (e - H.pre[k[u]]));
+        }
+        c[u] = key[u] & g.id_mask;
+    }
+#pragma unroll
+    for (uint32_t u = 0; u < kDfsIlp; u++) ok[u] = ok[u] && bit_test(d.filter[depth], c[u]);
+    for (uint32_t im = d.inj[depth]; im; im &= im - 1) {
+        const uint32_t q = static_cast<uint32_t>(__ffs(im)) - 1;
+#pragma unroll
+        for (uint32_t u = 0; u < kDfsIlp; u++) ok[u] = ok[u] && f[q * 64 + k[u]] != c[u];
+    }
+    for (uint32_t e = 0; e < ne; e++) {  // every entry's view; the generating entry's base run holds the candidate by construction
+        const BackEntry be = d.be[e0 + e];
+        const uint32_t hi_bits = be.slot << g.id_bits;
+        uint32_t pk[kDfsIlp];
+        bool act[kDfsIlp];
+#pragma unroll
+        for (uint32_t u = 0; u < kDfsIlp; u++) {
+            pk[u] = hi_bits | c[u];
+            act[u] = ok[u] && (gen[u] != e || be.view == kViewBaseMinusDelta);
+        }
+        if (e < kDfsRuns) {
+            uint32_t lo[kDfsIlp], hi[kDfsIlp];
+            bool sb[kDfsIlp], inb[kDfsIlp], ind[kDfsIlp], need[kDfsIlp];
+#pragma unroll
+            for (uint32_t u = 0; u < kDfsIlp; u++) {
+                const uint4 x = H.runs[e][k[u]];
+                lo[u] = x.x;
+                hi[u] = x.y;
+                sb[u] = act[u] && be.view != kViewDelta && gen[u] != e;
+                inb[u] = false;
+            }
+            contains_many<kDfsIlp>(g.arena, lo, hi, pk, sb, inb);
+#pragma unroll
+            for (uint32_t u = 0; u < kDfsIlp; u++) {
+                inb[u] = inb[u] || gen[u] == e;
+                const uint4 x = H.runs[e][k[u]];
+                lo[u] = x.z;
+                hi[u] = x.w;
+                need[u] = act[u] && (be.view == kViewDelta || (be.view == kViewBasePlusDelta ? !inb[u] : be.view == kViewBaseMinusDelta && inb[u]));
+                ind[u] = false;
+            }
+            if (be.view != kViewBase) contains_many<kDfsIlp>(entry_delta(g, d, be), lo, hi, pk, need, ind);
+#pragma unroll
+            for (uint32_t u = 0; u < kDfsIlp; u++) {
+                if (!act[u]) continue;
+                switch (be.view) {
+                    case kViewBase: ok[u] = inb[u]; break;
+                    case kViewBasePlusDelta: ok[u] = inb[u] || ind[u]; break;
+                    case kViewDelta: ok[u] = ind[u]; break;
+                    default: ok[u] = inb[u] && !ind[u]; break;
+                }
+            }
+        } else {
+#pragma unroll
+            for (uint32_t u = 0; u < kDfsIlp; u++)
+                if (act[u]) ok[u] = view_contains(g, d.phase, be.view, be.dir, be.slot, f[be.pos * 64 + k[u]], pk[u]);
+        }
+    }
+}
+
+// Back from frame j + 1 to frame j: the rows just searched leave frame j's buffer.
+__device__ __forceinline__ void dfs_pop(DfsHdr& H, DfsBuf* buf, uint32_t j, uint32_t lane) {
+    const uint32_t done = uniform(H.rows[j + 1]);
+    const uint32_t left = uniform(H.waiting[j]) - done;  // fewer than 64 * kDfsIlp
+    uint32_t mv[kDfsIlp];
+    uint8_t mp[kDfsIlp];
+#pragma unroll
+    for (uint32_t u = 0; u < kDfsIlp; u++) {
+        const uint32_t x = lane + 64 * u;
+        mv[u] = x < left ? buf[j].cand[done + x] : 0u;
+        mp[u] = x < left ? buf[j].parent[done + x] : 0u;
+    }
+    wave_sync();
+#pragma unroll
+    for (uint32_t u = 0; u < kDfsIlp; u++) {
+        const uint32_t x = lane + 64 * u;
+        if (x < left) {
+            buf[j].cand[x] = mv[u];
+            buf[j].parent[x] = mp[u];
+        }
+    }
+    if (lane == 0) H.waiting[j] = left;
+    wave_sync();
 }
 
 // Depth-first search from the records at depth d0.  The search is latency-bound, and one partial
@@ -308,7 +422,7 @@ __global__ void __launch_bounds__(kWaves * 64) k_extend(DevGraph g, StepDesc d, 
         }
         wave_sync();
         uint32_t j = 0, built = 0;
-        const uint32_t total0 = dfs_rows(g, d, d0, 0, rows0, r.in, H, f, buf, lane, my_bytes, !stolen && out.bytes);
+        const uint32_t total0 = dfs_rows<false>(g, d, d0, 0, rows0, r.in, d0, H, f, buf, lane, my_bytes, !stolen && out.bytes);
         // donating: publish the group's frame 0 candidates and take the first round from the word
         // (a range past 2^24 candidates stays the wave's own)
         uint32_t cur0 = stolen ? s_lo : 0u, end0 = stolen ? s_hi : total0;
@@ -353,7 +467,7 @@ __global__ void __launch_bounds__(kWaves * 64) k_extend(DevGraph g, StepDesc d, 
             if (waiting >= 64 || (cur >= tot && waiting)) {  // descend with a batch
                 const uint32_t rows = min(64u, waiting);
                 j += 1;
-                const uint32_t t = dfs_rows(g, d, d0, j, rows, r.in, H, f, buf, lane, my_bytes, out.bytes != nullptr);
+                const uint32_t t = dfs_rows<false>(g, d, d0, j, rows, r.in, d0, H, f, buf, lane, my_bytes, out.bytes != nullptr);
                 built = j;
                 if (lane == 0) {
                     H.rows[j] = rows;
@@ -366,112 +480,19 @@ __global__ void __launch_bounds__(kWaves * 64) k_extend(DevGraph g, StepDesc d, 
             }
             if (cur >= tot) {
                 if (j == 0) break;
-                // back to the frame above: the rows just searched leave its buffer
-                const uint32_t done = uniform(H.rows[j]);
                 j -= 1;
-                const uint32_t left = uniform(H.waiting[j]) - done;  // fewer than 64 * kDfsIlp
-                uint32_t mv[kDfsIlp];
-                uint8_t mp[kDfsIlp];
-#pragma unroll
-                for (uint32_t u = 0; u < kDfsIlp; u++) {
-                    const uint32_t x = lane + 64 * u;
-                    mv[u] = x < left ? buf[j].cand[done + x] : 0u;
-                    mp[u] = x < left ? buf[j].parent[done + x] : 0u;
-                }
-                wave_sync();
-#pragma unroll
-                for (uint32_t u = 0; u < kDfsIlp; u++) {
-                    const uint32_t x = lane + 64 * u;
-                    if (x < left) {
-                        buf[j].cand[x] = mv[u];
-                        buf[j].parent[x] = mp[u];
-                    }
-                }
-                if (lane == 0) H.waiting[j] = left;
-                wave_sync();
+                dfs_pop(H, buf, j, lane);
                 continue;
             }
             if (built != j) {
-                dfs_rows(g, d, d0, j, uniform(H.rows[j]), r.in, H, f, buf, lane, my_bytes, false);
+                dfs_rows<false>(g, d, d0, j, uniform(H.rows[j]), r.in, d0, H, f, buf, lane, my_bytes, false);
                 built = j;
             }
             // one round of frame j's candidates
-            const uint32_t depth = d0 + j, e0 = d.boff[depth], ne = d.boff[depth + 1] - e0;
-            uint32_t k[kDfsIlp], key[kDfsIlp], c[kDfsIlp], gen[kDfsIlp];
+            const uint32_t depth = d0 + j;
+            uint32_t k[kDfsIlp], c[kDfsIlp];
             bool ok[kDfsIlp];
-#pragma unroll
-            for (uint32_t u = 0; u < kDfsIlp; u++) {
-                const uint32_t e = cur + 64 * u + lane;
-                ok[u] = e < tot;
-                k[u] = 0;
-#pragma unroll
-                for (uint32_t st = 32; st; st >>= 1)
-                    if (H.pre[k[u] + st] <= e) k[u] += st;  // rows past the last hold the total
-                gen[u] = H.gen[k[u]];
-                key[u] = 0;
-                if (ok[u]) {
-                    const uint4 x = H.runs[gen[u]][k[u]];
-                    const BackEntry be = d.be[e0 + gen[u]];
-                    const RunView rv{x.x, x.y, x.z, x.w};
-                    key[u] = run_elem(g, entry_delta(g, d, be), rv, run_base_len(rv, be.view), H.skip[k[u]] + (e - H.pre[k[u]]));
-                }
-                c[u] = key[u] & g.id_mask;
-            }
-#pragma unroll
-            for (uint32_t u = 0; u < kDfsIlp; u++) ok[u] = ok[u] && bit_test(d.filter[depth], c[u]);
-            for (uint32_t im = d.inj[depth]; im; im &= im - 1) {
-                const uint32_t q = static_cast<uint32_t>(__ffs(im)) - 1;
-#pragma unroll
-                for (uint32_t u = 0; u < kDfsIlp; u++) ok[u] = ok[u] && f[q * 64 + k[u]] != c[u];
-            }
-            for (uint32_t e = 0; e < ne; e++) {  // every entry's view; the generating entry's base run holds the candidate by construction
-                const BackEntry be = d.be[e0 + e];
-                const uint32_t hi_bits = be.slot << g.id_bits;
-                uint32_t pk[kDfsIlp];
-                bool act[kDfsIlp];
-#pragma unroll
-                for (uint32_t u = 0; u < kDfsIlp; u++) {
-                    pk[u] = hi_bits | c[u];
-                    act[u] = ok[u] && (gen[u] != e || be.view == kViewBaseMinusDelta);
-                }
-                if (e < kDfsRuns) {
-                    uint32_t lo[kDfsIlp], hi[kDfsIlp];
-                    bool sb[kDfsIlp], inb[kDfsIlp], ind[kDfsIlp], need[kDfsIlp];
-#pragma unroll
-                    for (uint32_t u = 0; u < kDfsIlp; u++) {
-                        const uint4 x = H.runs[e][k[u]];
-                        lo[u] = x.x;
-                        hi[u] = x.y;
-                        sb[u] = act[u] && be.view != kViewDelta && gen[u] != e;
-                        inb[u] = false;
-                    }
-                    contains_many<kDfsIlp>(g.arena, lo, hi, pk, sb, inb);
-#pragma unroll
-                    for (uint32_t u = 0; u < kDfsIlp; u++) {
-                        inb[u] = inb[u] || gen[u] == e;
-                        const uint4 x = H.runs[e][k[u]];
-                        lo[u] = x.z;
-                        hi[u] = x.w;
-                        need[u] = act[u] && (be.view == kViewDelta || (be.view == kViewBasePlusDelta ? !inb[u] : be.view == kViewBaseMinusDelta && inb[u]));
-                        ind[u] = false;
-                    }
-                    if (be.view != kViewBase) contains_many<kDfsIlp>(entry_delta(g, d, be), lo, hi, pk, need, ind);
-#pragma unroll
-                    for (uint32_t u = 0; u < kDfsIlp; u++) {
-                        if (!act[u]) continue;
-                        switch (be.view) {
-                            case kViewBase: ok[u] = inb[u]; break;
-                            case kViewBasePlusDelta: ok[u] = inb[u] || ind[u]; break;
-                            case kViewDelta: ok[u] = ind[u]; break;
-                            default: ok[u] = inb[u] && !ind[u]; break;
-                        }
-                    }
-                } else {
-#pragma unroll
-                    for (uint32_t u = 0; u < kDfsIlp; u++)
-                        if (act[u]) ok[u] = view_contains(g, d.phase, be.view, be.dir, be.slot, f[be.pos * 64 + k[u]], pk[u]);
-                }
-            }
+            dfs_round(g, d, depth, cur, tot, H, f, lane, k, c, ok);
             uint64_t m[kDfsIlp];
             uint32_t found = 0;
 #pragma unroll
@@ -546,6 +567,259 @@ __global__ void __launch_bounds__(kWaves * 64) k_extend(DevGraph g, StepDesc d, 
         my_bytes = wave_sum_u64(my_bytes);
         if (lane == 0 && my_bytes) atomicAdd(out.bytes, my_bytes);
     }
+}
+
+// ---- Direct steps: whole steps searched depth-first from their anchors --------------------------
+// Pass 0 (grid.y = step): a wave searches groups of the step's anchor pairs, records of depth 2, with
+// the batches above; the global candidate bitmaps filter, so a step needs no local index, no levels
+// and no host.  A few heavy anchors would keep single waves busy for milliseconds, so a wave that has
+// taken its pass's rounds for a task hands the rest of its stack on: the unfinished ranges of its
+// rows and the partial results still waiting become items, up to kDirectTask of them a task, which
+// the waves of the next pass share.  Items go to kDirectShards queues, wave by wave: one counter
+// would serialise their reservations.  A step that is too large (anchors, candidates, items, tasks
+// left after the last pass) is given up: nothing of it is counted, and the host runs it with its local
+// index and levels.  The search is bound by the latency of its rounds (about 10 us each: row lookups, a
+// list element, the bitmap, binary searches); what it saves is the launches, gaps and host waits of the
+// other path, about 30 launches of 3 to 20 us per group of lanes.  Round trips: 32 queries, 1,024-edge
+// batches 5.2 -> 0.77 ms, 2K to 64K edges 46 -> 10.1 ms; one query on the 10K-vertex graph 1.20 -> 0.71 ms;
+// 64 queries, 65,536 edges 58.5 -> 48.3 ms.
+constexpr uint32_t kDirectPoll = 8;     // rounds between looks at the step's state
+constexpr uint32_t kDirectTask = 16;    // items per task
+constexpr uint32_t kDirectPiece = 512;  // candidates of one row per item
+constexpr uint32_t kDirectGrid = 1536;  // blocks of the later passes: what is resident at eight query vertices
+static_assert(kDirectGrid * kWaves % kDirectShards == 0, "the waves of a pass share the queues evenly");
+
+// Appends the active lanes' items (one each) to the pass's queue: record(p) is the lane's vertex at
+// position p below depth.  Returns false when the shard is full.
+template <class Record>
+__device__ __forceinline__ bool direct_emit(const DirectQueue& q, uint32_t shard, uint32_t job, uint32_t depth, bool active, uint32_t lo,
+                                            uint32_t hi, Record record) {
+    const uint64_t m = __ballot(active);
+    const uint32_t n = static_cast<uint32_t>(__popcll(m)), lane = lane_id();
+    if (!n) return true;
+    const uint32_t nt = (n + kDirectTask - 1) / kDirectTask;
+    unsigned long long at = 0;
+    if (lane == 0) at = atomicAdd(q.out_n + shard * 16, static_cast<unsigned long long>(nt) << 32 | n);
+    const uint32_t ib = uniform(__shfl(static_cast<uint32_t>(at), 0, 64)), tb = uniform(__shfl(static_cast<uint32_t>(at >> 32), 0, 64));
+    const bool fits = static_cast<uint64_t>(ib) + n <= q.cap;
+    if (lane < nt && static_cast<uint64_t>(tb) + lane < q.cap)  // a task that does not fit is empty
+        q.out_tasks[static_cast<uint64_t>(shard) * q.cap + tb + lane] =
+            make_uint4(job, depth, ib + lane * kDirectTask, fits ? min(kDirectTask, n - lane * kDirectTask) : 0u);
+    if (!fits) return false;
+    if (active) {
+        uint32_t* o = q.out_items + (static_cast<uint64_t>(shard) * q.cap + ib + lanes_below(m)) * q.stride;
+        o[0] = lo;
+        o[1] = hi;
+        for (uint32_t p = 0; p < depth; p++) o[2 + p] = record(p);
+    }
+    return true;
+}
+
+template <bool kFirst>
+__global__ void __launch_bounds__(kWaves * 64) k_direct_search(DevGraph g, const DirectJob* __restrict__ jobs, DirectCtr* ctr,
+                                                                const uint32_t* pairs, uint32_t cap, DirectQueue q, uint32_t max_rounds,
+                                                                unsigned long long max_work) {
+    extern __shared__ __align__(16) unsigned char lds_raw[];
+    const uint32_t lane = lane_id(), wv = threadIdx.x >> 6;
+    const uint32_t gw = (kFirst ? blockIdx.y * gridDim.x + blockIdx.x : blockIdx.x) * kWaves + wv;
+    const uint32_t out_shard = gw % kDirectShards;
+    unsigned char* const wave_base = lds_raw + wv * q.wave_lds;
+    DfsHdr& H = *reinterpret_cast<DfsHdr*>(wave_base);
+    uint32_t* const f = reinterpret_cast<uint32_t*>(wave_base + sizeof(DfsHdr));
+
+    // this wave's tasks: groups of the job's anchors, or every so-many-th task of its queue
+    uint32_t job = blockIdx.y, ntasks, G = 0, np = 0, t, t_step;
+    if (kFirst) {
+        np = ctr[job].n_pairs;
+        if (!np) return;
+        if (np > cap) {
+            if (blockIdx.x == 0 && threadIdx.x == 0) ctr[job].fail = 1;
+            return;
+        }
+        t = blockIdx.x * kWaves + wv;
+        t_step = gridDim.x * kWaves;
+        G = min(64u, (np + t_step - 1) / t_step);
+        ntasks = (np + G - 1) / G;
+    } else {
+        ntasks = static_cast<uint32_t>(min(q.in_n[out_shard * 16] >> 32, static_cast<unsigned long long>(q.cap)));
+        t = gw / kDirectShards;
+        t_step = gridDim.x * kWaves / kDirectShards;
+    }
+    for (; t < ntasks; t += t_step) {
+        uint32_t depth0 = 2, rows0, stride = 2;
+        const uint32_t* in = pairs + 2ull * cap * job;
+        if (kFirst) {
+            rows0 = min(G, np - t * G);
+            if (lane < rows0) {
+                H.rec[lane] = t * G + lane;
+                H.chunk[lane] = 0;
+                H.chunks[lane] = 0xFFFFFFFFu;
+            }
+        } else {
+            const uint4 task = q.in_tasks[static_cast<uint64_t>(out_shard) * q.cap + t];
+            job = uniform(task.x);
+            depth0 = uniform(task.y);
+            rows0 = uniform(task.w);
+            stride = q.stride;
+            in = q.in_items + (static_cast<uint64_t>(out_shard) * q.cap + uniform(task.z)) * stride;
+            if (lane < rows0) {
+                H.rec[lane] = lane;
+                H.chunk[lane] = in[lane * stride];
+                H.chunks[lane] = in[lane * stride + 1];
+            }
+            in += 2;
+        }
+        DirectCtr& C = ctr[job];
+        const StepDesc& d = jobs[job].d;
+        if (!rows0 || uniform(__hip_atomic_load(&C.fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) continue;
+        unsigned long long my_cnt = 0, my_hash = 0, no_bytes = 0;
+        if (kFirst && d.n == 2) {
+            if (lane < rows0) {
+                const uint32_t* r = in + 2 * (t * G + lane);
+                my_cnt = 1;
+                my_hash = embedding_hash(pair_hash(d.order[0], r[0]) + pair_hash(d.order[1], r[1]));
+            }
+        } else {
+            wave_sync();
+            DfsBuf* const buf = reinterpret_cast<DfsBuf*>(wave_base + sizeof(DfsHdr) + (d.n - 1) * 256u);
+            const uint32_t last = d.n - 1 - depth0;
+            uint32_t j = 0, built = 0, rounds = 0, state = 0;  // state 1: hand the rest on, 2: given up
+            const uint32_t total0 = dfs_rows<true>(g, d, depth0, 0, rows0, in, stride, H, f, buf, lane, no_bytes, false);
+            unsigned long long work = total0;
+            if (lane == 0) {
+                H.rows[0] = rows0;
+                H.waiting[0] = 0;
+                H.cur[0] = 0;
+                H.tot[0] = total0;
+            }
+            wave_sync();
+            for (;;) {
+                const uint32_t cur = uniform(H.cur[j]), tot = uniform(H.tot[j]);
+                const uint32_t waiting = j < last ? uniform(H.waiting[j]) : 0u;
+                const bool down = waiting >= 64 || (cur >= tot && waiting);
+                if (!down && cur >= tot) {
+                    if (j == 0) break;
+                    j -= 1;
+                    dfs_pop(H, buf, j, lane);
+                    continue;
+                }
+                rounds += 1;
+                if (rounds % kDirectPoll == 0 || rounds > max_rounds) {
+                    unsigned long long w = 0;
+                    if (lane == 0) w = atomicAdd(&C.work, work);
+                    work = 0;
+                    if (uniform(__shfl(static_cast<uint32_t>(w > max_work), 0, 64)) ||
+                        uniform(__hip_atomic_load(&C.fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)))
+                        state = 2;
+                    else if (rounds > max_rounds) state = 1;
+                    if (state) break;
+                }
+                if (down) {  // descend with a batch
+                    const uint32_t rows = min(64u, waiting);
+                    j += 1;
+                    const uint32_t tj = dfs_rows<true>(g, d, depth0, j, rows, in, stride, H, f, buf, lane, no_bytes, false);
+                    work += tj;
+                    built = j;
+                    if (lane == 0) {
+                        H.rows[j] = rows;
+                        H.waiting[j] = 0;
+                        H.cur[j] = 0;
+                        H.tot[j] = tj;
+                    }
+                    wave_sync();
+                    continue;
+                }
+                if (built != j) {
+                    dfs_rows<true>(g, d, depth0, j, uniform(H.rows[j]), in, stride, H, f, buf, lane, no_bytes, false);
+                    built = j;
+                }
+                const uint32_t depth = depth0 + j;
+                uint32_t k[kDfsIlp], c[kDfsIlp];
+                bool ok[kDfsIlp];
+                dfs_round(g, d, depth, cur, tot, H, f, lane, k, c, ok);
+                if (lane == 0) H.cur[j] = cur + 64 * kDfsIlp;
+                if (j < last) {
+                    uint32_t at = waiting;
+#pragma unroll
+                    for (uint32_t u = 0; u < kDfsIlp; u++) {
+                        const uint64_t m = __ballot(ok[u]);
+                        if (ok[u]) {
+                            const uint32_t x = at + lanes_below(m);
+                            buf[j].cand[x] = c[u];
+                            buf[j].parent[x] = static_cast<uint8_t>(k[u]);
+                        }
+                        at += static_cast<uint32_t>(__popcll(m));
+                    }
+                    if (lane == 0) H.waiting[j] = at;
+                } else {
+#pragma unroll
+                    for (uint32_t u = 0; u < kDfsIlp; u++)
+                        if (ok[u]) {
+                            my_cnt += 1;
+                            my_hash += embedding_hash(H.ph[k[u]] + pair_hash(d.order[depth], c[u]));
+                        }
+                }
+                wave_sync();
+            }
+            if (state == 1) {  // the rest of every frame, deepest first
+                if (lane == 0) __hip_atomic_store(&C.handed, q.pass + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                uint32_t searched = 0;  // rows of the frame's buffer that are the next frame's
+                bool fits = true;
+                for (uint32_t jj = j + 1; jj-- > 0;) {
+                    const uint32_t rows = uniform(H.rows[jj]), cur = uniform(H.cur[jj]), tot = uniform(H.tot[jj]), depth = depth0 + jj;
+                    if (built != jj) {
+                        dfs_rows<true>(g, d, depth0, jj, rows, in, stride, H, f, buf, lane, no_bytes, false);
+                        built = jj;
+                    }
+                    const uint32_t pre = H.pre[lane], end = lane < 63 ? H.pre[lane + 1] : tot, from = max(cur, pre);
+                    uint32_t lo = 0, hi = 0;
+                    if (lane < rows && from < end) {
+                        lo = H.skip[lane] + (from - pre);
+                        hi = H.skip[lane] + (end - pre);
+                    }
+                    while (__ballot(lo < hi)) {
+                        fits = direct_emit(q, out_shard, job, depth, lo < hi, lo, min(hi, lo + kDirectPiece),
+                                           [&](uint32_t p) { return f[p * 64 + lane]; }) && fits;
+                        lo += kDirectPiece;  // runs are shorter than 2^32 - kDirectPiece
+                    }
+                    if (jj < last) {
+                        const uint32_t waiting = uniform(H.waiting[jj]);
+                        for (uint32_t x0 = searched; x0 < waiting; x0 += 64) {
+                            const uint32_t x = x0 + lane;
+                            const uint32_t par = x < waiting ? buf[jj].parent[x] : 0u, v = x < waiting ? buf[jj].cand[x] : 0u;
+                            fits = direct_emit(q, out_shard, job, depth + 1, x < waiting, 0u, 0xFFFFFFFFu,
+                                               [&](uint32_t p) { return p < depth ? f[p * 64 + par] : v; }) && fits;
+                        }
+                    }
+                    searched = rows;
+                    wave_sync();
+                }
+                if (!fits) state = 2;
+            }
+            if (lane == 0) {
+                if (state == 2) __hip_atomic_store(&C.fail, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (work) atomicAdd(&C.work, work);
+            }
+        }
+        my_cnt = wave_sum_u64(my_cnt);
+        my_hash = wave_sum_u64(my_hash);
+        if (lane == 0 && my_cnt) { atomicAdd(&C.count, my_cnt); atomicAdd(&C.hash, my_hash); }
+    }
+}
+
+__global__ void __launch_bounds__(256) k_direct_commit(const DirectJob* jobs, const DirectCtr* ctr, uint32_t njobs, DirectQueue q,
+                                                       uint32_t committed, unsigned long long* results, uint32_t* state) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < kDirectShards) state[njobs + i] = static_cast<uint32_t>(q.out_n[i * 16] >> 32);
+    if (i >= njobs) return;
+    const DirectCtr& C = ctr[i];
+    if (committed && C.handed < committed) return;  // an earlier commit's
+    const bool on = C.handed == q.pass + 1;
+    state[i] = C.fail ? 1u : on ? 2u : 0u;
+    if (C.fail || on || !C.count) return;
+    unsigned long long* r = results + 4ull * jobs[i].result + 2 * jobs[i].d.phase;
+    atomicAdd(r, C.count);
+    atomicAdd(r + 1, C.hash);
 }
 
 // ---- One level, flattened over the whole level ------------------------------------------------
@@ -1429,6 +1703,24 @@ void extend(const DevGraph& g, const StepDesc& d, uint32_t d0, uint32_t end_dept
         k_extend<kCountAtEnd><<<grid, kWaves * 64, lds, s>>>(g, d, d0, end_depth, r, out, split, work_counter, schedule, dn.range, dn.rec);
     else
         k_extend<kWriteAtEnd><<<grid, kWaves * 64, lds, s>>>(g, d, d0, end_depth, r, out, split, work_counter, schedule, dn.range, dn.rec);
+}
+
+uint32_t direct_wave_lds(uint32_t max_qn) { return wave_lds_bytes(2, std::max<uint32_t>(max_qn, 3)); }
+
+void direct_search(const DevGraph& g, const DirectJob* jobs, uint32_t njobs, DirectCtr* ctr, const uint32_t* pairs, uint32_t cap,
+                   const DirectQueue& q, uint32_t max_rounds, unsigned long long max_work, hipStream_t s) {
+    const size_t lds = static_cast<size_t>(kWaves) * q.wave_lds;
+    if (q.pass == 0) {  // about the waves that are resident at once over all steps, at least eight blocks a step
+        const uint32_t blocks = std::max<uint32_t>(8, std::min<uint32_t>(128, 2048 / njobs));
+        k_direct_search<true><<<dim3(blocks, njobs), kWaves * 64, lds, s>>>(g, jobs, ctr, pairs, cap, q, max_rounds, max_work);
+    } else {
+        k_direct_search<false><<<kDirectGrid, kWaves * 64, lds, s>>>(g, jobs, ctr, pairs, cap, q, max_rounds, max_work);
+    }
+}
+
+void direct_commit(const DirectJob* jobs, const DirectCtr* ctr, uint32_t njobs, const DirectQueue& q, uint32_t committed,
+                   unsigned long long* results, uint32_t* state, hipStream_t s) {
+    k_direct_commit<<<(std::max(njobs, kDirectShards) + 255) / 256, 256, 0, s>>>(jobs, ctr, njobs, q, committed, results, state);
 }
 
 void level_prepare(const DevGraph& g, const StepDesc& d, uint32_t d0, const uint32_t* rec, uint32_t n, const LevelScratch& ls,

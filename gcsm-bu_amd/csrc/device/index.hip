@@ -91,8 +91,8 @@ __global__ void __launch_bounds__(256) k_nlf_touched(DevGraph g, const NlfEntry*
 
 __global__ void __launch_bounds__(256) k_relation_summary(DevGraph g, uint32_t dir, uint32_t slot, uint32_t vrank_u,
                                                           const uint32_t* cand_u, const uint32_t* cand_w, unsigned long long* out) {
-    __shared__ unsigned long long sc[256], ss[256];
-    unsigned long long card = 0, srcs = 0;
+    __shared__ unsigned long long sc[256], ss[256], sq[256];
+    unsigned long long card = 0, srcs = 0, squares = 0;
     for (uint32_t v = blockIdx.x * blockDim.x + threadIdx.x; v < g.dv; v += gridDim.x * blockDim.x) {
         if (g.vrank[v] != vrank_u || !bit_test(cand_u, v)) continue;
         uint32_t lo, hi;
@@ -101,15 +101,21 @@ __global__ void __launch_bounds__(256) k_relation_summary(DevGraph g, uint32_t d
         for (uint32_t k = lo; k < hi; k++) c += bit_test(cand_w, g.arena[k] & g.id_mask) ? 1u : 0u;
         card += c;
         srcs += c ? 1u : 0u;
+        squares += static_cast<unsigned long long>(c) * c;
     }
     sc[threadIdx.x] = card;
     ss[threadIdx.x] = srcs;
+    sq[threadIdx.x] = squares;
     __syncthreads();
     for (int o = 128; o > 0; o >>= 1) {
-        if (threadIdx.x < o) { sc[threadIdx.x] += sc[threadIdx.x + o]; ss[threadIdx.x] += ss[threadIdx.x + o]; }
+        if (threadIdx.x < o) {
+            sc[threadIdx.x] += sc[threadIdx.x + o];
+            ss[threadIdx.x] += ss[threadIdx.x + o];
+            sq[threadIdx.x] += sq[threadIdx.x + o];
+        }
         __syncthreads();
     }
-    if (threadIdx.x == 0) { atomicAdd(&out[0], sc[0]); atomicAdd(&out[1], ss[0]); }
+    if (threadIdx.x == 0) { atomicAdd(&out[0], sc[0]); atomicAdd(&out[1], ss[0]); atomicAdd(&out[2], sq[0]); }
 }
 
 // Work split of the local-index kernels.  The frontier (or queue) size is only known on the device,
@@ -345,6 +351,7 @@ __device__ __forceinline__ uint32_t wave_base(const uint32_t* c, uint32_t base) 
     return base;
 }
 
+template <bool kSets>  // also the sets L(u0), L(u1), else only the pairs
 __device__ __forceinline__ void anchors_body(const DevGraph& g, AnchorLds& lds, const AnchorJob& J, const uint32_t* by_label,
                                              const uint32_t* label_off) {
     if (J.vr0 == kNoVertex) return;
@@ -391,11 +398,11 @@ __device__ __forceinline__ void anchors_body(const DevGraph& g, AnchorLds& lds, 
 #pragma unroll
             for (uint32_t u = 0; u < kFlatIlp; u++) {
                 const uint32_t bit = 1u << (x[u] & 31);
-                fresh[u] = ok[u] && !(atomicOr(&J.L1.bitmap[x[u] >> 5], bit) & bit);
+                fresh[u] = kSets && ok[u] && !(atomicOr(&J.L1.bitmap[x[u] >> 5], bit) & bit);
             }
 #pragma unroll
             for (uint32_t u = 0; u < kFlatIlp; u++) {
-                if (ok[u]) lds.hit[k[u]] = 1u;
+                if (kSets && ok[u]) lds.hit[k[u]] = 1u;
                 mp[u] = __ballot(ok[u]);
                 mf[u] = __ballot(fresh[u]);
                 np += static_cast<uint32_t>(__popcll(mp[u]));
@@ -419,6 +426,7 @@ __device__ __forceinline__ void anchors_body(const DevGraph& g, AnchorLds& lds, 
             }
             __syncthreads();  // the counts are rewritten
         }
+        if (!kSets) continue;
         // a vertex is listed once per label: every one with an anchor is new to L(u0)
         const bool any = lds.hit[tid] != 0;
         const uint64_t m = __ballot(any);
@@ -440,7 +448,7 @@ __device__ __forceinline__ void anchors_body(const DevGraph& g, AnchorLds& lds, 
 
 __global__ void __launch_bounds__(256) k_local_anchors(DevGraph g, AnchorJob J, const uint32_t* by_label, const uint32_t* label_off) {
     __shared__ AnchorLds lds;
-    anchors_body(g, lds, J, by_label, label_off);
+    anchors_body<true>(g, lds, J, by_label, label_off);
 }
 
 // Adds the wave's byte counts to *out (once per wave).
@@ -503,7 +511,17 @@ __global__ void __launch_bounds__(256) k_local_anchors_multi(DevGraph g, const A
                                                              const uint32_t* by_label1, const uint32_t* label_off1) {
     __shared__ AnchorLds lds;
     const AnchorJob J = jobs[blockIdx.y];
-    anchors_body(g, lds, J, J.dir ? by_label1 : by_label0, J.dir ? label_off1 : label_off0);
+    anchors_body<true>(g, lds, J, J.dir ? by_label1 : by_label0, J.dir ? label_off1 : label_off0);
+}
+
+__global__ void __launch_bounds__(256) k_direct_anchors(DevGraph g, const DirectJob* __restrict__ jobs, DirectCtr* ctr, uint32_t* pairs,
+                                                        uint32_t cap, const uint32_t* by_label0, const uint32_t* label_off0,
+                                                        const uint32_t* by_label1, const uint32_t* label_off1) {
+    __shared__ AnchorLds lds;
+    const DirectJob& D = jobs[blockIdx.y];
+    const VSet none{nullptr, nullptr, nullptr, 0};
+    const AnchorJob J{D.d.phase, D.dir, D.slot, D.vr0, D.cand0, D.cand1, pairs + 2ull * cap * blockIdx.y, &ctr[blockIdx.y].n_pairs, cap, none, none};
+    anchors_body<false>(g, lds, J, J.dir ? by_label1 : by_label0, J.dir ? label_off1 : label_off0);
 }
 
 // Every block of a multi-job launch computes off[0..njobs] in LDS, the exclusive prefix of the jobs'
@@ -699,6 +717,14 @@ void local_anchors_multi(const DevGraph& g, const AnchorJob* jobs, uint32_t njob
     if (!njobs) return;
     const dim3 grid(static_cast<uint32_t>(grid_for(max_touched, 256, static_cast<int>(std::max<uint32_t>(16, 4096 / njobs)))), njobs);
     k_local_anchors_multi<<<grid, 256, 0, s>>>(g, jobs, by_label0, label_off0, by_label1, label_off1);
+}
+
+void direct_anchors(const DevGraph& g, const DirectJob* jobs, uint32_t njobs, DirectCtr* ctr, uint32_t* pairs, uint32_t cap,
+                    const uint32_t* by_label0, const uint32_t* label_off0, const uint32_t* by_label1, const uint32_t* label_off1,
+                    uint32_t max_touched, hipStream_t s) {
+    if (!njobs) return;
+    const dim3 grid(static_cast<uint32_t>(grid_for(max_touched, 256, static_cast<int>(std::max<uint32_t>(8, 2048 / njobs)))), njobs);
+    k_direct_anchors<<<grid, 256, 0, s>>>(g, jobs, ctr, pairs, cap, by_label0, label_off0, by_label1, label_off1);
 }
 
 void local_queue_multi(const DevGraph& g, const LocalJob* jobs, uint32_t njobs, int blocks, unsigned long long* bytes, hipStream_t s) {

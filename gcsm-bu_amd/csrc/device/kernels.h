@@ -89,7 +89,8 @@ void nlf_full(const DevGraph& g, const NlfEntry* entries, uint32_t n_entries, co
 void nlf_touched(const DevGraph& g, const NlfEntry* entries, uint32_t n_entries, const NlfGroup* groups, const BatchScratch& w,
                  uint32_t max_touched, int mode, hipStream_t s);
 // Cardinality and number of non-empty sources of the relation u->w restricted to candidates
-// (statisticIndex, indexing.cu:265-301).  out[0] += card, out[1] += #sources.
+// (statisticIndex, indexing.cu:265-301).  out[0] += card, out[1] += #sources, out[2] += the squares of
+// the sources' list lengths.
 void relation_summary(const DevGraph& g, uint32_t dir, uint32_t slot, uint32_t vrank_u, const uint32_t* cand_u,
                       const uint32_t* cand_w, unsigned long long* out, hipStream_t s);
 
@@ -244,6 +245,50 @@ struct Donation {
 void extend(const DevGraph& g, const StepDesc& d, uint32_t d0, uint32_t end_depth, int mode, Ring r,
             MatchOut out, const unsigned long long* split, unsigned long long* work_counter, int schedule, int blocks, Donation dn,
             hipStream_t s);
+// Direct steps: the step of one query edge searched depth-first from its anchor pairs alone (a matching
+// order that starts with the query edge, candidates filtered by the global bitmaps), many steps in one
+// launch.  Step k's anchors go to pairs[2 * cap * k ..] and its state to ctr[k] (clear before
+// direct_anchors).  direct_search's pass 0 searches them, max_rounds rounds of a wave's candidates a
+// task; what is left goes to the queue's out side, which is the next pass's in side.  direct_commit
+// after pass p adds the steps finished since the commit after pass committed - 1 (0: none yet) to
+// results[4 * result + 2 * phase ..] and says in state (pinned host memory) which steps are finished
+// (0), were given up (1: more than cap anchors or max_work candidates, a full queue; nothing of it is
+// counted) or were handed on (2), and behind them the tasks in each shard of the out side.
+struct DirectJob {
+    StepDesc d;                // order starts with the query edge; filters are the global candidates
+    uint32_t dir, slot, vr0;   // relation of the query edge and its first vertex's label rank
+    uint32_t result;           // the query's result row
+    const uint32_t* cand0;     // candidates of the edge's two vertices
+    const uint32_t* cand1;
+};
+struct DirectCtr {             // a line of its own: the steps' atomics do not serialise on each other
+    unsigned long long count, hash;
+    unsigned long long work;   // candidates of the batches searched so far
+    uint32_t n_pairs, fail;
+    uint32_t handed;           // 1 + the last pass that handed tasks on
+    uint32_t pad[23];
+};
+static_assert(sizeof(DirectCtr) == 128, "one cache line per step");
+void direct_anchors(const DevGraph& g, const DirectJob* jobs, uint32_t njobs, DirectCtr* ctr, uint32_t* pairs, uint32_t cap,
+                    const uint32_t* by_label0, const uint32_t* label_off0, const uint32_t* by_label1, const uint32_t* label_off1,
+                    uint32_t max_touched, hipStream_t s);
+constexpr uint32_t kDirectShards = 16;
+struct DirectQueue {           // kDirectShards queues of cap tasks and cap items each
+    const unsigned long long* in_n;  // per shard, 16 words apart: items | tasks << 32
+    const uint4* in_tasks;           // {step, depth, first item, items}
+    const uint32_t* in_items;        // {first, last element of the generating run, matched vertices}
+    unsigned long long* out_n;
+    uint4* out_tasks;
+    uint32_t* out_items;
+    uint32_t cap, stride;            // words per item
+    uint32_t pass;
+    uint32_t wave_lds;               // direct_wave_lds of the largest query
+};
+uint32_t direct_wave_lds(uint32_t max_qn);
+void direct_search(const DevGraph& g, const DirectJob* jobs, uint32_t njobs, DirectCtr* ctr, const uint32_t* pairs, uint32_t cap,
+                   const DirectQueue& q, uint32_t max_rounds, unsigned long long max_work, hipStream_t s);
+void direct_commit(const DirectJob* jobs, const DirectCtr* ctr, uint32_t njobs, const DirectQueue& q, uint32_t committed,
+                   unsigned long long* results, uint32_t* state, hipStream_t s);
 // One level from the n records of depth d0 at rec (n known on the host), flattened over all its
 // candidates: level_prepare writes, per record, the view runs of the depth's backward entries, the
 // entry with the shortest view sequence (it generates the candidates; the others are probed), the

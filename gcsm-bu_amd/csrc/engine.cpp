@@ -5,6 +5,7 @@
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
+#include <limits>
 #include <atomic>
 #include <map>
 #include <mutex>
@@ -67,6 +68,7 @@ Engine::~Engine() {
     if (h_jobs_) (void)hipHostFree(h_jobs_);
     if (h_chain_jobs_) (void)hipHostFree(h_chain_jobs_);
     if (h_tajobs_) (void)hipHostFree(h_tajobs_);
+    if (h_direct_state_) (void)hipHostFree(h_direct_state_);
     if (s_) (void)hipStreamDestroy(s_);
 }
 
@@ -93,6 +95,7 @@ std::string Engine::init(const EngineOptions& o) {
     if (const char* t = std::getenv("CSM_SPLIT_ROOTS")) if (std::atoi(t) == 0) opt_.waves_per_anchor = 1;
     if (const char* t = std::getenv("CSM_SLOT_DIRECTORY")) opt_.slot_directory = std::atoi(t) != 0;
     if (const char* t = std::getenv("CSM_CHAIN_LEVELS")) opt_.chain_levels = std::atoi(t) != 0;
+    if (const char* t = std::getenv("CSM_DIRECT_STEPS")) opt_.direct_steps = std::atoi(t) != 0;
     if (const char* t = std::getenv("CSM_GRAPH_CHAINS")) opt_.graph_chains = std::atoi(t) != 0;
     if (const char* t = std::getenv("CSM_ARENA_SLACK_WORDS")) opt_.arena_slack_words = std::strtoull(t, nullptr, 10);
     if (const char* t = std::getenv("CSM_CP_MAX_RECORDS")) opt_.cp_max_records = static_cast<uint32_t>(std::max(1024L, std::atol(t)));
@@ -284,6 +287,8 @@ std::string Engine::build() {
     add(qs_.size() * 32 + 64);
     add(kKFamilies * 8);
     add(64 * 8);                                                // batch admission words
+    direct_cap_ = 0;
+    for (auto& qs : qs_) direct_cap_ += qs->q.m;
     // free arena blocks: per size class 2^c (c >= 3) at most min(2^20, arena / 2^c) entries, twice
     uint64_t free_entries = 0;
     for (uint32_t c = 3; c < kFreeClasses; c++) free_entries += std::min<uint64_t>(1u << 20, arena_words >> c);
@@ -294,6 +299,9 @@ std::string Engine::build() {
     if (use_sdir)
         for (int d = 0; d < ndirs_; d++) add(sdir_bytes);
     need += 1 << 20;
+    const uint64_t direct_bytes = (2ull * direct_cap_ + 1) * sizeof(DirectJob) + kDirectWords * 4 + 1024;
+    if (opt_.pool_bytes && need + direct_bytes > opt_.pool_bytes) opt_.direct_steps = false;  // a budget that is just enough
+    if (opt_.direct_steps) need += direct_bytes;
     if (opt_.pool_bytes && need > opt_.pool_bytes)
         return tagged(Code::kMemory, "device pool budget too small: need " + std::to_string(need >> 20) + " MiB, budget " + std::to_string(opt_.pool_bytes >> 20) + " MiB");
     std::string err = pool_.reserve(need);
@@ -522,6 +530,13 @@ std::string Engine::build() {
     d_chain_jobs_ = pool_.take<ChainJob>(lanes_.size());
     if (!d_chain_jobs_) return tagged(Code::kMemory, "device pool exhausted (level-chain jobs)");
     CSM_HIP(hipHostMalloc(reinterpret_cast<void**>(&h_chain_jobs_), lanes_.size() * sizeof(ChainJob), hipHostMallocDefault));
+    if (opt_.direct_steps) {
+        d_direct_ = pool_.take<DirectJob>(2ull * direct_cap_ + 1);
+        direct_buf_ = pool_.take<uint32_t>(kDirectWords);
+        if (!d_direct_ || !direct_buf_) return tagged(Code::kMemory, "device pool exhausted (direct steps)");
+    }
+    CSM_HIP(hipHostMalloc(reinterpret_cast<void**>(&h_direct_state_), (kDirectJobs + kDirectShards) * 4ull, hipHostMallocDefault));
+    direct_stale_ = true;
     results_ = pool_.take<unsigned long long>(qs_.size() * 4 + 4);
     prof_bytes_ = pool_.take<unsigned long long>(kKFamilies);
     CSM_HIP(hipMemsetAsync(prof_bytes_, 0, kKFamilies * 8, s_));
@@ -607,24 +622,29 @@ std::string Engine::build() {
         const Query& q = qs.q;
         qs.card.assign(2 * q.m, 0);
         qs.avg.assign(2 * q.m, 0.0f);
+        qs.fan.assign(2 * q.m, 0.0);
+        qs.src.assign(2 * q.m, 0.0);
         for (uint32_t r = 0; r < 2 * q.m; r++) {
             const auto ep = q.rel_endpoints(r);
-            uint64_t c = 0, ns = 0;
+            uint64_t c = 0, ns = 0, sq = 0;
             if (qs.rel[r].valid && qs.matchable) {
-                CSM_HIP(hipMemsetAsync(summary_, 0, 16, s_));
+                CSM_HIP(hipMemsetAsync(summary_, 0, 24, s_));
                 relation_summary(g_, qs.rel[r].dir, qs.rel[r].slot, qs.vrank[ep.first], qs.cand + static_cast<uint64_t>(ep.first) * words_,
                                  qs.cand + static_cast<uint64_t>(ep.second) * words_, summary_, s_);
-                CSM_HIP(hipMemcpyAsync(h_pinned_, summary_, 16, hipMemcpyDeviceToHost, s_));
+                CSM_HIP(hipMemcpyAsync(h_pinned_, summary_, 24, hipMemcpyDeviceToHost, s_));
                 CSM_HIP(hipStreamSynchronize(s_));
-                unsigned long long v[2];
-                std::memcpy(v, h_pinned_, 16);
+                unsigned long long v[3];
+                std::memcpy(v, h_pinned_, 24);
                 c = v[0];
                 ns = v[1];
+                sq = v[2];
             }
             // match_gpu.cu:606-607: 32-bit sums, float division (0/0 gives NaN)
             const uint32_t c32 = static_cast<uint32_t>(c), n32 = static_cast<uint32_t>(ns);
             qs.card[r] = c32;
             qs.avg[r] = static_cast<float>(c32) / static_cast<float>(n32);
+            qs.fan[r] = c ? static_cast<double>(sq) / static_cast<double>(c) : 0.0;
+            qs.src[r] = ns;
         }
     }
     CSM_HIP(hipStreamSynchronize(s_));
@@ -640,6 +660,7 @@ std::string Engine::plan(uint32_t qid, const Technique& t) {
     std::string err = make_plan(qs.q, t.order, qs.card.data(), qs.avg.data(), qs.plan);
     if (!err.empty()) return err;
     qs.planned = true;
+    direct_stale_ = true;
     return "";
 }
 
@@ -804,24 +825,11 @@ std::string Engine::initial_count(const uint32_t* counters, uint32_t& count) {
     return "";
 }
 
-// Step descriptor and initial partial results (depth 2, at the bottom of the lane's ring).  With
-// the anchor pairs as the first two vertices their count is np; otherwise init_from_set runs and
-// `pending` says that its count arrives in the lane's pinned buffer (initial_count, after a wait).
-std::string Engine::enumerate_begin(Lane& w, QState& qs, uint32_t i, uint32_t ph, const VSet* L, uint32_t built, const uint32_t* pairs,
-                                    const uint32_t* n_pairs, uint32_t np, StepDesc& d, bool& pending, uint32_t& count, InitJob* defer) {
+// Everything the search kernels need of one step along the order `o` of the query's vertices: the
+// vertices in `built` are filtered by their local sets, the others by their global candidates.
+StepDesc Engine::step_desc(const QState& qs, uint32_t i, uint32_t ph, const OrderPerEdge& o, const VSet* L, uint32_t built) const {
     const Query& q = qs.q;
-    w.sched = sched_of(qs.tech.strategy);
-    const Plan& p = qs.plan;
-    const uint32_t u0 = q.qe_list[i].first, u1 = q.qe_list[i].second;
-    const uint32_t max_arcs = 2 * max_batch_;
-    auto cand = [&](uint32_t u) { return qs.cand + static_cast<uint64_t>(u) * words_; };
-    fill_u32(w.counters, 0u, kLaneWords - kStepCounters, w.s);
-
-    // ---- step descriptor ----
-    const OrderPerEdge& o = p.orders[i];
-    d = StepDesc{};
-    pending = false;
-    count = 0;
+    StepDesc d{};
     d.n = q.n;
     d.phase = ph;
     uint32_t ne = 0;
@@ -831,7 +839,7 @@ std::string Engine::enumerate_begin(Lane& w, QState& qs, uint32_t i, uint32_t ph
         d.vrank[k] = qs.vrank[u];
         d.boff[k] = static_cast<uint8_t>(ne);
         d.pivot[k] = static_cast<uint8_t>(ne);
-        d.filter[k] = (built >> u & 1u) ? L[u].bitmap : cand(u);
+        d.filter[k] = (built >> u & 1u) ? L[u].bitmap : qs.cand + static_cast<uint64_t>(u) * words_;
         if (k == 0) continue;
         bool have_delta = false;
         for (uint32_t kk = o.bni_offs[k]; kk < o.bni_offs[k + 1]; kk++) {
@@ -853,6 +861,197 @@ std::string Engine::enumerate_begin(Lane& w, QState& qs, uint32_t i, uint32_t ph
         for (uint32_t j = 0; j < k; j++)
             if (d.vrank[j] == d.vrank[k] && !(back >> j & 1u)) d.inj[k] |= static_cast<uint16_t>(1u << j);
     }
+    return d;
+}
+
+// A connected order that starts with query edge (u0, u1): the vertex with the most neighbours in
+// the order so far comes next, then the one with the shortest lists to read.
+static OrderPerEdge direct_order(const Query& q, const std::vector<float>& avg, uint32_t u0, uint32_t u1) {
+    OrderPerEdge o{};
+    uint32_t in = 0, ne = 0;
+    for (uint32_t k = 0; k < q.n; k++) {
+        uint32_t u = k == 0 ? u0 : u1;
+        if (k >= 2) {
+            uint32_t most = 0;
+            float least = 0;
+            for (uint32_t x = 0; x < q.n; x++) {
+                if (in >> x & 1u) continue;
+                uint32_t n = 0;
+                float len = std::numeric_limits<float>::infinity();
+                for (const auto& e : q.nbrs[x])
+                    if (in >> e.first & 1u) {
+                        n++;
+                        len = std::min(len, avg[q.rel(e.first, x)]);
+                    }
+                if (n > most || (n && n == most && len < least)) {
+                    most = n;
+                    least = len;
+                    u = x;
+                }
+            }
+        }
+        o.vs[k] = static_cast<uint8_t>(u);
+        in |= 1u << u;
+        o.bni_offs[k] = static_cast<uint8_t>(ne);
+        for (uint32_t j = 0; j < k; j++)
+            if (q.adjacent(u, o.vs[j])) o.bni[ne++] = static_cast<uint8_t>(j);
+    }
+    o.bni_offs[q.n] = static_cast<uint8_t>(ne);
+    return o;
+}
+
+// Candidates that a search along `o` is expected to test per anchor: per vertex the shortest list of its
+// neighbours so far, thinned by the others it must be in.  Lists are taken at their mean over arcs, not
+// over vertices: a matched vertex was reached over an arc, and on power-law graphs the mean over
+// vertices is 10 to 1,000 times too low (this one is mostly within 3).
+static double direct_estimate(const Query& q, const std::vector<double>& fan, const std::vector<double>& src, const OrderPerEdge& o) {
+    double rec = 1, work = 0;
+    for (uint32_t k = 2; k < q.n; k++) {
+        const uint32_t u = o.vs[k];
+        double least = std::numeric_limits<double>::infinity(), p = 1, p0 = 1;
+        for (uint32_t e = o.bni_offs[k]; e < o.bni_offs[k + 1]; e++) {
+            const uint32_t b = o.vs[o.bni[e]];
+            const double len = fan[q.rel(b, u)], in = std::min(1.0, len / std::max(1.0, src[q.rel(u, b)]));
+            p *= in;
+            if (len < least) { least = len; p0 = in; }
+        }
+        work += rec * least;
+        rec *= least * p / std::max(p0, 1e-12);
+    }
+    return work;
+}
+
+std::string Engine::direct_tables() {
+    direct_steps_.clear();
+    direct_qn_ = 2;
+    for (size_t qi = 0; qi < qs_.size(); qi++) {
+        const QState& qs = *qs_[qi];
+        // the other strategies are searched as the user asked; the stack depth bounds the LDS stack here too
+        if (!qs.planned || !qs.matchable || qs.tech.strategy != SearchStrategy::kDynamicBfsDfs || qs.q.n > opt_.stack_depth + 3) continue;
+        direct_qn_ = std::max(direct_qn_, qs.q.n);
+        for (uint32_t i = 0; i < qs.q.m; i++) {
+            const double arcs = qs.card[qs.q.rel(qs.q.qe_list[i].first, qs.q.qe_list[i].second)];
+            const OrderPerEdge o = direct_order(qs.q, qs.avg, qs.q.qe_list[i].first, qs.q.qe_list[i].second);
+            direct_steps_.push_back({static_cast<uint32_t>(qi), i, arcs / std::max<size_t>(1, host_g_.src.size()), 0, 0});
+            DirectStep& st = direct_steps_.back();
+            st.work = st.anchors * direct_estimate(qs.q, qs.fan, qs.src, o);
+            st.key = std::max(st.anchors / kDirectPairs, st.work / kDirectTry);
+        }
+    }
+    // small steps first: a phase tries a prefix
+    std::stable_sort(direct_steps_.begin(), direct_steps_.end(), [](const DirectStep& x, const DirectStep& y) { return x.key < y.key; });
+    std::vector<DirectJob> jobs[2];
+    for (const DirectStep& st : direct_steps_) {
+        const QState& qs = *qs_[st.q];
+        const uint32_t u0 = qs.q.qe_list[st.i].first, u1 = qs.q.qe_list[st.i].second;
+        const RelInfo& R = qs.rel[qs.q.rel(u0, u1)];
+        const OrderPerEdge o = direct_order(qs.q, qs.avg, u0, u1);
+        for (uint32_t ph = 0; ph < 2; ph++)
+            jobs[ph].push_back(DirectJob{step_desc(qs, st.i, ph, o, nullptr, 0), R.dir, R.slot, qs.vrank[u0], st.q,
+                                         qs.cand + static_cast<uint64_t>(u0) * words_, qs.cand + static_cast<uint64_t>(u1) * words_});
+    }
+    for (uint32_t ph = 0; ph < 2; ph++)
+        if (!jobs[ph].empty())
+            CSM_HIP(hipMemcpyAsync(d_direct_ + static_cast<uint64_t>(ph) * direct_cap_, jobs[ph].data(), jobs[ph].size() * sizeof(DirectJob),
+                                   hipMemcpyHostToDevice, s_));
+    CSM_HIP(hipStreamSynchronize(s_));
+    direct_stale_ = false;
+    return "";
+}
+
+// Steps of the table's front that a phase of `edges` insertions or deletions and nsteps steps tries.  The
+// other steps run lanes_.size() at a time, and what a group of them takes hardly depends on their
+// number, so direct steps pay when they save such a group: about a third of the tried ones are
+// left over, unless there are few candidates in all.
+uint32_t Engine::direct_tries(uint64_t edges, uint32_t nsteps) const {
+    const uint32_t lanes = static_cast<uint32_t>(lanes_.size());
+    uint32_t n = 0;
+    double work = 0;
+    while (n < direct_steps_.size() && direct_steps_[n].key * static_cast<double>(edges) <= 1.0) work += direct_steps_[n++].work * static_cast<double>(edges);
+    auto groups = [&](uint32_t steps) { return (steps + lanes - 1) / lanes; };
+    const uint32_t after = groups(nsteps - n) + (n == nsteps && work <= kDirectFew ? 0u : groups((n + 2) / 3));
+    return after < groups(nsteps) ? n : 0u;
+}
+
+// Tries the first n direct steps of the phase on the main stream; done[q * kMaxQE + i] = 1 for every step
+// (q, i) that is finished, its counts in the results.  `others`: the phase's steps besides these n.
+std::string Engine::direct_phase(uint32_t ph, uint32_t n, uint32_t others, std::vector<char>& done) {
+    for (uint32_t k = 0; k < n; k += kDirectJobs) {
+        const uint32_t nj = std::min(kDirectJobs, n - k);
+        uint32_t* at = direct_buf_;
+        uint64_t left = kDirectWords;
+        auto take = [&](uint64_t words) {
+            uint32_t* p = at;
+            at += words;
+            left -= words;
+            return p;
+        };
+        const uint64_t zero = nj * sizeof(DirectCtr) / 4 + kDirectPasses * kDirectShards * 32;
+        DirectCtr* ctr = reinterpret_cast<DirectCtr*>(take(nj * sizeof(DirectCtr) / 4));
+        unsigned long long* qn = reinterpret_cast<unsigned long long*>(take(kDirectPasses * kDirectShards * 32));
+        const uint32_t cap = static_cast<uint32_t>(std::min<uint64_t>(2 * kDirectPairs, left / 4 / (2ull * nj)) & ~1ull);
+        uint32_t* pairs = take(2ull * nj * cap);
+        DirectQueue q{};
+        q.stride = 2 + direct_qn_;
+        q.cap = static_cast<uint32_t>(left / (2ull * kDirectShards * (4 + q.stride))) & ~3u;
+        uint4* tasks[2];
+        uint32_t* items[2];
+        for (int x = 0; x < 2; x++) tasks[x] = reinterpret_cast<uint4*>(take(4ull * kDirectShards * q.cap));
+        for (int x = 0; x < 2; x++) items[x] = take(static_cast<uint64_t>(q.stride) * kDirectShards * q.cap);
+        q.wave_lds = direct_wave_lds(direct_qn_);
+        const DirectJob* jobs = d_direct_ + static_cast<uint64_t>(ph) * direct_cap_ + k;
+        auto pass = [&](uint32_t p) {
+            q.in_n = qn + (p - 1) * kDirectShards * 16;  // not read by pass 0
+            q.in_tasks = tasks[(p + 1) & 1];
+            q.in_items = items[(p + 1) & 1];
+            q.out_n = qn + p * kDirectShards * 16;
+            q.out_tasks = tasks[p & 1];
+            q.out_items = items[p & 1];
+            q.pass = p;
+            direct_search(g_, jobs, nj, ctr, pairs, cap, q, kDirectRounds, kDirectWork, s_);
+        };
+        fill_u32(direct_buf_, 0u, zero, s_);
+        direct_anchors(g_, jobs, nj, ctr, pairs, cap, bs_[0].by_label, bs_[0].label_off, bs_[1].by_label, bs_[1].label_off, batch_arcs_, s_);
+        const uint32_t behind = others + (n - k - nj);  // steps not in this launch
+        const uint32_t small = n + others <= lanes_.size() ? kDirectTailFew : kDirectTail;
+        for (uint32_t p = 0, before = 2 * small, committed = 0;;) {
+            pass(p);
+            if (p % 2 == 0) {  // one wait for two passes after the first
+                direct_commit(jobs, ctr, nj, q, committed, results_, h_direct_state_, s_);
+                CSM_HIP(hipStreamSynchronize(s_));
+                committed = p + 1;
+                uint32_t left = 0, tasks_left = 0;
+                for (uint32_t x = 0; x < kDirectShards; x++) tasks_left += h_direct_state_[nj + x];
+                for (uint32_t x = 0; x < nj; x++) left += h_direct_state_[x] != 0;
+                // go on while the tasks get fewer, or as long as the steps left are more than one group
+                if (!tasks_left || p + 2 >= kDirectPasses || (2 * tasks_left > before && behind + left <= lanes_.size())) break;
+                before = std::max(tasks_left, small);
+            }
+            p++;
+        }
+        for (uint32_t x = 0; x < nj; x++)
+            if (!h_direct_state_[x]) done[direct_steps_[k + x].q * kMaxQE + direct_steps_[k + x].i] = 1;
+    }
+    return "";
+}
+
+// Step descriptor and initial partial results (depth 2, at the bottom of the lane's ring).  With
+// the anchor pairs as the first two vertices their count is np; otherwise init_from_set runs and
+// `pending` says that its count arrives in the lane's pinned buffer (initial_count, after a wait).
+std::string Engine::enumerate_begin(Lane& w, QState& qs, uint32_t i, uint32_t ph, const VSet* L, uint32_t built, const uint32_t* pairs,
+                                    const uint32_t* n_pairs, uint32_t np, StepDesc& d, bool& pending, uint32_t& count, InitJob* defer) {
+    const Query& q = qs.q;
+    w.sched = sched_of(qs.tech.strategy);
+    const Plan& p = qs.plan;
+    const uint32_t u0 = q.qe_list[i].first, u1 = q.qe_list[i].second;
+    const uint32_t max_arcs = 2 * max_batch_;
+    auto cand = [&](uint32_t u) { return qs.cand + static_cast<uint64_t>(u) * words_; };
+    fill_u32(w.counters, 0u, kLaneWords - kStepCounters, w.s);
+
+    const OrderPerEdge& o = p.orders[i];
+    d = step_desc(qs, i, ph, o, L, built);
+    pending = false;
+    count = 0;
 
     // ---- initial partial results (depth 2) at the bottom of the lane's ring ----
     uint32_t* ring = w.ring;
@@ -1576,12 +1775,32 @@ std::string Engine::run_team_steps(size_t first_lane, std::vector<GroupStep>& it
     return "";
 }
 
-std::string Engine::run_phase(uint32_t ph) {
+std::string Engine::run_phase(uint32_t ph, uint64_t edges) {
     std::vector<std::pair<uint32_t, uint32_t>> steps;  // (query, edge)
+    std::vector<char> finished(qs_.size() * kMaxQE, 0);
+    uint32_t nsteps = 0, tries = 0;
+    for (const auto& qs : qs_)
+        if (qs->planned && qs->matchable) nsteps += qs->q.m;
+    if (opt_.direct_steps && opt_.chain_levels && !opt_.graph_chains && !trace_ && !prof_mask_ && lanes_[0].ring_words >= kDirectRingWords) {
+        if (direct_stale_) {
+            std::string err = direct_tables();
+            if (!err.empty()) return err;
+        }
+        tries = direct_tries(edges, nsteps);
+    }
+    CSM_HIP(hipEventRecord(phase_start_, s_));
+    // the direct steps first if there are no others, else beside them
+    const bool beside = tries && tries < nsteps && team_ > 1;
+    for (uint32_t k = 0; k < tries && beside; k++) finished[direct_steps_[k].q * kMaxQE + direct_steps_[k].i] = 1;
+    if (tries && !beside) {
+        std::string err = direct_phase(ph, tries, nsteps - tries, finished);
+        if (!err.empty()) return err;
+    }
     for (size_t qi = 0; qi < qs_.size(); qi++) {
         const QState& qs = *qs_[qi];
         if (!qs.planned || !qs.matchable) continue;
-        for (uint32_t i = 0; i < qs.q.m; i++) steps.push_back({static_cast<uint32_t>(qi), i});
+        for (uint32_t i = 0; i < qs.q.m; i++)
+            if (!finished[qi * kMaxQE + i]) steps.push_back({static_cast<uint32_t>(qi), i});
     }
     if (steps.empty()) return "";
     // Longest steps first (host time of the same step in the previous batch): the phase ends when
@@ -1593,7 +1812,6 @@ std::string Engine::run_phase(uint32_t ph) {
     };
     std::stable_sort(steps.begin(), steps.end(), [&](const auto& x, const auto& y) { return cost_of(x) > cost_of(y); });
     cost.resize(qs_.size() * kMaxQE, 0.0);
-    CSM_HIP(hipEventRecord(phase_start_, s_));
     const auto phase_t0 = std::chrono::steady_clock::now();
     // Work items for the lanes: steps that build their own local index (slot -1), and steps
     // whose local index a group stage built (their slot).  The main thread stages group g + 1
@@ -1720,6 +1938,23 @@ std::string Engine::run_phase(uint32_t ph) {
     else
         for (size_t li = 0; li < lanes_.size(); li++) th.emplace_back(worker, li);
     std::string stage_err;
+    if (beside) {
+        for (uint32_t k = 0; k < tries; k++) finished[direct_steps_[k].q * kMaxQE + direct_steps_[k].i] = 0;
+        stage_err = direct_phase(ph, tries, nsteps - tries, finished);
+        if (!stage_err.empty()) failed.store(true);
+        std::vector<std::pair<uint32_t, uint32_t>> rest;
+        for (uint32_t k = 0; k < tries; k++)
+            if (!finished[direct_steps_[k].q * kMaxQE + direct_steps_[k].i]) rest.push_back({direct_steps_[k].q, direct_steps_[k].i});
+        std::lock_guard<std::mutex> lk(work.mu);
+        std::stable_sort(rest.begin(), rest.end(), [&](const auto& x, const auto& y) { return cost_of(x) > cost_of(y); });
+        for (const auto& st : rest) {
+            GroupStep g;
+            g.q = st.first;
+            g.i = st.second;
+            work.q.push_back(g);
+        }
+        work.cv.notify_all();
+    }
     for (size_t g0 = 0, gi = 0; g0 < grouped.size() && !failed.load(); g0 += group_, gi++) {
         const uint32_t half = static_cast<uint32_t>(gi % 2);
         {
@@ -1851,6 +2086,7 @@ std::string Engine::run_resident(uint64_t lo, uint64_t n, const uint32_t* hsrc, 
     for (uint64_t k = 0; k < n; k++) (hop[k] ? info.deletes : info.inserts)++;
     const auto t0 = std::chrono::steady_clock::now();
     const uint32_t max_arcs = static_cast<uint32_t>(2 * n);
+    batch_arcs_ = max_arcs;
     if (n == 0) { out.assign(qs_.size(), QueryResult{}); return ""; }
     prof_begin(prof_main_, s_, kKBatchBuild);
     batch_begin(bs_, ndirs_, nvl_, reinterpret_cast<uint32_t*>(results_), static_cast<uint32_t>(qs_.size() * 8), s_);
@@ -1892,7 +2128,7 @@ std::string Engine::run_resident(uint64_t lo, uint64_t n, const uint32_t* hsrc, 
     double match_ms = 0;
     if (info.deletes) {
         const auto a = std::chrono::steady_clock::now();
-        err = run_phase(1);
+        err = run_phase(1, info.deletes);
         if (!err.empty()) return fail(err);
         CSM_HIP(hipStreamSynchronize(s_));
         match_ms += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - a).count();
@@ -1907,7 +2143,7 @@ std::string Engine::run_resident(uint64_t lo, uint64_t n, const uint32_t* hsrc, 
     if (info.inserts) {
         CSM_HIP(hipStreamSynchronize(s_));
         const auto a = std::chrono::steady_clock::now();
-        err = run_phase(0);
+        err = run_phase(0, info.inserts);
         if (!err.empty()) return fail(err);
         CSM_HIP(hipStreamSynchronize(s_));
         match_ms += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - a).count();

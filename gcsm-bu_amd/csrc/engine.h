@@ -59,6 +59,7 @@ struct EngineOptions {
     // slower than direct launches on every workload (C3 34.4-37.3 against 33.7-34.1 ms per batch,
     // C4 85-91 against 81-82 ms, C2 19.7-20.8 against 18.8-18.9 ms).
     bool graph_chains = false;
+    bool direct_steps = true;         // small steps searched from their anchors, many in one launch (CSM_DIRECT_STEPS)
     uint32_t lanes = 32;              // concurrent matching steps, each with its own scratch
     uint32_t team = 0;                // lanes per team (0: a quarter of the lanes, four teams): a team's steps share a
                                       // stream, host waits and multi-step launches
@@ -71,6 +72,27 @@ constexpr uint32_t kSplitMaxRecords = 1u << 14;  // root splitting only below th
 // go breadth-first, so that a heavy subtree is not one wave's alone.
 constexpr uint32_t kDfsMinRecords = 2048;
 constexpr uint32_t kMaxLanes = 64;
+// Direct steps (kernels.h).  A step is tried when its query edge is expected to have at most kDirectPairs
+// anchors in the batch and its search kDirectTry candidates; where one group of lanes would do for all
+// steps, when all of them together are expected to test at most kDirectFew (else a try that fails costs
+// more than it saves: 20 steps 2.9 -> 3.1 ms).  Measured per round trip against kDirectTry: 32 queries,
+// 1K to 64K edges 16.0 ms at 3e3, 14.1 at 1e4, 10.5 at 5e4, 10.2 at 2e5 (46 without direct steps); 64
+// queries, 64K edges 59.0, 55.5, 48.6, 48.1 (58.5 without).
+constexpr uint32_t kDirectPairs = 2048;
+constexpr double kDirectTry = 2e5;
+constexpr double kDirectFew = 3e4;
+// Rounds of a wave per task and pass (8: 0.87 ms for 32 queries and 1,024 edges, 16: 0.77, 24: 0.78),
+// candidates after which a step is given up, passes, tasks that a further pass is worth when the steps left
+// are one group of lanes (and when no more were to begin with), steps per launch, words of scratch, and the
+// smallest ring of a session that uses direct steps (smaller rings exist only by explicit setting, which
+// is about the levels).
+constexpr uint32_t kDirectRounds = 16;
+constexpr unsigned long long kDirectWork = 1ull << 20;
+constexpr uint32_t kDirectPasses = 7;
+constexpr uint32_t kDirectTail = 128, kDirectTailFew = 32;
+constexpr uint32_t kDirectJobs = 1024;
+constexpr uint64_t kDirectWords = 12ull << 20;
+constexpr uint64_t kDirectRingWords = 1ull << 20;
 // Per-entry view runs a lane's level scratch holds, in records' worth of cp_max_records: levels
 // whose depth has more backward entries than this take fewer records per call.
 constexpr uint64_t kLevelRunsPerRecord = 3;
@@ -230,6 +252,7 @@ class Engine {
         uint32_t* cand = nullptr;           // n bitmaps of `words` words
         std::vector<uint32_t> card;
         std::vector<float> avg;
+        std::vector<double> fan, src;       // per relation: mean list length over arcs, vertices with a list
         uint32_t entry0 = 0, entry1 = 0;    // NLF entries [entry0, entry1)
     };
 
@@ -292,7 +315,7 @@ class Engine {
 
     std::string run_resident(uint64_t lo, uint64_t n, const uint32_t* hsrc, const uint32_t* hdst, const uint8_t* hop,
                              std::vector<QueryResult>& out, BatchInfo& info);
-    std::string run_phase(uint32_t ph);
+    std::string run_phase(uint32_t ph, uint64_t edges);
     std::string run_step(Lane& w, QState& qs, uint32_t i, uint32_t ph);
     // the stages of run_step, so that a team can run each stage for all its steps before one wait
     void step_anchors(Lane& w, QState& qs, uint32_t i, uint32_t ph);
@@ -309,7 +332,25 @@ class Engine {
     std::string chain_finish(Lane& w, QState& qs, const StepDesc& d, uint32_t i, uint32_t count, uint32_t res_slot, const LevelChain& c,
                              uint32_t L, const uint32_t* ctr);
     uint32_t slot_of(const QState& qs) const;
+    StepDesc step_desc(const QState& qs, uint32_t i, uint32_t ph, const OrderPerEdge& o, const VSet* L, uint32_t built) const;
     static int sched_of(SearchStrategy st);
+    // Direct steps of the semi-BFS queries, the ones that are tried at the largest batches first, and the job
+    // tables of both phases in this order (rebuilt after a plan).
+    struct DirectStep {
+        uint32_t q, i;
+        double anchors, work;  // expected anchors and tested candidates per edge of the phase
+        double key;            // 1 / the most edges at which the step is tried
+    };
+    std::string direct_tables();
+    uint32_t direct_tries(uint64_t edges, uint32_t nsteps) const;
+    std::string direct_phase(uint32_t ph, uint32_t n, uint32_t others, std::vector<char>& done);
+    std::vector<DirectStep> direct_steps_;
+    uint32_t* direct_buf_ = nullptr;     // [kDirectWords]
+    DirectJob* d_direct_ = nullptr;      // [2][direct_cap_]
+    uint32_t* h_direct_state_ = nullptr; // pinned [kDirectJobs + kDirectShards]
+    uint32_t direct_cap_ = 0;            // steps the tables hold
+    uint32_t direct_qn_ = 0;             // most query vertices among them
+    bool direct_stale_ = true;
     // Teams: lanes [t * team_, (t + 1) * team_) run up to team_ steps at a time on the first lane's
     // stream from one host thread, each stage for all of them before one wait, and their level
     // chains as one chain of multi-job launches (ChainJob tables at d_chain_jobs_ + first lane).
@@ -376,6 +417,7 @@ class Engine {
     DevGraph g_{};
     BatchInput bin_{};
     uint64_t stream_cap_ = 0;       // edges the device stream buffers hold
+    uint32_t batch_arcs_ = 0;       // arcs of the running batch
     uint32_t max_batch_ = 0;        // edges per batch the scratch is sized for
     BatchScratch bs_[2]{};
     NlfEntry* d_entries_ = nullptr;

@@ -36,7 +36,10 @@ std::string Engine::set_tunables(const Tunables& t) {
     if (t.level_blocks && (t.level_blocks < 64 || t.level_blocks > 4096)) return tagged(Code::kArgument, "level_blocks outside 64..4096");
     if (t.semi_bfs_threshold) opt_.semi_bfs_threshold = t.semi_bfs_threshold;
     if (t.waves_per_anchor) opt_.waves_per_anchor = t.waves_per_anchor;
-    if (t.stack_depth) opt_.stack_depth = t.stack_depth;
+    if (t.stack_depth) {
+        opt_.stack_depth = t.stack_depth;
+        direct_stale_ = true;  // the direct steps are the ones whose stack fits
+    }
     if (t.dfs_blocks) opt_.dfs_blocks = t.dfs_blocks;
     if (t.local_blocks) local_grid_ = static_cast<int>(t.local_blocks);
     if (t.team) team_ = std::min<uint32_t>(t.team, std::max<size_t>(1, lanes_.size()));
