@@ -1097,6 +1097,22 @@ uint32_t Engine::slot_of(const QState& qs) const {
                                  qs_.begin());
 }
 
+// First depth from 2 on that is a tree leaf of the step's Cartesian-product tail (the query's size: none).
+uint32_t Engine::product_tail(const QState& qs, uint32_t i) {
+    const uint8_t* cpi = qs.plan.cp_info[i];
+    uint32_t nd = 2;
+    while (nd < qs.q.n && cpi[nd] != kCpTreeProduct && cpi[nd] != kCpTreeSingle) nd++;
+    return nd;
+}
+
+// Depth at which the levels of a breadth-first strategy end: the Cartesian-product tail for kBfs
+// (match_gpu.cu:2129-2294); the query's size for semi-BFS, whose levels end where they hold enough
+// records (match_gpu.cu:1916-2127).
+uint32_t Engine::level_target(const QState& qs, uint32_t i) {
+    if (qs.tech.strategy != SearchStrategy::kBfs) return qs.q.n;
+    return qs.tech.cartesian_product ? std::min(product_tail(qs, i), qs.q.n - 1) : qs.q.n - 1;
+}
+
 // The search of a step from its `count` initial partial results (enumerate_begin).
 std::string Engine::enumerate_rest(Lane& w, QState& qs, uint32_t i, uint32_t ph, const StepDesc& d, uint32_t count) {
     const Query& q = qs.q;
@@ -1111,22 +1127,14 @@ std::string Engine::enumerate_rest(Lane& w, QState& qs, uint32_t i, uint32_t ph,
     }
 
     const uint8_t* cpi = p.cp_info[i];
-    auto tail_from = [&](uint32_t from) {
-        uint32_t nd = from;
-        while (nd < q.n && cpi[nd] != kCpTreeProduct && cpi[nd] != kCpTreeSingle) nd++;
-        return nd;
-    };
     const uint64_t top = 2ull * count;  // first free word of the ring
     switch (qs.tech.strategy) {
-        case SearchStrategy::kDynamicBfsDfs:  // match_gpu.cu:1916-2127
-            if (opt_.chain_levels && !trace_) return search_chained(w, qs, d, i, count, res_slot);
-            return search(w, qs, d, i, ring, count, 2, top, q.n, res_slot);
-        case SearchStrategy::kBfs: {  // match_gpu.cu:2129-2294: breadth-first to the Cartesian-product tail
-            const uint32_t target = qs.tech.cartesian_product ? std::min(tail_from(2), q.n - 1) : q.n - 1;
-            return search(w, qs, d, i, ring, count, 2, top, target, res_slot);
-        }
+        case SearchStrategy::kDynamicBfsDfs:
+        case SearchStrategy::kBfs:
+            if (opt_.chain_levels && !trace_ && level_target(qs, i) > 2) return search_chained(w, qs, d, i, count, res_slot);
+            return search(w, qs, d, i, ring, count, 2, top, level_target(qs, i), res_slot);
         default: {  // DFS, with or without work stealing (match_gpu.cu:1721-1914)
-            const uint32_t t = tail_from(2);
+            const uint32_t t = product_tail(qs, i);
             if (qs.tech.cartesian_product && t < q.n && t > 2 && cpi[t] == kCpTreeProduct) {
                 // depth-first down to the tail, written for the Cartesian product; levels of few
                 // records go breadth-first, which gives the depth-first waves enough to start from
@@ -1202,7 +1210,7 @@ std::string Engine::extend_to(Lane& w, const StepDesc& d, const uint32_t* rec, u
     return "";
 }
 
-// The semi-BFS search of `search` from the initial records (depth 2 at the bottom of the ring)
+// The breadth-first search of `search` (semi-BFS, kBfs) from the initial records (depth 2 at the bottom of the ring)
 // with its levels chained on the device: every writing level and the final counting level are
 // enqueued at once, each reading its size from the counters of the levels before it, and the host
 // waits once.  The chain runs exactly the levels `search` would run while they need no host
@@ -1237,6 +1245,7 @@ std::string Engine::search_chained(Lane& w, QState& qs, const StepDesc& d, uint3
 uint32_t Engine::chain_build(Lane& w, QState& qs, const StepDesc& d, uint32_t i, uint32_t count, LevelChain& c) {
     const uint32_t depth0 = 2, L = d.n - 1 - depth0;
     const uint8_t* cpi = qs.plan.cp_info[i];
+    const uint32_t target = level_target(qs, i);
     c = LevelChain{};
     c.ring = w.ring;
     c.ring_words = w.ring_words;
@@ -1248,7 +1257,8 @@ uint32_t Engine::chain_build(Lane& w, QState& qs, const StepDesc& d, uint32_t i,
         const uint32_t depth = depth0 + k;
         const bool cp_depth = qs.tech.cartesian_product && cpi[depth] == kCpTreeProduct;
         c.cap[k] = level_max_records(d, depth, w.level);
-        c.stop_at[k] = !cp_depth ? 0xFFFFFFFFu : k < L ? opt_.semi_bfs_threshold : 0u;
+        if (qs.tech.strategy == SearchStrategy::kBfs) c.stop_at[k] = depth >= target && (k < L || cp_depth) ? 0u : 0xFFFFFFFFu;
+        else c.stop_at[k] = !cp_depth ? 0xFFFFFFFFu : k < L ? opt_.semi_bfs_threshold : 0u;
     }
     return L;
 }
@@ -1270,7 +1280,7 @@ std::string Engine::chain_finish(Lane& w, QState& qs, const StepDesc& d, uint32_
         const uint32_t depth = depth0 + k;
         if (n == 0) return "";
         if (n > c.cap[k] || n >= c.stop_at[k] || (k < L && ctr[2 * k + 1]))
-            return search(w, qs, d, i, w.ring + off, n, depth, off + static_cast<uint64_t>(n) * depth, d.n, res_slot);
+            return search(w, qs, d, i, w.ring + off, n, depth, off + static_cast<uint64_t>(n) * depth, level_target(qs, i), res_slot);
         if (k == L) return "";  // the leaf level counted
         off += static_cast<uint64_t>(n) * depth;
         n = ctr[2 * k];
@@ -1682,14 +1692,16 @@ std::string Engine::run_team_steps(size_t first_lane, std::vector<GroupStep>& it
             std::string err = initial_count(hl + k * kLaneWords + kStepCounters, count[k]);
             if (!err.empty()) return err;
         }
-    // the level chains of the semi-BFS steps as one chain of multi-job launches, one wait
+    // the level chains of the breadth-first steps as one chain of multi-job launches, one wait
     ChainJob* hj = h_chain_jobs_ + first_lane;
     std::vector<size_t> job_step;
     uint32_t max_l = 0;
     std::vector<char> chained(n, 0);
     for (size_t k = 0; k < n; k++) {
         QState& qs = *qs_[items[k].q];
-        if (!np[k] || !count[k] || qs.q.n <= 2 || qs.tech.strategy != SearchStrategy::kDynamicBfsDfs || !opt_.chain_levels || trace_) continue;
+        if (!np[k] || !count[k] || qs.q.n <= 2 || !opt_.chain_levels || trace_) continue;
+        if (qs.tech.strategy != SearchStrategy::kDynamicBfsDfs && qs.tech.strategy != SearchStrategy::kBfs) continue;
+        if (level_target(qs, items[k].i) <= 2) continue;  // no level to chain
         Lane& w = lane(k);
         ChainJob& J = hj[job_step.size()];
         J = ChainJob{};

@@ -334,6 +334,8 @@ class Engine {
     uint32_t slot_of(const QState& qs) const;
     StepDesc step_desc(const QState& qs, uint32_t i, uint32_t ph, const OrderPerEdge& o, const VSet* L, uint32_t built) const;
     static int sched_of(SearchStrategy st);
+    static uint32_t product_tail(const QState& qs, uint32_t i);
+    static uint32_t level_target(const QState& qs, uint32_t i);
     // Direct steps of the semi-BFS queries, the ones that are tried at the largest batches first, and the job
     // tables of both phases in this order (rebuilt after a plan).
     struct DirectStep {
