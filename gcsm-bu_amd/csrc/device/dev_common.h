@@ -96,6 +96,14 @@ struct StepDesc {
     const uint32_t* filter[kMaxQV];   // candidate bitmap of the vertex at depth d (local or global)
 };
 
+// A pointer that was read from memory (a job table, LDS) as one to global memory.  The compiler takes it for
+// a generic one otherwise, and flat accesses count as LDS accesses too: every wait for one of them
+// also waits for the other kind.  Kernel arguments need no help.
+template <typename T>
+__device__ __forceinline__ T* as_global(T* p) {
+    return (T*)((__attribute__((address_space(1))) T*)reinterpret_cast<uint64_t>(p));  // a cast of the pointer itself would be folded away
+}
+
 // ---- wave64 helpers --------------------------------------------------------------------------
 __device__ __forceinline__ uint32_t lane_id() { return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)); }
 __device__ __forceinline__ uint32_t lanes_below(uint64_t mask) {

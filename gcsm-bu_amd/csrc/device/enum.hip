@@ -60,6 +60,20 @@ __device__ __forceinline__ const uint32_t* entry_delta(const DevGraph& g, const 
     return phase_delta(g, e.dir, d.phase);
 }
 
+// A uniform entry in two scalar loads (its bytes one by one would be vector loads).
+__device__ __forceinline__ BackEntry load_entry(const BackEntry* p) {
+    static_assert(sizeof(BackEntry) == 8 && alignof(BackEntry) == 4, "two words");
+    uint32_t w[2];
+    __builtin_memcpy(w, p, 8);
+    BackEntry e;
+    e.slot = w[0];
+    e.pos = static_cast<uint8_t>(w[1]);
+    e.view = static_cast<uint8_t>(w[1] >> 8);
+    e.dir = static_cast<uint8_t>(w[1] >> 16);
+    e.pad = 0;
+    return e;
+}
+
 // Last record r with off[r] <= item, given off[0] <= item < off[n]: a 64-ary search in which every
 // lane probes one of 64 evenly spaced offsets per round.
 __device__ __forceinline__ uint32_t find_record(const unsigned long long* off, uint32_t n, unsigned long long item, uint32_t lane) {
@@ -270,7 +284,7 @@ __device__ __forceinline__ void dfs_round(const DevGraph& g, const StepDesc& d, 
         c[u] = key[u] & g.id_mask;
     }
 #pragma unroll
-    for (uint32_t u = 0; u < kDfsIlp; u++) ok[u] = ok[u] && bit_test(d.filter[depth], c[u]);
+    for (uint32_t u = 0; u < kDfsIlp; u++) ok[u] = ok[u] && bit_test(as_global(d.filter[depth]), c[u]);
     for (uint32_t im = d.inj[depth]; im; im &= im - 1) {
         const uint32_t q = static_cast<uint32_t>(__ffs(im)) - 1;
 #pragma unroll
@@ -895,14 +909,15 @@ constexpr int kChainFlatGrid = 1024;  // blocks of a chained level's candidate k
 // takes, or large enough for the host's Cartesian-product decision).  Every thread computes the
 // same answer from the host-known start and the counters of the levels before k.
 __device__ __forceinline__ bool chain_at(const LevelChain& c, uint32_t k, uint64_t& off, uint32_t& n) {
+    const uint32_t* ctr = as_global(c.ctr);
     off = c.off0;
     n = c.n0;
     for (uint32_t j = 0;; j++) {
         if (n == 0 || n > c.cap[j] || n >= c.stop_at[j]) return false;
         if (j == k) return true;
-        if (c.ctr[2 * j + 1]) return false;
+        if (ctr[2 * j + 1]) return false;
         off += static_cast<uint64_t>(n) * (c.depth0 + j);
-        n = c.ctr[2 * j];
+        n = ctr[2 * j];
     }
 }
 
@@ -912,6 +927,14 @@ __device__ __forceinline__ bool chain_at(const LevelChain& c, uint32_t k, uint64
 __device__ __forceinline__ void level_len_tiles(const DevGraph& g, const StepDesc& d, uint32_t d0, const uint32_t* rec, uint32_t n,
                                                 unsigned long long* len, uint4* prun, uint4* runs, uint8_t* piv, unsigned long long* ph,
                                                 unsigned long long* tile_sum, unsigned long long* bytes_out) {
+    rec = as_global(rec);
+    len = as_global(len);
+    prun = as_global(prun);
+    runs = as_global(runs);
+    piv = as_global(piv);
+    ph = as_global(ph);
+    tile_sum = as_global(tile_sum);
+    bytes_out = as_global(bytes_out);
     __shared__ unsigned long long s_wave[kLenThreads / 64];
     const uint32_t ne = d.boff[d0 + 1] - d.boff[d0];
     const uint32_t tiles = (n + kLenTile - 1) / kLenTile;
@@ -976,6 +999,8 @@ __global__ void __launch_bounds__(kLenThreads) k_level_len_chain(DevGraph g, Ste
 // Exclusive scan of the lengths in place (total at off[n]): the block of a tile adds the totals of
 // the tiles before it (at most a few thousand words, read by the whole block) to the tile's scan.
 __device__ __forceinline__ void level_scan_tiles(unsigned long long* off, uint32_t n, const unsigned long long* tile_sum) {
+    off = as_global(off);
+    tile_sum = as_global(tile_sum);
     __shared__ unsigned long long s_wave[kLenThreads / 64];
     const uint32_t tiles = (n + kLenTile - 1) / kLenTile;
     if (tiles == 1) return;  // scanned by level_len_tiles
@@ -1080,14 +1105,26 @@ __device__ __forceinline__ void flush_records(const uint32_t* rec, uint32_t d0, 
     uint32_t* o = r.out + static_cast<uint64_t>(wb) * rw;
     for (uint32_t w = lane; w < cnt * rw; w += 64) {
         const uint32_t e = w / rw, q = w - e * rw;
-        o[w] = q < d0 ? rec[static_cast<uint64_t>(sk[e]) * d0 + q] : sc[e];
+        uint32_t v = sc[e];  // read before the branch: one load of either would be a flat one
+        if (q < d0) v = rec[static_cast<uint64_t>(sk[e]) * d0 + q];
+        o[w] = v;
     }
 }
 
 template <int kMode>
 __device__ __forceinline__ void level_flat_body(const DevGraph& g, const StepDesc& d, uint32_t d0, const uint32_t* rec, uint32_t n,
                                                 const unsigned long long* off, const uint4* prun, const uint4* runs, const uint8_t* piv,
-                                                const unsigned long long* ph, Ring r, const MatchOut& out) {
+                                                const unsigned long long* ph, Ring r, MatchOut out) {
+    rec = as_global(rec);
+    off = as_global(off);
+    prun = as_global(prun);
+    runs = as_global(runs);
+    piv = as_global(piv);
+    ph = as_global(ph);
+    r.out = as_global(r.out);
+    r.out_count = as_global(r.out_count);
+    r.overflow = as_global(r.overflow);
+    out = MatchOut{as_global(out.count), as_global(out.hash), as_global(out.bytes)};
     // window of record offsets, relative to off[rb] (a window spans fewer than 2^32 candidates)
     __shared__ uint32_t s_win[4][kLevelStep + 1];
     __shared__ uint32_t s_out[4][kMode == kWriteAtEnd ? 2 * kOutBuf : 1];
@@ -1097,8 +1134,8 @@ __device__ __forceinline__ void level_flat_body(const DevGraph& g, const StepDes
     uint32_t* const out_c = out_k + (kMode == kWriteAtEnd ? kOutBuf : 0);
     uint32_t staged = 0;  // pairs in the wave's LDS buffer
     const uint32_t e0 = d.boff[d0], ne = d.boff[d0 + 1] - e0;
-    const uint32_t* filter = d.filter[d0];
-    const uint32_t qv = d.order[d0];
+    const uint32_t* filter = as_global(d.filter[d0]);
+    const uint32_t qv = d.order[d0], inj = uniform(d.inj[d0]);
     const unsigned long long total = off[n];
     const unsigned long long waves = static_cast<unsigned long long>(gridDim.x) * (blockDim.x >> 6);
     const unsigned long long gw = static_cast<unsigned long long>(blockIdx.x) * (blockDim.x >> 6) + (threadIdx.x >> 6);
@@ -1185,7 +1222,7 @@ __device__ __forceinline__ void level_flat_body(const DevGraph& g, const StepDes
 #pragma unroll
         for (uint32_t j = 0; j < kLevelIlp; j++)
             ok[j] = ok[j] && run_elem_live(phase_delta(g, pv[j] >> 6, d.phase), rv[j], (pv[j] >> 4) & 3u, key[j]);
-        for (uint32_t im = d.inj[d0]; im; im &= im - 1) {
+        for (uint32_t im = inj; im; im &= im - 1) {
             const uint32_t q = static_cast<uint32_t>(__ffs(im)) - 1;
 #pragma unroll
             for (uint32_t j = 0; j < kLevelIlp; j++) ok[j] = ok[j] && rec[static_cast<uint64_t>(k[j]) * d0 + q] != c[j];
@@ -1193,7 +1230,7 @@ __device__ __forceinline__ void level_flat_body(const DevGraph& g, const StepDes
         // probe the other entries' precomputed runs (each with its own slot bits); the searches of
         // the kLevelIlp candidates advance in lock-step so their loads are in flight together
         for (uint32_t e = 0; e < ne; e++) {
-            const BackEntry be = d.be[e0 + e];
+            const BackEntry be = load_entry(d.be + e0 + e);
             const uint32_t hi_bits = be.slot << g.id_bits;
             // runs as {lo, hi} / {dlo, dhi} halves: the delta half is loaded only for views that use it
             const uint2* rh = reinterpret_cast<const uint2*>(runs);
@@ -1319,7 +1356,7 @@ __global__ void __launch_bounds__(256) k_level_flat_chain(DevGraph g, StepDesc d
 __global__ void __launch_bounds__(kLenThreads) k_level_len_chain_multi(DevGraph g, const ChainJob* jobs, uint32_t k) {
     const ChainJob& J = jobs[blockIdx.y];
     if (k > J.L) return;
-    if (k == 0 && blockIdx.x == 0 && threadIdx.x < 2 * kMaxQV) J.c.ctr[threadIdx.x] = 0;
+    if (k == 0 && blockIdx.x == 0 && threadIdx.x < 2 * kMaxQV) as_global(J.c.ctr)[threadIdx.x] = 0;
     uint64_t off;
     uint32_t n;
     if (!chain_at(J.c, k, off, n)) return;
@@ -1385,7 +1422,13 @@ __global__ void k_init_from_pairs(const uint32_t* pairs, const uint32_t* n_pairs
 // its survivors' output once per round of kInitIlp elements a lane, whose loads are in flight
 // together: most start vertices have a run of a few elements.
 constexpr uint32_t kInitIlp = 4;
-__device__ __forceinline__ void init_set_body(const DevGraph& g, const InitJob& J) {
+__device__ __forceinline__ void init_set_body(const DevGraph& g, InitJob J) {
+    J.list = as_global(J.list);
+    J.len = as_global(J.len);
+    J.filter_b = as_global(J.filter_b);
+    J.out = as_global(J.out);
+    J.out_count = as_global(J.out_count);
+    J.overflow = as_global(J.overflow);
     __shared__ uint32_t s_pre[4][65];
     __shared__ RunView s_run[4][64];
     __shared__ uint32_t s_nb[4][64], s_v[4][64];

@@ -205,7 +205,7 @@ __device__ __forceinline__ uint64_t expand_flat(const DevGraph& g, FlatLds& lds,
                 y[u] = key[u] & g.id_mask;
             }
 #pragma unroll
-            for (uint32_t u = 0; u < kFlatIlp; u++) ok[u] = ok[u] && bit_test(lds.cand[wv][kk[u]], y[u]);
+            for (uint32_t u = 0; u < kFlatIlp; u++) ok[u] = ok[u] && bit_test(as_global(lds.cand[wv][kk[u]]), y[u]);
 #pragma unroll
             for (uint32_t u = 0; u < kFlatIlp; u++) {
                 const uint32_t v = lds.vd[wv][kk[u]];
@@ -216,7 +216,7 @@ __device__ __forceinline__ uint64_t expand_flat(const DevGraph& g, FlatLds& lds,
             for (uint32_t u = 0; u < kFlatIlp; u++) {
                 const uint32_t bit = 1u << (y[u] & 31);
                 // else offered by another visitor
-                fresh[u] = ok[u] && !(atomicOr(const_cast<uint32_t*>(lds.bm[wv][kk[u]]) + (y[u] >> 5), bit) & bit);
+                fresh[u] = ok[u] && !(atomicOr(as_global(const_cast<uint32_t*>(lds.bm[wv][kk[u]])) + (y[u] >> 5), bit) & bit);
             }
             emit(fresh, y, jj);
 #pragma unroll
@@ -286,7 +286,7 @@ __device__ __forceinline__ uint64_t check_flat(const DevGraph& g, FlatLds& lds, 
                 }
                 bool hit[kFlatIlp];
 #pragma unroll
-                for (uint32_t u = 0; u < kFlatIlp; u++) hit[u] = act[u] && bit_test(lds.bm[wv][o[u]], fk[u] & g.id_mask);
+                for (uint32_t u = 0; u < kFlatIlp; u++) hit[u] = act[u] && bit_test(as_global(lds.bm[wv][o[u]]), fk[u] & g.id_mask);
 #pragma unroll
                 for (uint32_t u = 0; u < kFlatIlp; u++) {
                     const uint32_t v = lds.vd[wv][o[u]];
@@ -309,6 +309,8 @@ __device__ __forceinline__ uint64_t check_flat(const DevGraph& g, FlatLds& lds, 
 // one cache line serialise at about 9 ns, and each is a round trip for its wave.
 template <uint32_t N>
 __device__ __forceinline__ void append_fresh(const bool* fresh, const uint32_t* y, uint32_t* list, uint32_t* len, uint32_t cap) {
+    list = as_global(list);
+    len = as_global(len);
     uint64_t m[N];
     uint32_t n = 0;
 #pragma unroll
@@ -334,6 +336,8 @@ __device__ __forceinline__ void append_fresh(const bool* fresh, const uint32_t* 
 // pairs and new set members with one device atomic each: the counters of a step share a cache line,
 // where atomics serialise.  (One thread per vertex walked a hub's run alone, three dependent atomics
 // an arc: 264 us for a triangle query's three steps on a 500,000-edge batch.)
+__device__ __forceinline__ VSet global_set(const VSet& v) { return VSet{as_global(v.bitmap), as_global(v.list), as_global(v.len), v.cap}; }
+
 struct AnchorLds {
     uint32_t pre[256], lo[256], v[256], hit[256];
     uint32_t n[2][4], base[2];
@@ -355,6 +359,9 @@ template <bool kSets>  // also the sets L(u0), L(u1), else only the pairs
 __device__ __forceinline__ void anchors_body(const DevGraph& g, AnchorLds& lds, const AnchorJob& J, const uint32_t* by_label,
                                              const uint32_t* label_off) {
     if (J.vr0 == kNoVertex) return;
+    const uint32_t *cand0 = as_global(J.cand0), *cand1 = as_global(J.cand1);
+    const VSet L0 = global_set(J.L0), L1 = global_set(J.L1);
+    uint32_t *pairs = as_global(J.pairs), *n_pairs = as_global(J.n_pairs);
     const uint32_t tid = threadIdx.x, lane = lane_id(), wv = tid >> 6;
     const uint32_t first = label_off[J.vr0], T = label_off[J.vr0 + 1] - first;
     const uint32_t* touched = by_label + first;
@@ -365,7 +372,7 @@ __device__ __forceinline__ void anchors_body(const DevGraph& g, AnchorLds& lds, 
         uint32_t v = 0, lo = 0, hi = 0;
         if (i < T) {
             v = touched[i];
-            const bool cand = bit_test(J.cand0, v);
+            const bool cand = bit_test(cand0, v);
             const uint4 s = g.delta[J.dir].seg[v];
             const uint32_t off = J.phase ? s.z : s.x, len = J.phase ? s.w : s.y;
             if (cand && len) slot_range(dl, off, off + len, J.slot, g.id_bits, lo, hi);
@@ -394,11 +401,11 @@ __device__ __forceinline__ void anchors_body(const DevGraph& g, AnchorLds& lds, 
             }
             uint32_t np = 0, nf = 0;
 #pragma unroll
-            for (uint32_t u = 0; u < kFlatIlp; u++) ok[u] = ok[u] && bit_test(J.cand1, x[u]);
+            for (uint32_t u = 0; u < kFlatIlp; u++) ok[u] = ok[u] && bit_test(cand1, x[u]);
 #pragma unroll
             for (uint32_t u = 0; u < kFlatIlp; u++) {
                 const uint32_t bit = 1u << (x[u] & 31);
-                fresh[u] = kSets && ok[u] && !(atomicOr(&J.L1.bitmap[x[u] >> 5], bit) & bit);
+                fresh[u] = kSets && ok[u] && !(atomicOr(&L1.bitmap[x[u] >> 5], bit) & bit);
             }
 #pragma unroll
             for (uint32_t u = 0; u < kFlatIlp; u++) {
@@ -412,15 +419,15 @@ __device__ __forceinline__ void anchors_body(const DevGraph& g, AnchorLds& lds, 
             __syncthreads();
             if (tid < 2) {
                 const uint32_t c = wave_total(lds.n[tid]);
-                lds.base[tid] = c ? atomicAdd(tid ? J.L1.len : J.n_pairs, c) : 0u;
+                lds.base[tid] = c ? atomicAdd(tid ? L1.len : n_pairs, c) : 0u;
             }
             __syncthreads();
             uint32_t p = wave_base(lds.n[0], lds.base[0]), f = wave_base(lds.n[1], lds.base[1]);
 #pragma unroll
             for (uint32_t u = 0; u < kFlatIlp; u++) {
                 const uint32_t qp = p + lanes_below(mp[u]), qf = f + lanes_below(mf[u]);
-                if (ok[u] && qp < J.max_pairs) reinterpret_cast<uint2*>(J.pairs)[qp] = make_uint2(lds.v[k[u]], x[u]);
-                if (fresh[u] && qf < J.L1.cap) J.L1.list[qf] = x[u];
+                if (ok[u] && qp < J.max_pairs) reinterpret_cast<uint2*>(pairs)[qp] = make_uint2(lds.v[k[u]], x[u]);
+                if (fresh[u] && qf < L1.cap) L1.list[qf] = x[u];
                 p += static_cast<uint32_t>(__popcll(mp[u]));
                 f += static_cast<uint32_t>(__popcll(mf[u]));
             }
@@ -434,13 +441,13 @@ __device__ __forceinline__ void anchors_body(const DevGraph& g, AnchorLds& lds, 
         __syncthreads();
         if (tid == 0) {
             const uint32_t c = wave_total(lds.n[0]);
-            lds.base[0] = c ? atomicAdd(J.L0.len, c) : 0u;
+            lds.base[0] = c ? atomicAdd(L0.len, c) : 0u;
         }
         __syncthreads();
         if (any) {
-            atomicOr(&J.L0.bitmap[v >> 5], 1u << (v & 31));
+            atomicOr(&L0.bitmap[v >> 5], 1u << (v & 31));
             const uint32_t q = wave_base(lds.n[0], lds.base[0]) + lanes_below(m);
-            if (q < J.L0.cap) J.L0.list[q] = v;
+            if (q < L0.cap) L0.list[q] = v;
         }
         __syncthreads();  // the LDS rows are rewritten by the next tile
     }
@@ -530,7 +537,7 @@ __global__ void __launch_bounds__(256) k_direct_anchors(DevGraph g, const Direct
 template <int kKind>
 __device__ __forceinline__ void job_offsets(const LocalJob* jobs, uint32_t njobs, uint32_t max_len, uint32_t* off) {
     for (uint32_t t = threadIdx.x; t < njobs; t += blockDim.x)
-        off[t + 1] = min(kKind == 0 ? *jobs[t].frontier_len : *jobs[t].queue_len, max_len);
+        off[t + 1] = min(*as_global(kKind == 0 ? jobs[t].frontier_len : jobs[t].queue_len), max_len);
     __syncthreads();
     if (threadIdx.x < 64) {
         uint32_t carry = 0;
@@ -586,10 +593,10 @@ __device__ __forceinline__ void append_jobs(const bool* flag, const uint32_t* y,
         if (!flag[u]) continue;
         const LocalJob& J = jobs[j[u]];
         if (to_queue) {
-            J.queue[atomicAdd(J.queue_len, 1u)] = y[u];
+            as_global(J.queue)[atomicAdd(as_global(J.queue_len), 1u)] = y[u];
         } else {
-            const uint32_t p = atomicAdd(J.out.len, 1u);
-            if (p < J.out.cap) J.out.list[p] = y[u];
+            const uint32_t p = atomicAdd(as_global(J.out.len), 1u);
+            if (p < J.out.cap) as_global(J.out.list)[p] = y[u];
         }
     }
 }
@@ -605,7 +612,7 @@ __global__ void __launch_bounds__(256, 8) k_local_queue_multi(DevGraph g, const 
         g, lds, s_off[njobs],
         [&](uint32_t i, uint32_t& j, uint32_t& x) {
             j = job_of(s_off, njobs, i);
-            x = jobs[j].frontier[i - s_off[j]];
+            x = as_global(jobs[j].frontier)[i - s_off[j]];
         },
         [&](uint32_t j) { return Rel4{jobs[j].phase, jobs[j].view, jobs[j].dir, jobs[j].slot}; },
         [&](uint32_t j, const uint32_t*& c, uint32_t*& bm) { c = jobs[j].cand_u; bm = jobs[j].out.bitmap; },
@@ -621,20 +628,20 @@ __global__ void __launch_bounds__(256, 7) k_local_check_multi(DevGraph g, const 
         g, lds, s_off[njobs],
         [&](uint32_t i, uint32_t& j, uint32_t& y, uint32_t& nf) {
             j = job_of(s_off, njobs, i);
-            y = jobs[j].queue[i - s_off[j]];
+            y = as_global(jobs[j].queue)[i - s_off[j]];
             nf = jobs[j].fl.n;
         },
         [&](uint32_t j, uint32_t k) { return jobs[j].fl.f[k]; }, [&](uint32_t j) { return jobs[j].phase; },
         [&](bool active, bool pass, uint32_t y, uint32_t j) {
             const bool kept = active && pass;
             append_jobs<1>(&kept, &y, &j, jobs, false);
-            if (active && !pass) atomicAnd(&jobs[j].out.bitmap[y >> 5], ~(1u << (y & 31)));
+            if (active && !pass) atomicAnd(as_global(jobs[j].out.bitmap) + (y >> 5), ~(1u << (y & 31)));
         });
     add_bytes(nbytes, bytes);
 }
 
 __global__ void __launch_bounds__(256) k_clear_sets_multi(const VSet* sets, uint32_t max_len) {
-    const VSet v = sets[blockIdx.y];
+    const VSet v = global_set(sets[blockIdx.y]);
     const uint32_t n = min(*v.len, max_len);
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) v.bitmap[v.list[i] >> 5] = 0u;
 }
