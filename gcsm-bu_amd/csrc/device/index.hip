@@ -81,10 +81,15 @@ __global__ void __launch_bounds__(256) k_nlf_touched(DevGraph g, const NlfEntry*
         const uint32_t first = label_off[en.vrank], T = label_off[en.vrank + 1] - first;
         for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < T; i += gridDim.x * blockDim.x) {
             const uint32_t v = by_label[first + i];
-            const bool pass = nlf_pass(g, en, groups, v, mode);
+            uint32_t* word = as_global(en.bitmap) + (v >> 5);
             const uint32_t bit = 1u << (v & 31);
-            if (pass) atomicOr(&en.bitmap[v >> 5], bit);
-            else if (mode == 1) atomicAnd(&en.bitmap[v >> 5], ~bit);
+            // only this thread writes the vertex's bit, and few vertices change: an atomic for those alone
+            const bool was = *word & bit;
+            if (mode == 0 && was) continue;  // insertions only add
+            const bool pass = nlf_pass(g, en, groups, v, mode);
+            if (pass == was) continue;
+            if (pass) atomicOr(word, bit);
+            else if (mode == 1) atomicAnd(word, ~bit);
         }
     }
 }
