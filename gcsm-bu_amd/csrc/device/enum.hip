@@ -2,12 +2,14 @@
 //
 //   init_from_pairs / init_from_set   initial partial results of the first matching-order edge
 //                                      (write_initial_partial_results, enumeration.cu:24-79)
-//   extend                             one wave per partial result, depth-first down to end_depth
-//                                      with a per-wave LDS stack of 64-candidate chunks; counts and
+//   extend                             depth-first search down to end_depth, a wave with an LDS stack
+//                                      of batches of up to 64 partial results; counts and
 //                                      hashes complete embeddings or writes partial results of
 //                                      end_depth (a BFS level when end_depth = d0 + 1).  Replaces
 //                                      extendBFSDFSRegTwo (enumeration.cu:407-781) and gamma_enumerate
 //                                      (gamma_enumeration.cu:359-880).
+//   direct_search                      the same search from the anchor pairs of many small steps in one
+//                                      launch, without a local index
 //   level_prepare / level_flat         one breadth-first level flattened over its candidates: per
 //   (and the _chain variants)          record, the runs of every backward entry and the shortest as
 //                                      the generator, then four candidates per lane tested in
@@ -16,10 +18,10 @@
 //   cp_prepare / cp_enumerate          Cartesian-product flattening of trailing tree leaves
 //                                      (GetNumTree + enumerateCartesianProductTree,
 //                                      cartesian_product.cu:193-284).
-// In the depth-first kernel, candidates of depth d come from the pivot backward neighbour's view
-// run; each lane tests one candidate: candidate bitmap, injectivity against the matched prefix, and
-// membership in every other backward neighbour's view run by binary search (search.cuh:7-25
-// semantics).
+// In the depth-first kernels, candidates of a depth come from the shortest of the first backward
+// neighbours' view runs; each is tested for its bit in the candidate bitmap, injectivity against the
+// matched prefix, and membership in every other backward neighbour's view run by binary search
+// (search.cuh:7-25 semantics).
 #include "kernels.h"
 #include "view.h"
 
@@ -1374,10 +1376,9 @@ __global__ void __launch_bounds__(kLenThreads) k_level_scan_chain_multi(const Ch
     level_scan_tiles(J.ls.off, n, J.ls.tile_sum);
 }
 
-// At least six waves per SIMD.  The writing form otherwise takes 86 VGPRs and five waves; bounded it
-// takes 80 and spills one 8-byte value per lane, stored once before its candidate loop and reloaded
-// only when staged records are flushed to the ring.  The kernel is latency-bound and shares the GPU
-// with the other teams' launches, so the extra resident wave measured faster.
+// At least six waves per SIMD (74 and 80 VGPRs, no spills).  The kernel is latency-bound and shares the
+// GPU with the other teams' launches: six waves measured faster than the five that the writing form
+// takes unbounded.
 template <int kMode>
 __global__ void __launch_bounds__(256, 6) k_level_flat_chain_multi(DevGraph g, const ChainJob* jobs, uint32_t k) {
     const ChainJob& J = jobs[blockIdx.y];
