@@ -196,15 +196,20 @@ __device__ __forceinline__ void contains_many(const uint32_t* a, const uint32_t*
 }
 
 // Matched vertices, prefix hashes, backward runs and generating lengths of the rows of frame j; the
-// frame's candidates are the rows' generating runs one after another.  Returns their number.  The
-// rows of frame 0 are records `stride` words apart; with kRanged, row r takes the elements
-// [chunk[r], chunks[r]) of its run instead of a whole chunk of it.
+// frame's candidates are the rows' generating runs one after another.  Returns their number, and in
+// `rows` how many of the rows it took: the first ones that have at most kFrameMax candidates together, or
+// one row alone (a list is shorter than 2^31), since 64 rows may share a list and their sum has 32 bits.
+// The rows of frame 0 are records `stride` words apart; with kRanged, row r takes the elements
+// [chunk[r], chunks[r]) of its run instead of a whole chunk of it, and all rows are taken: a number past
+// kFrameMax then only says that there are too many.
+constexpr uint32_t kFrameMax = kRangeMask;  // a frame of several rows fits a donated range
 template <bool kRanged>
-__device__ __forceinline__ uint32_t dfs_rows(const DevGraph& g, const StepDesc& d, uint32_t d0, uint32_t j, uint32_t rows, const uint32_t* in,
+__device__ __forceinline__ uint32_t dfs_rows(const DevGraph& g, const StepDesc& d, uint32_t d0, uint32_t j, uint32_t& rows, const uint32_t* in,
                                              uint32_t stride, DfsHdr& H, uint32_t* f, const DfsBuf* buf, uint32_t lane, unsigned long long& bytes,
                                              bool count_bytes) {
     const uint32_t depth = d0 + j, e0 = d.boff[depth], ne = d.boff[depth + 1] - e0;
     uint32_t len = 0, skip = 0;
+    unsigned long long row_bytes = 0;
     if (lane < rows) {
         unsigned long long h = 0;
         uint32_t r = lane;
@@ -238,7 +243,7 @@ __device__ __forceinline__ uint32_t dfs_rows(const DevGraph& g, const StepDesc& 
                 best = l;
                 gen = e;
             }
-            if (count_bytes && (j || H.chunk[lane] == 0)) bytes += 4ull * ((rv[e].hi - rv[e].lo) + (rv[e].dhi - rv[e].dlo));
+            if (count_bytes && (j || H.chunk[lane] == 0)) row_bytes += 4ull * ((rv[e].hi - rv[e].lo) + (rv[e].dhi - rv[e].dlo));
         }
         H.gen[lane] = gen;
         len = best;
@@ -253,12 +258,20 @@ __device__ __forceinline__ uint32_t dfs_rows(const DevGraph& g, const StepDesc& 
             len = min(best - skip, width);
         }
     }
+    const uint32_t part = min(len, kFrameMax + 1);  // 64 of them stay under 2^31
     uint32_t total;
-    const uint32_t pre = wave_prefix(len, total);
+    uint32_t pre = wave_prefix(part, total);
+    total = uniform(total);
+    if (!kRanged && total > kFrameMax) {
+        rows = max(1u, static_cast<uint32_t>(__popcll(__ballot(lane < rows && pre + part <= kFrameMax))));
+        total = uniform(__shfl(rows == 1 ? len : pre + part, static_cast<int>(rows) - 1, 64));
+        if (lane >= rows) pre = total;
+    }
+    if (lane < rows) bytes += row_bytes;
     H.pre[lane] = pre;
     H.skip[lane] = skip;
     wave_sync();
-    return uniform(total);
+    return total;
 }
 
 // One round of a frame's candidates, flattened elements cur + 64 u + lane below tot: their row k, vertex
@@ -345,23 +358,17 @@ __device__ __forceinline__ void dfs_round(const DevGraph& g, const StepDesc& d, 
 // Back from frame j + 1 to frame j: the rows just searched leave frame j's buffer.
 __device__ __forceinline__ void dfs_pop(DfsHdr& H, DfsBuf* buf, uint32_t j, uint32_t lane) {
     const uint32_t done = uniform(H.rows[j + 1]);
-    const uint32_t left = uniform(H.waiting[j]) - done;  // fewer than 64 * kDfsIlp
-    uint32_t mv[kDfsIlp];
-    uint8_t mp[kDfsIlp];
-#pragma unroll
-    for (uint32_t u = 0; u < kDfsIlp; u++) {
-        const uint32_t x = lane + 64 * u;
-        mv[u] = x < left ? buf[j].cand[done + x] : 0u;
-        mp[u] = x < left ? buf[j].parent[done + x] : 0u;
-    }
-    wave_sync();
-#pragma unroll
-    for (uint32_t u = 0; u < kDfsIlp; u++) {
-        const uint32_t x = lane + 64 * u;
+    const uint32_t left = uniform(H.waiting[j]) - done;
+    for (uint32_t x0 = 0; x0 < left; x0 += 64) {  // 64 at a time: what is written is not read any more
+        const uint32_t x = x0 + lane;
+        const uint32_t c = x < left ? buf[j].cand[done + x] : 0u;
+        const uint8_t p = x < left ? buf[j].parent[done + x] : uint8_t(0);
+        wave_sync();
         if (x < left) {
-            buf[j].cand[x] = mv[u];
-            buf[j].parent[x] = mp[u];
+            buf[j].cand[x] = c;
+            buf[j].parent[x] = p;
         }
+        wave_sync();
     }
     if (lane == 0) H.waiting[j] = left;
     wave_sync();
@@ -396,7 +403,7 @@ __global__ void __launch_bounds__(kWaves * 64) k_extend(DevGraph g, StepDesc d, 
     unsigned long long my_cnt = 0, my_hash = 0, my_bytes = 0;
 
     const bool donating = schedule == 2;
-    uint32_t version = 0;
+    uint32_t version = 0, sub = 0;  // sub: items of the group that earlier frames took
     unsigned long long group;
     if (schedule == 0) group = gw;
     else {
@@ -417,8 +424,9 @@ __global__ void __launch_bounds__(kWaves * 64) k_extend(DevGraph g, StepDesc d, 
         }
         if (kMode == kWriteAtEnd && uniform(__hip_atomic_load(r.overflow, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) break;
         // frame 0: the group's items, one per lane
-        const unsigned long long item = static_cast<unsigned long long>(grp) * G + lane;
-        const uint32_t rows0 = static_cast<uint32_t>(min(static_cast<unsigned long long>(G), nitems - static_cast<unsigned long long>(grp) * G));
+        const unsigned long long item = static_cast<unsigned long long>(grp) * G + sub + lane;
+        const uint32_t items = static_cast<uint32_t>(min(static_cast<unsigned long long>(G), nitems - static_cast<unsigned long long>(grp) * G));
+        uint32_t rows0 = items - sub;
         if (lane < rows0) {
             uint32_t rec = static_cast<uint32_t>(item), chunk = 0, chunks = 1;
             if (split) {  // last record with split[rec] <= item
@@ -440,9 +448,9 @@ __global__ void __launch_bounds__(kWaves * 64) k_extend(DevGraph g, StepDesc d, 
         uint32_t j = 0, built = 0;
         const uint32_t total0 = dfs_rows<false>(g, d, d0, 0, rows0, r.in, d0, H, f, buf, lane, my_bytes, !stolen && out.bytes);
         // donating: publish the group's frame 0 candidates and take the first round from the word
-        // (a range past 2^24 candidates stays the wave's own)
+        // (a range past 2^24 candidates, or of a part of the group, stays the wave's own)
         uint32_t cur0 = stolen ? s_lo : 0u, end0 = stolen ? s_hi : total0;
-        const bool published = donating && end0 <= kRangeMask;
+        const bool published = donating && rows0 == items && end0 <= kRangeMask;
         if (published) {
             version = (version + 1) & 0xFFFFu;
             uint32_t t = 0, t_end = 0;
@@ -481,7 +489,7 @@ __global__ void __launch_bounds__(kWaves * 64) k_extend(DevGraph g, StepDesc d, 
             }
             const uint32_t waiting = j < last ? uniform(H.waiting[j]) : 0u;
             if (waiting >= 64 || (cur >= tot && waiting)) {  // descend with a batch
-                const uint32_t rows = min(64u, waiting);
+                uint32_t rows = min(64u, waiting);
                 j += 1;
                 const uint32_t t = dfs_rows<false>(g, d, d0, j, rows, r.in, d0, H, f, buf, lane, my_bytes, out.bytes != nullptr);
                 built = j;
@@ -501,7 +509,8 @@ __global__ void __launch_bounds__(kWaves * 64) k_extend(DevGraph g, StepDesc d, 
                 continue;
             }
             if (built != j) {
-                dfs_rows<false>(g, d, d0, j, uniform(H.rows[j]), r.in, d0, H, f, buf, lane, my_bytes, false);
+                uint32_t rows = uniform(H.rows[j]);
+                dfs_rows<false>(g, d, d0, j, rows, r.in, d0, H, f, buf, lane, my_bytes, false);
                 built = j;
             }
             // one round of frame j's candidates
@@ -560,6 +569,9 @@ __global__ void __launch_bounds__(kWaves * 64) k_extend(DevGraph g, StepDesc d, 
             wave_sync();
         }
         if (stolen) continue;  // the launch's items are used up: steal again
+        sub += rows0;
+        if (sub < items) continue;  // the rest of the group
+        sub = 0;
         if (schedule == 0) group += total_waves;
         else {
             unsigned long long t2 = 0;
@@ -701,6 +713,7 @@ __global__ void __launch_bounds__(kWaves * 64) k_direct_search(DevGraph g, const
             const uint32_t last = d.n - 1 - depth0;
             uint32_t j = 0, built = 0, rounds = 0, state = 0;  // state 1: hand the rest on, 2: given up
             const uint32_t total0 = dfs_rows<true>(g, d, depth0, 0, rows0, in, stride, H, f, buf, lane, no_bytes, false);
+            if (total0 > kFrameMax) state = 2;  // far more than a step may have
             unsigned long long work = total0;
             if (lane == 0) {
                 H.rows[0] = rows0;
@@ -709,7 +722,7 @@ __global__ void __launch_bounds__(kWaves * 64) k_direct_search(DevGraph g, const
                 H.tot[0] = total0;
             }
             wave_sync();
-            for (;;) {
+            while (!state) {
                 const uint32_t cur = uniform(H.cur[j]), tot = uniform(H.tot[j]);
                 const uint32_t waiting = j < last ? uniform(H.waiting[j]) : 0u;
                 const bool down = waiting >= 64 || (cur >= tot && waiting);
@@ -731,9 +744,10 @@ __global__ void __launch_bounds__(kWaves * 64) k_direct_search(DevGraph g, const
                     if (state) break;
                 }
                 if (down) {  // descend with a batch
-                    const uint32_t rows = min(64u, waiting);
+                    uint32_t rows = min(64u, waiting);
                     j += 1;
                     const uint32_t tj = dfs_rows<true>(g, d, depth0, j, rows, in, stride, H, f, buf, lane, no_bytes, false);
+                    if (tj > kFrameMax) state = 2;
                     work += tj;
                     built = j;
                     if (lane == 0) {
@@ -746,7 +760,8 @@ __global__ void __launch_bounds__(kWaves * 64) k_direct_search(DevGraph g, const
                     continue;
                 }
                 if (built != j) {
-                    dfs_rows<true>(g, d, depth0, j, uniform(H.rows[j]), in, stride, H, f, buf, lane, no_bytes, false);
+                    uint32_t rows = uniform(H.rows[j]);
+                    dfs_rows<true>(g, d, depth0, j, rows, in, stride, H, f, buf, lane, no_bytes, false);
                     built = j;
                 }
                 const uint32_t depth = depth0 + j;
@@ -782,7 +797,8 @@ __global__ void __launch_bounds__(kWaves * 64) k_direct_search(DevGraph g, const
                 uint32_t searched = 0;  // rows of the frame's buffer that are the next frame's
                 bool fits = true;
                 for (uint32_t jj = j + 1; jj-- > 0;) {
-                    const uint32_t rows = uniform(H.rows[jj]), cur = uniform(H.cur[jj]), tot = uniform(H.tot[jj]), depth = depth0 + jj;
+                    uint32_t rows = uniform(H.rows[jj]);
+                    const uint32_t cur = uniform(H.cur[jj]), tot = uniform(H.tot[jj]), depth = depth0 + jj;
                     if (built != jj) {
                         dfs_rows<true>(g, d, depth0, jj, rows, in, stride, H, f, buf, lane, no_bytes, false);
                         built = jj;
