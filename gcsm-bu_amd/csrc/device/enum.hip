@@ -23,6 +23,7 @@
 // matched prefix, and membership in every other backward neighbour's view run by binary search
 // (search.cuh:7-25 semantics).
 #include "kernels.h"
+#include "range_word.h"
 #include "view.h"
 
 namespace csm {
@@ -91,23 +92,18 @@ __device__ __forceinline__ uint32_t find_record(const unsigned long long* off, u
 }
 
 // ---- Range donation (work stealing) of the depth-first kernel --------------------------------
-// Each wave owns one word per launch: the candidate range [cur, end) of its current record's first
-// frame still to be explored, packed as version (16 bits) | cur (24) | end (24), with the item
-// group's index in a second array.  The owner takes its next 64-candidate round by moving cur up; a wave
-// out of work takes the upper half of another wave's range by moving that wave's end down to the
-// midpoint.  Both are compare-and-swaps on the one word, so the rounds taken and the halves
-// donated never overlap.  The owner publishes only when its range is used up, and then another
-// version, so a thief's swap fails if the group index it read belongs to another range.  Ranges only
-// shrink, so every wave's search ends.  All of it is relaxed: the two words are the only data the
-// waves exchange, and the agent-scope acquire and release that ordered them before (an L1
-// invalidation per probe, an L2 write-back per publication) took more than half of the kernel's time.
+// Each wave owns a pair of words per launch (range_word.h): the candidate range [cur, end) of its current
+// frame 0 still to be explored, and which items that frame holds.  The owner takes its next 64-candidate
+// round by moving cur up; a wave out of work takes the upper half of another wave's range by moving
+// that wave's end down to the midpoint.  Both are compare-and-swaps on the range word, so the rounds taken
+// and the halves donated never overlap.  The owner publishes only when its range is used up, and then
+// another version, so a thief's swap fails if the range was published anew since it was read.  Ranges only
+// shrink, so every wave's search ends.  All of it is relaxed, the agent-scope acquire and release of an
+// ordered protocol (an L1 invalidation per probe, an L2 write-back per publication) took more than half
+// of the kernel's time: the two words are the only data the waves exchange, and a thief uses a frame
+// word only if it carries the range's version, whatever order the two stores become visible in.
 // (The reference's disabled design: gamma_enumeration.cu:209-357.)
-constexpr uint32_t kRangeBits = 24;
-constexpr uint32_t kRangeMask = (1u << kRangeBits) - 1;
 constexpr uint32_t kStealRounds = 8;  // victim probes of 64 waves each before a wave gives up
-
-__device__ __forceinline__ uint32_t range_cur(unsigned long long w) { return static_cast<uint32_t>(w >> kRangeBits) & kRangeMask; }
-__device__ __forceinline__ uint32_t range_end(unsigned long long w) { return static_cast<uint32_t>(w) & kRangeMask; }
 
 // Owner (one lane): the next round [t, t_end) of its published range, false when it is used up.
 __device__ __forceinline__ bool claim_round(unsigned long long* slot, uint32_t& t, uint32_t& t_end) {
@@ -129,26 +125,28 @@ __device__ __forceinline__ bool claim_round(unsigned long long* slot, uint32_t& 
 }
 
 // Thief (whole wave): the upper half of some wave's range with at least two rounds left.
-__device__ __forceinline__ bool steal_range(unsigned long long* donate, const uint32_t* donate_rec, uint32_t total_waves, uint32_t gw,
-                                            uint32_t lane, uint32_t& rec, uint32_t& lo, uint32_t& hi) {
+__device__ __forceinline__ bool steal_range(unsigned long long* donate, uint32_t total_waves, uint32_t gw, uint32_t lane, uint32_t& grp,
+                                            uint32_t& first, uint32_t& lo, uint32_t& hi) {
     for (uint32_t a = 0; a < kStealRounds; a++) {
         const uint32_t v = (gw + 1 + a * 64 + lane * (1 + a)) % total_waves;
-        const unsigned long long w = v != gw ? __hip_atomic_load(donate + v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0ull;
+        const unsigned long long w = v != gw ? __hip_atomic_load(donate + 2ull * v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0ull;
         const uint32_t cur = range_cur(w), end = range_end(w);
         const uint32_t rem = end > cur ? end - cur : 0u;
         uint32_t key = rem << 6 | lane;  // rem < 2^24: fits
         for (int o = 32; o > 0; o >>= 1) key = max(key, static_cast<uint32_t>(__shfl_xor(key, o, 64)));
         if ((key >> 6) < 128u) continue;
         const uint32_t src = key & 63u;
-        uint32_t got = 0, r = 0, mid = 0;
+        uint32_t got = 0, mid = 0;
+        unsigned long long r = 0;
         if (lane == src) {
             mid = cur + (((rem >> 1) + 63u) & ~63u);  // cur + 64 <= mid < end
-            r = __hip_atomic_load(donate_rec + v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            r = __hip_atomic_load(donate + 2ull * v + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             const unsigned long long nw = (w & ~static_cast<unsigned long long>(kRangeMask)) | mid;
-            got = atomicCAS(donate + v, w, nw) == w ? 1u : 0u;
+            got = same_publication(w, r) && atomicCAS(donate + 2ull * v, w, nw) == w ? 1u : 0u;
         }
         if (__shfl(got, src, 64)) {
-            rec = __shfl(r, src, 64);
+            grp = __shfl(frame_group(r), src, 64);
+            first = __shfl(frame_first(r), src, 64);
             lo = __shfl(mid, src, 64);
             hi = __shfl(end, src, 64);
             return true;
@@ -386,7 +384,7 @@ constexpr int kDfsGridWaves = 2048;
 template <int kMode>
 __global__ void __launch_bounds__(kWaves * 64) k_extend(DevGraph g, StepDesc d, uint32_t d0, uint32_t end_depth, Ring r, MatchOut out,
                                                          const unsigned long long* split, unsigned long long* work, int schedule,
-                                                         unsigned long long* donate, uint32_t* donate_rec) {
+                                                         unsigned long long* donate) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     unsigned char* const wave_base = lds_raw + (threadIdx.x >> 6) * wave_lds_bytes(d0, end_depth);
     DfsHdr& H = *reinterpret_cast<DfsHdr*>(wave_base);
@@ -413,20 +411,20 @@ __global__ void __launch_bounds__(kWaves * 64) k_extend(DevGraph g, StepDesc d, 
     }
     for (;;) {
         // the next group of the launch, else (donating) a range taken from another wave
-        uint32_t grp, s_lo = 0, s_hi = 0;
+        uint32_t grp, first = sub, s_lo = 0, s_hi = 0;
         bool stolen = false;
         if (group < ngroups) {
             grp = static_cast<uint32_t>(group);
-        } else if (donating && steal_range(donate, donate_rec, total_waves, gw, lane, grp, s_lo, s_hi)) {
+        } else if (donating && steal_range(donate, total_waves, gw, lane, grp, first, s_lo, s_hi)) {
             stolen = true;
         } else {
             break;
         }
         if (kMode == kWriteAtEnd && uniform(__hip_atomic_load(r.overflow, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) break;
-        // frame 0: the group's items, one per lane
-        const unsigned long long item = static_cast<unsigned long long>(grp) * G + sub + lane;
+        // frame 0: the group's items from `first` on, one per lane
+        const unsigned long long item = static_cast<unsigned long long>(grp) * G + first + lane;
         const uint32_t items = static_cast<uint32_t>(min(static_cast<unsigned long long>(G), nitems - static_cast<unsigned long long>(grp) * G));
-        uint32_t rows0 = items - sub;
+        uint32_t rows0 = items - first;
         if (lane < rows0) {
             uint32_t rec = static_cast<uint32_t>(item), chunk = 0, chunks = 1;
             if (split) {  // last record with split[rec] <= item
@@ -447,22 +445,17 @@ __global__ void __launch_bounds__(kWaves * 64) k_extend(DevGraph g, StepDesc d, 
         wave_sync();
         uint32_t j = 0, built = 0;
         const uint32_t total0 = dfs_rows<false>(g, d, d0, 0, rows0, r.in, d0, H, f, buf, lane, my_bytes, !stolen && out.bytes);
-        // donating: publish the group's frame 0 candidates and take the first round from the word
-        // (a range past 2^24 candidates, or of a part of the group, stays the wave's own)
+        // donating: publish frame 0's candidates and take the first round from the word (a single row
+        // of more than kRangeMask candidates stays the wave's own)
         uint32_t cur0 = stolen ? s_lo : 0u, end0 = stolen ? s_hi : total0;
-        const bool published = donating && rows0 == items && end0 <= kRangeMask;
+        const bool published = donating && end0 <= kRangeMask;
         if (published) {
-            version = (version + 1) & 0xFFFFu;
+            version = next_version(version);
             uint32_t t = 0, t_end = 0;
             if (lane == 0) {
-                __hip_atomic_store(donate_rec + gw, grp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __builtin_amdgcn_s_waitcnt(0);  // the group's store is done before the range's is issued
-                asm volatile("" ::: "memory");
-                __hip_atomic_store(donate + gw,
-                                   static_cast<unsigned long long>(version) << (2 * kRangeBits) |
-                                       static_cast<unsigned long long>(cur0) << kRangeBits | end0,
-                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if (!claim_round(donate + gw, t, t_end)) t = t_end = 0;
+                __hip_atomic_store(donate + 2ull * gw + 1, frame_word(version, grp, first), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_store(donate + 2ull * gw, range_word(version, cur0, end0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (!claim_round(donate + 2ull * gw, t, t_end)) t = t_end = 0;
             }
             cur0 = __shfl(t, 0, 64);
             end0 = __shfl(t_end, 0, 64);
@@ -478,7 +471,7 @@ __global__ void __launch_bounds__(kWaves * 64) k_extend(DevGraph g, StepDesc d, 
             uint32_t cur = uniform(H.cur[j]), tot = uniform(H.tot[j]);
             if (j == 0 && cur >= tot && published) {  // frame 0's next round from the published range
                 uint32_t t = 0, t_end = 0;
-                if (lane == 0 && !claim_round(donate + gw, t, t_end)) t = t_end = 0;
+                if (lane == 0 && !claim_round(donate + 2ull * gw, t, t_end)) t = t_end = 0;
                 cur = uniform(__shfl(t, 0, 64));
                 tot = uniform(__shfl(t_end, 0, 64));
                 if (lane == 0) {
@@ -1758,11 +1751,11 @@ void extend(const DevGraph& g, const StepDesc& d, uint32_t d0, uint32_t end_dept
     blocks = std::min<int>(std::min<int>(blocks, static_cast<int>(kMaxDfsBlocks)) * 4, kDfsGridWaves) / static_cast<int>(kWaves);
     const int grid = split || schedule == 2 ? blocks : grid_for(r.in_max, kWaves, blocks);
     const size_t lds = static_cast<size_t>(kWaves) * wave_lds_bytes(d0, end_depth);
-    if (schedule == 2) fill_u32(reinterpret_cast<uint32_t*>(dn.range), 0u, 2ull * grid * kWaves, s);  // every word: nothing to take
+    if (schedule == 2) fill_u32(reinterpret_cast<uint32_t*>(dn.words), 0u, 4ull * grid * kWaves, s);  // every pair: nothing to take
     if (mode == kCountAtEnd)
-        k_extend<kCountAtEnd><<<grid, kWaves * 64, lds, s>>>(g, d, d0, end_depth, r, out, split, work_counter, schedule, dn.range, dn.rec);
+        k_extend<kCountAtEnd><<<grid, kWaves * 64, lds, s>>>(g, d, d0, end_depth, r, out, split, work_counter, schedule, dn.words);
     else
-        k_extend<kWriteAtEnd><<<grid, kWaves * 64, lds, s>>>(g, d, d0, end_depth, r, out, split, work_counter, schedule, dn.range, dn.rec);
+        k_extend<kWriteAtEnd><<<grid, kWaves * 64, lds, s>>>(g, d, d0, end_depth, r, out, split, work_counter, schedule, dn.words);
 }
 
 uint32_t direct_wave_lds(uint32_t max_qn) { return wave_lds_bytes(2, std::max<uint32_t>(max_qn, 3)); }

@@ -227,12 +227,11 @@ void count_records(const StepDesc& d, const uint32_t* rec, const uint32_t* n_rec
 void bitmap_to_list(const uint32_t* bitmap, uint32_t dv, uint32_t* list, uint32_t* len, hipStream_t s);
 
 enum ExtendMode : int { kCountAtEnd = 0, kWriteAtEnd = 1 };
-// Range donation of the depth-first kernel (schedule 2): one range word and one record index per
-// wave of the launch (kMaxDfsBlocks * 4 waves at most); extend clears the words before the launch.
+// Range donation of the depth-first kernel (schedule 2): a range word and a frame word per wave of the
+// launch (kMaxDfsBlocks * 4 waves at most); extend clears them before the launch.
 constexpr uint32_t kMaxDfsBlocks = 16384;
 struct Donation {
-    unsigned long long* range;  // [kMaxDfsBlocks * 4]
-    uint32_t* rec;              // [kMaxDfsBlocks * 4]
+    unsigned long long* words;  // [kMaxDfsBlocks * 4][2]
 };
 // DFS from the records at depth d0 down to end_depth: counts/hashes complete embeddings when
 // end_depth == n, or writes the partial results of depth end_depth to the ring.
