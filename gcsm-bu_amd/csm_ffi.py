@@ -18,7 +18,7 @@ EXPORTED = [
     "csm_get_relation_edge_counts",
     "csm_get_counts", "csm_pool_usage", "csm_read_candidates", "csm_read_adjacency",
     "csm_synchronize", "csm_snapshot", "csm_restore", "csm_get_tunables", "csm_set_tunables", "csm_tune",
-    "csm_profile_enable", "csm_profile_read", "csm_calibration_copy",
+    "csm_profile_enable", "csm_profile_read", "csm_get_direct_counts", "csm_calibration_copy",
 ]
 
 STATUS = {0: "OK", 1: "ARGUMENT", 2: "IO", 3: "FORMAT", 4: "LIMIT", 5: "DEVICE", 6: "MEMORY", 7: "STATE",
@@ -55,6 +55,10 @@ class Tunables(ctypes.Structure):
 
     def as_dict(self):
         return {name: getattr(self, name) for name in TUNABLES}
+
+
+class DirectCounts(ctypes.Structure):
+    _fields_ = [(name, ctypes.c_uint64) for name in ("tried", "finished", "handed_on", "given_up", "left_over", "beside")]
 
 
 class CsmError(RuntimeError):
@@ -108,6 +112,7 @@ def load():
         lib.csm_tune.argtypes = [vp, u64, u64, u32, u32, P(Tunables), u32, P(Tunables), P(ctypes.c_double), u32, P(u32), P(u32)]
         lib.csm_profile_enable.argtypes = [vp, u32]
         lib.csm_profile_read.argtypes = [vp, u32, P(u64), P(ctypes.c_double), P(u64)]
+        lib.csm_get_direct_counts.argtypes = [vp, P(DirectCounts)]
         lib.csm_calibration_copy.argtypes = [vp, u64, P(ctypes.c_double)]
         for name in EXPORTED:
             f = getattr(lib, name)
@@ -328,6 +333,12 @@ class Session:
         n, ms, b = ctypes.c_uint64(), ctypes.c_double(), ctypes.c_uint64()
         self._check(self.lib.csm_profile_read(self.h, family, ctypes.byref(n), ctypes.byref(ms), ctypes.byref(b)))
         return n.value, ms.value, b.value
+
+    def direct_counts(self):
+        """What became of the steps that were searched directly (csm_get_direct_counts), as a dict."""
+        c = DirectCounts()
+        self._check(self.lib.csm_get_direct_counts(self.h, ctypes.byref(c)))
+        return {name: getattr(c, name) for name, _ in DirectCounts._fields_}
 
     def calibration_copy(self, words):
         ms = ctypes.c_double()

@@ -340,6 +340,13 @@ csm_status csm_profile_read(csm_session* s, uint32_t family, uint64_t* launches,
     return CSM_OK;
 }
 
+csm_status csm_get_direct_counts(csm_session* s, csm_direct_counts* out) {
+    if (!s || !out) return CSM_ERR_ARGUMENT;
+    const Engine::DirectCounts& c = s->engine.direct_counts();
+    *out = csm_direct_counts{c.tried, c.finished, c.handed_on, c.given_up, c.left_over, c.beside};
+    return CSM_OK;
+}
+
 csm_status csm_calibration_copy(csm_session* s, uint64_t words, double* ms) {
     if (!s) return CSM_ERR_ARGUMENT;
     double m = 0;

@@ -1013,6 +1013,7 @@ std::string Engine::direct_phase(uint32_t ph, uint32_t n, uint32_t others, std::
         direct_anchors(g_, jobs, nj, ctr, pairs, cap, bs_[0].by_label, bs_[0].label_off, bs_[1].by_label, bs_[1].label_off, batch_arcs_, s_);
         const uint32_t behind = others + (n - k - nj);  // steps not in this launch
         const uint32_t small = n + others <= lanes_.size() ? kDirectTailFew : kDirectTail;
+        std::vector<char> handed(nj, 0);
         for (uint32_t p = 0, before = 2 * small, committed = 0;;) {
             pass(p);
             if (p % 2 == 0) {  // one wait for two passes after the first
@@ -1021,15 +1022,23 @@ std::string Engine::direct_phase(uint32_t ph, uint32_t n, uint32_t others, std::
                 committed = p + 1;
                 uint32_t left = 0, tasks_left = 0;
                 for (uint32_t x = 0; x < kDirectShards; x++) tasks_left += h_direct_state_[nj + x];
-                for (uint32_t x = 0; x < nj; x++) left += h_direct_state_[x] != 0;
+                for (uint32_t x = 0; x < nj; x++) {
+                    left += h_direct_state_[x] != 0;
+                    if (h_direct_state_[x] == 2) handed[x] = 1;
+                }
                 // go on while the tasks get fewer, or as long as the steps left are more than one group
                 if (!tasks_left || p + 2 >= kDirectPasses || (2 * tasks_left > before && behind + left <= lanes_.size())) break;
                 before = std::max(tasks_left, small);
             }
             p++;
         }
-        for (uint32_t x = 0; x < nj; x++)
-            if (!h_direct_state_[x]) done[direct_steps_[k + x].q * kMaxQE + direct_steps_[k + x].i] = 1;
+        for (uint32_t x = 0; x < nj; x++) {
+            const uint32_t state = h_direct_state_[x];
+            if (!state) done[direct_steps_[k + x].q * kMaxQE + direct_steps_[k + x].i] = 1;
+            direct_counts_.handed_on += handed[x];
+            (state == 0 ? direct_counts_.finished : state == 1 ? direct_counts_.given_up : direct_counts_.left_over)++;
+        }
+        direct_counts_.tried += nj;
     }
     return "";
 }
@@ -1802,6 +1811,7 @@ std::string Engine::run_phase(uint32_t ph, uint64_t edges) {
     CSM_HIP(hipEventRecord(phase_start_, s_));
     // the direct steps first if there are no others, else beside them
     const bool beside = tries && tries < nsteps && team_ > 1;
+    direct_counts_.beside += beside;
     for (uint32_t k = 0; k < tries && beside; k++) finished[direct_steps_[k].q * kMaxQE + direct_steps_[k].i] = 1;
     if (tries && !beside) {
         std::string err = direct_phase(ph, tries, nsteps - tries, finished);

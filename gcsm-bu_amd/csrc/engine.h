@@ -9,6 +9,7 @@
 #include <hip/hip_runtime.h>
 
 #include <chrono>
+#include <atomic>
 #include <condition_variable>
 #include <cstdint>
 #include <cstdio>
@@ -234,6 +235,11 @@ class Engine {
     };
     std::string profile_enable(uint32_t mask);
     std::string profile_read(uint32_t family, KernelStat& st);
+    // What became of the steps searched directly (csm.h csm_direct_counts); read while the request loop runs too.
+    struct DirectCounts {
+        std::atomic<uint64_t> tried{0}, finished{0}, handed_on{0}, given_up{0}, left_over{0}, beside{0};
+    };
+    const DirectCounts& direct_counts() const { return direct_counts_; }
     std::string calibration_copy(uint64_t words, double& ms);
 
   private:
@@ -353,6 +359,7 @@ class Engine {
     uint32_t direct_cap_ = 0;            // steps the tables hold
     uint32_t direct_qn_ = 0;             // most query vertices among them
     bool direct_stale_ = true;
+    DirectCounts direct_counts_;
     // Teams: lanes [t * team_, (t + 1) * team_) run up to team_ steps at a time on the first lane's
     // stream from one host thread, each stage for all of them before one wait, and their level
     // chains as one chain of multi-job launches (ChainJob tables at d_chain_jobs_ + first lane).

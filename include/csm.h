@@ -222,6 +222,20 @@ csm_status csm_tune(csm_session* s, uint64_t first, uint64_t batch_edges, uint32
  * written). */
 csm_status csm_profile_enable(csm_session* s, uint32_t mask);
 csm_status csm_profile_read(csm_session* s, uint32_t family, uint64_t* launches, double* ms, uint64_t* bytes);
+/* Direct steps (no counterpart in the reference): under search strategy 2 a step that is expected to test few
+ * candidates is searched depth-first from its update edges in an order of its own, without the
+ * technique's matching order and local index, many such steps in one launch; a step that turns out
+ * large is then run as the technique says.  Results are the same (the environment variable
+ * CSM_DIRECT_STEPS=0 switches them off).  What became of the steps tried since csm_build_index: */
+typedef struct {
+    uint64_t tried;       /* finished + given_up + left_over */
+    uint64_t finished;    /* counted by the direct search */
+    uint64_t handed_on;   /* did not finish in the first pass (they may finish in a later one) */
+    uint64_t given_up;    /* more update edges or candidates than a direct step may have, or a full queue */
+    uint64_t left_over;   /* unfinished when no further pass was worth it */
+    uint64_t beside;      /* phases whose direct steps ran while the lanes ran the others */
+} csm_direct_counts;
+csm_status csm_get_direct_counts(csm_session* s, csm_direct_counts* out);
 /* Times a plain device copy of `words` 32-bit words (calibration of HBM traffic counters). */
 csm_status csm_calibration_copy(csm_session* s, uint64_t words, double* ms);
 
