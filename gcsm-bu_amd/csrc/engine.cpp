@@ -922,40 +922,67 @@ static double direct_estimate(const Query& q, const std::vector<double>& fan, co
 
 std::string Engine::direct_tables() {
     direct_steps_.clear();
+    for (auto& jobs : direct_jobs_) jobs.clear();
     direct_qn_ = 2;
+    direct_seen_.resize(qs_.size() * kMaxQE);
     for (size_t qi = 0; qi < qs_.size(); qi++) {
         const QState& qs = *qs_[qi];
         // the other strategies are searched as the user asked; the stack depth bounds the LDS stack here too
         if (!qs.planned || !qs.matchable || qs.tech.strategy != SearchStrategy::kDynamicBfsDfs || qs.q.n > opt_.stack_depth + 3) continue;
         direct_qn_ = std::max(direct_qn_, qs.q.n);
         for (uint32_t i = 0; i < qs.q.m; i++) {
-            const double arcs = qs.card[qs.q.rel(qs.q.qe_list[i].first, qs.q.qe_list[i].second)];
-            const OrderPerEdge o = direct_order(qs.q, qs.avg, qs.q.qe_list[i].first, qs.q.qe_list[i].second);
-            direct_steps_.push_back({static_cast<uint32_t>(qi), i, arcs / std::max<size_t>(1, host_g_.src.size()), 0, 0});
+            const uint32_t u0 = qs.q.qe_list[i].first, u1 = qs.q.qe_list[i].second;
+            const RelInfo& R = qs.rel[qs.q.rel(u0, u1)];
+            const double arcs = qs.card[qs.q.rel(u0, u1)];
+            const OrderPerEdge o = direct_order(qs.q, qs.avg, u0, u1);
+            direct_steps_.push_back({static_cast<uint32_t>(qi), i, arcs / std::max<size_t>(1, host_g_.src.size()), 0, 0, 0,
+                                     static_cast<uint32_t>(direct_steps_.size())});
             DirectStep& st = direct_steps_.back();
             st.work = st.anchors * direct_estimate(qs.q, qs.fan, qs.src, o);
             st.key = std::max(st.anchors / kDirectPairs, st.work / kDirectTry);
+            for (uint32_t ph = 0; ph < 2; ph++)
+                direct_jobs_[ph].push_back(DirectJob{step_desc(qs, i, ph, o, nullptr, 0), R.dir, R.slot, qs.vrank[u0], st.q,
+                                                     qs.cand + static_cast<uint64_t>(u0) * words_,
+                                                     qs.cand + static_cast<uint64_t>(u1) * words_});
         }
     }
-    // small steps first: a phase tries a prefix
-    std::stable_sort(direct_steps_.begin(), direct_steps_.end(), [](const DirectStep& x, const DirectStep& y) { return x.key < y.key; });
-    std::vector<DirectJob> jobs[2];
-    for (const DirectStep& st : direct_steps_) {
-        const QState& qs = *qs_[st.q];
-        const uint32_t u0 = qs.q.qe_list[st.i].first, u1 = qs.q.qe_list[st.i].second;
-        const RelInfo& R = qs.rel[qs.q.rel(u0, u1)];
-        const OrderPerEdge o = direct_order(qs.q, qs.avg, u0, u1);
-        for (uint32_t ph = 0; ph < 2; ph++)
-            jobs[ph].push_back(DirectJob{step_desc(qs, st.i, ph, o, nullptr, 0), R.dir, R.slot, qs.vrank[u0], st.q,
-                                         qs.cand + static_cast<uint64_t>(u0) * words_, qs.cand + static_cast<uint64_t>(u1) * words_});
+    std::string err = direct_rank();
+    direct_stale_ = !err.empty();
+    return err;
+}
+
+// Small steps first: a phase tries a prefix.
+std::string Engine::direct_rank() {
+    direct_rank_at_ = ~0ull;
+    for (DirectStep& st : direct_steps_) {
+        const DirectSeen& seen = direct_seen_[st.q * kMaxQE + st.i];
+        st.rank = st.key;
+        if (seen.until <= direct_seq_) continue;
+        st.rank = std::max(st.key, (1.0 + 1e-9) / static_cast<double>(seen.limit));
+        direct_rank_at_ = std::min(direct_rank_at_, seen.until);
     }
-    for (uint32_t ph = 0; ph < 2; ph++)
-        if (!jobs[ph].empty())
-            CSM_HIP(hipMemcpyAsync(d_direct_ + static_cast<uint64_t>(ph) * direct_cap_, jobs[ph].data(), jobs[ph].size() * sizeof(DirectJob),
-                                   hipMemcpyHostToDevice, s_));
+    std::stable_sort(direct_steps_.begin(), direct_steps_.end(), [](const DirectStep& x, const DirectStep& y) { return x.rank < y.rank; });
+    std::vector<DirectJob> jobs[2];
+    for (uint32_t ph = 0; ph < 2 && !direct_steps_.empty(); ph++) {
+        jobs[ph].reserve(direct_steps_.size());
+        for (const DirectStep& st : direct_steps_) jobs[ph].push_back(direct_jobs_[ph][st.job]);
+        CSM_HIP(hipMemcpyAsync(d_direct_ + static_cast<uint64_t>(ph) * direct_cap_, jobs[ph].data(), jobs[ph].size() * sizeof(DirectJob),
+                               hipMemcpyHostToDevice, s_));
+    }
     CSM_HIP(hipStreamSynchronize(s_));
-    direct_stale_ = false;
     return "";
+}
+
+void Engine::direct_outcome(uint32_t q, uint32_t i, uint64_t edges, bool finished) {
+    DirectSeen& seen = direct_seen_[q * kMaxQE + i];
+    if (finished) {
+        if (edges >= seen.limit) seen.pause /= 2;
+        return;
+    }
+    seen.limit = seen.until > direct_seq_ ? std::min(seen.limit, edges) : edges;
+    seen.pause = seen.pause ? std::min(2 * seen.pause, kDirectPauseMax) : kDirectPause;
+    seen.until = direct_seq_ + seen.pause + 1;
+    direct_rank_at_ = 0;  // the table's order changes before the next phase
 }
 
 // Steps of the table's front that a phase of `edges` insertions or deletions and nsteps steps tries.  The
@@ -966,7 +993,7 @@ uint32_t Engine::direct_tries(uint64_t edges, uint32_t nsteps) const {
     const uint32_t lanes = static_cast<uint32_t>(lanes_.size());
     uint32_t n = 0;
     double work = 0;
-    while (n < direct_steps_.size() && direct_steps_[n].key * static_cast<double>(edges) <= 1.0) work += direct_steps_[n++].work * static_cast<double>(edges);
+    while (n < direct_steps_.size() && direct_steps_[n].rank * static_cast<double>(edges) <= 1.0) work += direct_steps_[n++].work * static_cast<double>(edges);
     auto groups = [&](uint32_t steps) { return (steps + lanes - 1) / lanes; };
     const uint32_t after = groups(nsteps - n) + (n == nsteps && work <= kDirectFew ? 0u : groups((n + 2) / 3));
     return after < groups(nsteps) ? n : 0u;
@@ -974,7 +1001,7 @@ uint32_t Engine::direct_tries(uint64_t edges, uint32_t nsteps) const {
 
 // Tries the first n direct steps of the phase on the main stream; done[q * kMaxQE + i] = 1 for every step
 // (q, i) that is finished, its counts in the results.  `others`: the phase's steps besides these n.
-std::string Engine::direct_phase(uint32_t ph, uint32_t n, uint32_t others, std::vector<char>& done) {
+std::string Engine::direct_phase(uint32_t ph, uint64_t edges, uint32_t n, uint32_t others, std::vector<char>& done) {
     for (uint32_t k = 0; k < n; k += kDirectJobs) {
         const uint32_t nj = std::min(kDirectJobs, n - k);
         uint32_t* at = direct_buf_;
@@ -1034,7 +1061,9 @@ std::string Engine::direct_phase(uint32_t ph, uint32_t n, uint32_t others, std::
         }
         for (uint32_t x = 0; x < nj; x++) {
             const uint32_t state = h_direct_state_[x];
-            if (!state) done[direct_steps_[k + x].q * kMaxQE + direct_steps_[k + x].i] = 1;
+            const DirectStep& st = direct_steps_[k + x];
+            if (!state) done[st.q * kMaxQE + st.i] = 1;
+            direct_outcome(st.q, st.i, edges, !state);
             direct_counts_.handed_on += handed[x];
             (state == 0 ? direct_counts_.finished : state == 1 ? direct_counts_.given_up : direct_counts_.left_over)++;
         }
@@ -1802,8 +1831,9 @@ std::string Engine::run_phase(uint32_t ph, uint64_t edges) {
     for (const auto& qs : qs_)
         if (qs->planned && qs->matchable) nsteps += qs->q.m;
     if (opt_.direct_steps && opt_.chain_levels && !opt_.graph_chains && !trace_ && !prof_mask_ && lanes_[0].ring_words >= kDirectRingWords) {
-        if (direct_stale_) {
-            std::string err = direct_tables();
+        direct_seq_++;
+        if (direct_stale_ || direct_rank_at_ <= direct_seq_) {
+            std::string err = direct_stale_ ? direct_tables() : direct_rank();
             if (!err.empty()) return err;
         }
         tries = direct_tries(edges, nsteps);
@@ -1814,7 +1844,7 @@ std::string Engine::run_phase(uint32_t ph, uint64_t edges) {
     direct_counts_.beside += beside;
     for (uint32_t k = 0; k < tries && beside; k++) finished[direct_steps_[k].q * kMaxQE + direct_steps_[k].i] = 1;
     if (tries && !beside) {
-        std::string err = direct_phase(ph, tries, nsteps - tries, finished);
+        std::string err = direct_phase(ph, edges, tries, nsteps - tries, finished);
         if (!err.empty()) return err;
     }
     for (size_t qi = 0; qi < qs_.size(); qi++) {
@@ -1961,7 +1991,7 @@ std::string Engine::run_phase(uint32_t ph, uint64_t edges) {
     std::string stage_err;
     if (beside) {
         for (uint32_t k = 0; k < tries; k++) finished[direct_steps_[k].q * kMaxQE + direct_steps_[k].i] = 0;
-        stage_err = direct_phase(ph, tries, nsteps - tries, finished);
+        stage_err = direct_phase(ph, edges, tries, nsteps - tries, finished);
         if (!stage_err.empty()) failed.store(true);
         std::vector<std::pair<uint32_t, uint32_t>> rest;
         for (uint32_t k = 0; k < tries; k++)
@@ -2347,6 +2377,8 @@ std::string Engine::snapshot() {
     }
     CSM_HIP(hipStreamSynchronize(s_));
     snap_top_ = top;
+    direct_seen_snap_ = direct_seen_;
+    direct_seq_snap_ = direct_seq_;
     return "";
 }
 
@@ -2373,6 +2405,10 @@ std::string Engine::restore() {
     std::memcpy(h_pinned_ + 64, &top, 8);
     CSM_HIP(hipMemcpyAsync(g_.arena_top, h_pinned_ + 64, 8, hipMemcpyHostToDevice, s_));
     CSM_HIP(hipStreamSynchronize(s_));
+    direct_seen_ = direct_seen_snap_;
+    direct_seen_.resize(qs_.size() * kMaxQE);
+    direct_seq_ = direct_seq_snap_;
+    direct_rank_at_ = 0;
     failed_.clear();
     return check_err("restore");
 }

@@ -82,6 +82,8 @@ constexpr uint32_t kMaxLanes = 64;
 constexpr uint32_t kDirectPairs = 2048;
 constexpr double kDirectTry = 2e5;
 constexpr double kDirectFew = 3e4;
+// Phases that a step is left out for after it failed, at first and at most.
+constexpr uint32_t kDirectPause = 8, kDirectPauseMax = 1024;
 // Rounds of a wave per task and pass (8: 0.87 ms for 32 queries and 1,024 edges, 16: 0.77, 24: 0.78),
 // candidates after which a step is given up, passes, tasks that a further pass is worth when the steps left
 // are one group of lanes (and when no more were to begin with), steps per launch, words of scratch, and the
@@ -342,17 +344,32 @@ class Engine {
     static int sched_of(SearchStrategy st);
     static uint32_t product_tail(const QState& qs, uint32_t i);
     static uint32_t level_target(const QState& qs, uint32_t i);
-    // Direct steps of the semi-BFS queries, the ones that are tried at the largest batches first, and the job
-    // tables of both phases in this order (rebuilt after a plan).
+    // Direct steps of the semi-BFS queries (rebuilt after a plan), the ones that are tried at the largest
+    // batches first, and the job tables of both phases in this order.
     struct DirectStep {
         uint32_t q, i;
         double anchors, work;  // expected anchors and tested candidates per edge of the phase
-        double key;            // 1 / the most edges at which the step is tried
+        double key;            // 1 / the most edges at which the step is expected to be small
+        double rank;           // 1 / the most edges at which it is tried
+        uint32_t job;          // its place in direct_jobs_
+    };
+    // The expectations are those of the graph that the session was built on, and the stream changes it: a step
+    // that did not finish in a phase of `limit` edges is not tried at as many again for `pause` phases (until
+    // phase `until`), twice as many each time it fails again.
+    struct DirectSeen {
+        uint64_t limit = 0, until = 0;
+        uint32_t pause = 0;
     };
     std::string direct_tables();
+    std::string direct_rank();
+    void direct_outcome(uint32_t q, uint32_t i, uint64_t edges, bool finished);
     uint32_t direct_tries(uint64_t edges, uint32_t nsteps) const;
-    std::string direct_phase(uint32_t ph, uint32_t n, uint32_t others, std::vector<char>& done);
+    std::string direct_phase(uint32_t ph, uint64_t edges, uint32_t n, uint32_t others, std::vector<char>& done);
     std::vector<DirectStep> direct_steps_;
+    std::vector<DirectJob> direct_jobs_[2];
+    std::vector<DirectSeen> direct_seen_, direct_seen_snap_;  // per q * kMaxQE + i; the latter as of the snapshot
+    uint64_t direct_seq_ = 0, direct_seq_snap_ = 0;  // phases that could try direct steps
+    uint64_t direct_rank_at_ = 0;        // the next of them that a pause ends at
     uint32_t* direct_buf_ = nullptr;     // [kDirectWords]
     DirectJob* d_direct_ = nullptr;      // [2][direct_cap_]
     uint32_t* h_direct_state_ = nullptr; // pinned [kDirectJobs + kDirectShards]

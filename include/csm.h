@@ -225,8 +225,9 @@ csm_status csm_profile_read(csm_session* s, uint32_t family, uint64_t* launches,
 /* Direct steps (no counterpart in the reference): under search strategy 2 a step that is expected to test few
  * candidates is searched depth-first from its update edges in an order of its own, without the
  * technique's matching order and local index, many such steps in one launch; a step that turns out
- * large is then run as the technique says.  Results are the same (the environment variable
- * CSM_DIRECT_STEPS=0 switches them off).  What became of the steps tried since csm_build_index: */
+ * large is then run as the technique says, and left out for the next batches of its size (8 phases, twice
+ * as many each time).  Results are the same (the environment variable CSM_DIRECT_STEPS=0 switches
+ * direct steps off).  What became of the steps tried since csm_build_index: */
 typedef struct {
     uint64_t tried;       /* finished + given_up + left_over */
     uint64_t finished;    /* counted by the direct search */

@@ -92,3 +92,30 @@ def test_more_steps_than_one_launch_takes(lib, tmp_path):  # noqa: F811
     c = run(lib, tmp_path, labels, start, held, gone, queries, (2,), lanes=64)
     assert c["tried"] == 2 * 110 * len(clique)  # both phases
     assert c["finished"] == c["tried"]
+
+
+def test_a_step_that_fails_is_left_out_for_a_while(lib, tmp_path):  # noqa: F811
+    """A step is expected to be small from the graph that the session was built on, where the hub has no vertex of
+    label 2; the stream's every edge then has 1,100 squared candidates behind it."""
+    leaves, batches = 1100, 12
+    labels = [0] + [1] * leaves + [2] * batches
+    write_graph(tmp_path / "data.graph", labels, [(0, v, 0) for v in range(1, leaves + 1)])
+    (tmp_path / "update.stream").write_text("".join(f"e 0 {leaves + 1 + k} 0\n" for k in range(batches)))
+    write_graph(tmp_path / "q.graph", [0, 2, 1, 1], [(0, 1, 0), (0, 2, 0), (0, 3, 0)], "t # 0\n")
+    want, _ = util.oracle_stream(tmp_path / "data.graph", tmp_path / "update.stream", 1, [tmp_path / "q.graph"], threads=8)
+    with lib.Session(device=0, ring_bytes=64 << 20, cp_list_bytes=32 << 20, lanes=4) as s:
+        s.load_graph(str(tmp_path / "data.graph"))
+        q = s.add_query(tmp_path / "q.graph")
+        assert s.open_updates(str(tmp_path / "update.stream"), 1) == batches
+        s.build()
+        s.plan(q)
+        s.snapshot()
+        failed = []
+        for _ in range(2):  # the restored session starts over
+            for b in range(batches):
+                assert tuple(s.apply_batch(b)[0][0]) == want[b, 0]
+                c = s.direct_counts()
+                failed.append(c["given_up"] + c["left_over"])
+            s.restore()
+    once = [1] * 9 + [2] * 3  # tried in the first phase, left out of eight, tried again
+    assert failed == once + [2 + k for k in once]
