@@ -22,6 +22,7 @@
 // neighbours' view runs; each is tested for its bit in the candidate bitmap, injectivity against the
 // matched prefix, and membership in every other backward neighbour's view run by binary search
 // (search.cuh:7-25 semantics).
+#include "dfs_grid.h"
 #include "kernels.h"
 #include "range_word.h"
 #include "view.h"
@@ -29,7 +30,7 @@
 namespace csm {
 namespace {
 
-constexpr uint32_t kWaves = 2;  // waves per block of the depth-first kernel (their LDS stacks stay under 64 KB at 16 depths)
+constexpr uint32_t kWaves = kDfsWaves;
 
 // Per-wave state of the depth-first search in LDS.  The wave searches batches of up to 64 partial
 // results: frame j extends its rows (partial results of depth d0 + j, at most one per lane) by the
@@ -380,7 +381,6 @@ __device__ __forceinline__ void dfs_pop(DfsHdr& H, DfsBuf* buf, uint32_t j, uint
 // depth in LDS.  Items (records, or chunks of records) are taken in groups of up to 64, sized so
 // that the grid has a few groups per resident wave.
 constexpr uint32_t kDfsGroupWaves = 2048;
-constexpr int kDfsGridWaves = 2048;
 template <int kMode>
 __global__ void __launch_bounds__(kWaves * 64) k_extend(DevGraph g, StepDesc d, uint32_t d0, uint32_t end_depth, Ring r, MatchOut out,
                                                          const unsigned long long* split, unsigned long long* work, int schedule,
@@ -1744,12 +1744,9 @@ void bitmap_to_list(const uint32_t* bitmap, uint32_t dv, uint32_t* list, uint32_
 
 void extend(const DevGraph& g, const StepDesc& d, uint32_t d0, uint32_t end_depth, int mode, Ring r, MatchOut out,
             const unsigned long long* split, unsigned long long* work_counter, int schedule, int blocks, Donation dn, hipStream_t s) {
-    // Persistent grid: 4 * `blocks` waves, at most the kDfsGridWaves that are resident when two launches
-    // share the chip (waves that start when the items are used up only contend for them), never
-    // more than records (a split launch has at least as many items as records with candidates; a
-    // donating launch keeps the full grid, its waves share the heavy records' ranges).
-    blocks = std::min<int>(std::min<int>(blocks, static_cast<int>(kMaxDfsBlocks)) * 4, kDfsGridWaves) / static_cast<int>(kWaves);
-    const int grid = split || schedule == 2 ? blocks : grid_for(r.in_max, kWaves, blocks);
+    // Persistent grid, never more waves than records (a split launch has at least as many items as records
+    // with candidates; a donating launch keeps the full grid, its waves share the heavy records' ranges).
+    const uint32_t grid = dfs_grid(static_cast<uint32_t>(blocks), r.in_max, split || schedule == 2);
     const size_t lds = static_cast<size_t>(kWaves) * wave_lds_bytes(d0, end_depth);
     if (schedule == 2) fill_u32(reinterpret_cast<uint32_t*>(dn.words), 0u, 4ull * grid * kWaves, s);  // every pair: nothing to take
     if (mode == kCountAtEnd)

@@ -228,10 +228,9 @@ void bitmap_to_list(const uint32_t* bitmap, uint32_t dv, uint32_t* list, uint32_
 
 enum ExtendMode : int { kCountAtEnd = 0, kWriteAtEnd = 1 };
 // Range donation of the depth-first kernel (schedule 2): a range word and a frame word per wave of the
-// launch (kMaxDfsBlocks * 4 waves at most); extend clears them before the launch.
-constexpr uint32_t kMaxDfsBlocks = 16384;
+// launch; extend clears them before the launch.
 struct Donation {
-    unsigned long long* words;  // [kMaxDfsBlocks * 4][2]
+    unsigned long long* words;  // [kMaxDfsBlocks * kDfsWaves][2]
 };
 // DFS from the records at depth d0 down to end_depth: counts/hashes complete embeddings when
 // end_depth == n, or writes the partial results of depth end_depth to the ring.
@@ -240,7 +239,7 @@ struct Donation {
 // first-depth candidate range another wave is still exploring (dn).  Without `split` an item is one record.  With `split` (the exclusive scan of
 // root_chunks, total at [n]) an item is one of a record's k chunks: its depth-d0 candidates cut
 // into k equal pieces of whole 64-candidate rounds, so a heavy record spreads over k waves.
-// blocks: the persistent grid (fewer when there are fewer items).
+// blocks: the persistent grid, kDfsWaves waves each (fewer when there are fewer items).
 void extend(const DevGraph& g, const StepDesc& d, uint32_t d0, uint32_t end_depth, int mode, Ring r,
             MatchOut out, const unsigned long long* split, unsigned long long* work_counter, int schedule, int blocks, Donation dn,
             hipStream_t s);

@@ -257,7 +257,7 @@ std::string Engine::build() {
         add(cp_list_words * 4); add(64);
         add(64 << 10);                                             // alignment slack of the takes
         add(sizeof(ChainJob) + 256);                               // the lane's level-chain job
-        add(kMaxDfsBlocks * 4ull * 16 + 512);                      // range donation words
+        add(kMaxDfsBlocks * kDfsWaves * 16ull + 512);              // range donation words
         add(kLaneWords * 4 + sizeof(AnchorJob) + sizeof(InitJob) + kMaxQV * (sizeof(LocalJob) + sizeof(VSet)) + 2 * kMaxQV * 4 + 1024);  // team jobs
     }
     // local-index slots: two groups of group_ steps (each: its sets, anchor pairs, queue, counters)
@@ -490,7 +490,7 @@ std::string Engine::build() {
         uint4* level_runs = pool_.take<uint4>(kLevelRunsPerRecord * cp_rec);
         unsigned long long* tile_sum = pool_.take<unsigned long long>(cp_rec / kLevelTile + 2);
         w.chain_ctr = chain_ctr_all_ + static_cast<uint64_t>(&w - lanes_.data()) * 2 * kMaxQV;
-        w.dn.words = pool_.take<unsigned long long>(kMaxDfsBlocks * 8ull);
+        w.dn.words = pool_.take<unsigned long long>(kMaxDfsBlocks * kDfsWaves * 2ull);
         if (!w.dn.words) return tagged(Code::kMemory, "device pool exhausted (lane scratch)");
         if (!level_runs || !tile_sum || !w.chain_ctr) return tagged(Code::kMemory, "device pool exhausted (lane scratch)");
         w.level = LevelScratch{w.cp.prod, w.cp.seg_run, level_runs, reinterpret_cast<uint8_t*>(w.cp.seg_cnt), w.cp.rec_hash,

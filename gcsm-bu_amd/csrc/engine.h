@@ -24,6 +24,7 @@
 
 #include "../../include/csm.h"
 #include "common/errors.h"
+#include "device/dfs_grid.h"
 #include "device/kernels.h"
 #include "host/graph_io.h"
 #include "host/plan.h"
@@ -52,7 +53,7 @@ struct EngineOptions {
     // Launch settings that change scheduling only, never results (Tunables):
     uint32_t waves_per_anchor = 1024; // most waves one record of the counting DFS is split over (1: no split)
     uint32_t stack_depth = kMaxQV;    // most LDS stack rows of a counting DFS launch; deeper searches run levels first
-    uint32_t dfs_blocks = 2048;       // blocks of the persistent DFS grid
+    uint32_t dfs_blocks = kDfsBlocks; // blocks of the persistent DFS grid
     uint32_t level_blocks = 384;      // blocks per step of a team's multi-step level kernels
     bool slot_directory = true;       // per-vertex label-slot offsets (when they fit kMaxSlotDirectoryBytes)
     bool chain_levels = true;         // semi-BFS levels of a step chained on the device (one host wait per step)

@@ -184,7 +184,7 @@ typedef struct {
     uint32_t stack_depth;        /* depth-first counting: most LDS stack rows (depths below the first) one
                                     launch descends; deeper searches run breadth-first levels first
                                     (1..16, default 16) */
-    uint32_t dfs_blocks;         /* blocks of the persistent depth-first grid (64..16384, default 2048) */
+    uint32_t dfs_blocks;         /* blocks of the persistent depth-first grid, two waves each (64..16384, default 1024) */
     uint32_t local_blocks;       /* blocks of the local-index kernels (16..2048; default 512 for batches of
                                     2^18 edges or more, else 256) */
     uint32_t team;               /* lanes per team (1..64, default a quarter of the lanes, so four teams, one per
