@@ -26,7 +26,8 @@ ORACLE = os.path.join(ROOT, "oracle", "bin", "oracle")
 METRIC = "incremental matches/s & update edges/s on 1 GPU; p50/p99 batch latency"
 HBM_PEAK_GBS = 8000.0
 FAMILIES = ["enumerate_count", "enumerate_write", "cartesian_product", "local_index", "batch_build", "apply_batch",
-            "cartesian_prepare", "anchors", "level_count", "level_write", "level_prepare", "local_check", "merge_insert"]
+            "cartesian_prepare", "anchors", "level_count", "level_write", "level_prepare", "local_check", "merge_insert",
+            "direct_steps"]
 # families whose kernels count algorithmic bytes on the device (the roofline candidates)
 BYTE_FAMILIES = ["enumerate_count", "enumerate_write", "level_count", "level_write", "local_index", "local_check",
                  "merge_insert"]

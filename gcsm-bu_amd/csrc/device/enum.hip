@@ -242,7 +242,7 @@ __device__ __forceinline__ uint32_t dfs_rows(const DevGraph& g, const StepDesc& 
                 best = l;
                 gen = e;
             }
-            if (count_bytes && (j || H.chunk[lane] == 0)) row_bytes += 4ull * ((rv[e].hi - rv[e].lo) + (rv[e].dhi - rv[e].dlo));
+            if (count_bytes && (j || (kRanged ? H.chunks[lane] == 0xFFFFFFFFu : H.chunk[lane] == 0))) row_bytes += 4ull * ((rv[e].hi - rv[e].lo) + (rv[e].dhi - rv[e].dlo));
         }
         H.gen[lane] = gen;
         len = best;
@@ -693,7 +693,8 @@ __global__ void __launch_bounds__(kWaves * 64) k_direct_search(DevGraph g, const
         DirectCtr& C = ctr[job];
         const StepDesc& d = jobs[job].d;
         if (!rows0 || uniform(__hip_atomic_load(&C.fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) continue;
-        unsigned long long my_cnt = 0, my_hash = 0, no_bytes = 0;
+        unsigned long long my_cnt = 0, my_hash = 0, my_bytes = 0;
+        const bool count_bytes = q.bytes != nullptr;  // of rows that are new: the pieces of a row are counted with the row
         if (kFirst && d.n == 2) {
             if (lane < rows0) {
                 const uint32_t* r = in + 2 * (t * G + lane);
@@ -705,7 +706,7 @@ __global__ void __launch_bounds__(kWaves * 64) k_direct_search(DevGraph g, const
             DfsBuf* const buf = reinterpret_cast<DfsBuf*>(wave_base + sizeof(DfsHdr) + (d.n - 1) * 256u);
             const uint32_t last = d.n - 1 - depth0;
             uint32_t j = 0, built = 0, rounds = 0, state = 0;  // state 1: hand the rest on, 2: given up
-            const uint32_t total0 = dfs_rows<true>(g, d, depth0, 0, rows0, in, stride, H, f, buf, lane, no_bytes, false);
+            const uint32_t total0 = dfs_rows<true>(g, d, depth0, 0, rows0, in, stride, H, f, buf, lane, my_bytes, count_bytes);
             if (total0 > kFrameMax) state = 2;  // far more than a step may have
             unsigned long long work = total0;
             if (lane == 0) {
@@ -739,7 +740,7 @@ __global__ void __launch_bounds__(kWaves * 64) k_direct_search(DevGraph g, const
                 if (down) {  // descend with a batch
                     uint32_t rows = min(64u, waiting);
                     j += 1;
-                    const uint32_t tj = dfs_rows<true>(g, d, depth0, j, rows, in, stride, H, f, buf, lane, no_bytes, false);
+                    const uint32_t tj = dfs_rows<true>(g, d, depth0, j, rows, in, stride, H, f, buf, lane, my_bytes, count_bytes);
                     if (tj > kFrameMax) state = 2;
                     work += tj;
                     built = j;
@@ -754,7 +755,7 @@ __global__ void __launch_bounds__(kWaves * 64) k_direct_search(DevGraph g, const
                 }
                 if (built != j) {
                     uint32_t rows = uniform(H.rows[j]);
-                    dfs_rows<true>(g, d, depth0, j, rows, in, stride, H, f, buf, lane, no_bytes, false);
+                    dfs_rows<true>(g, d, depth0, j, rows, in, stride, H, f, buf, lane, my_bytes, false);
                     built = j;
                 }
                 const uint32_t depth = depth0 + j;
@@ -762,6 +763,8 @@ __global__ void __launch_bounds__(kWaves * 64) k_direct_search(DevGraph g, const
                 bool ok[kDfsIlp];
                 dfs_round(g, d, depth, cur, tot, H, f, lane, k, c, ok);
                 if (lane == 0) H.cur[j] = cur + 64 * kDfsIlp;
+                if (count_bytes)
+                    for (uint32_t u = 0; u < kDfsIlp; u++) my_bytes += ok[u] ? 4u : 0u;
                 if (j < last) {
                     uint32_t at = waiting;
 #pragma unroll
@@ -793,7 +796,7 @@ __global__ void __launch_bounds__(kWaves * 64) k_direct_search(DevGraph g, const
                     uint32_t rows = uniform(H.rows[jj]);
                     const uint32_t cur = uniform(H.cur[jj]), tot = uniform(H.tot[jj]), depth = depth0 + jj;
                     if (built != jj) {
-                        dfs_rows<true>(g, d, depth0, jj, rows, in, stride, H, f, buf, lane, no_bytes, false);
+                        dfs_rows<true>(g, d, depth0, jj, rows, in, stride, H, f, buf, lane, my_bytes, false);
                         built = jj;
                     }
                     const uint32_t pre = H.pre[lane], end = lane < 63 ? H.pre[lane + 1] : tot, from = max(cur, pre);
@@ -829,6 +832,10 @@ __global__ void __launch_bounds__(kWaves * 64) k_direct_search(DevGraph g, const
         my_cnt = wave_sum_u64(my_cnt);
         my_hash = wave_sum_u64(my_hash);
         if (lane == 0 && my_cnt) { atomicAdd(&C.count, my_cnt); atomicAdd(&C.hash, my_hash); }
+        if (count_bytes) {
+            my_bytes = wave_sum_u64(my_bytes);
+            if (lane == 0 && my_bytes) atomicAdd(q.bytes, my_bytes);
+        }
     }
 }
 

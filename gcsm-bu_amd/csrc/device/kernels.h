@@ -281,6 +281,7 @@ struct DirectQueue {           // kDirectShards queues of cap tasks and cap item
     uint32_t cap, stride;            // words per item
     uint32_t pass;
     uint32_t wave_lds;               // direct_wave_lds of the largest query
+    unsigned long long* bytes;       // += algorithmic bytes (may be null)
 };
 uint32_t direct_wave_lds(uint32_t max_qn);
 void direct_search(const DevGraph& g, const DirectJob* jobs, uint32_t njobs, DirectCtr* ctr, const uint32_t* pairs, uint32_t cap,

@@ -1025,6 +1025,7 @@ std::string Engine::direct_phase(uint32_t ph, uint64_t edges, uint32_t n, uint32
         for (int x = 0; x < 2; x++) tasks[x] = reinterpret_cast<uint4*>(take(4ull * kDirectShards * q.cap));
         for (int x = 0; x < 2; x++) items[x] = take(static_cast<uint64_t>(q.stride) * kDirectShards * q.cap);
         q.wave_lds = direct_wave_lds(direct_qn_);
+        q.bytes = bytes_ptr(kKDirect);
         const DirectJob* jobs = d_direct_ + static_cast<uint64_t>(ph) * direct_cap_ + k;
         auto pass = [&](uint32_t p) {
             q.in_n = qn + (p - 1) * kDirectShards * 16;  // not read by pass 0
@@ -1034,10 +1035,14 @@ std::string Engine::direct_phase(uint32_t ph, uint64_t edges, uint32_t n, uint32
             q.out_tasks = tasks[p & 1];
             q.out_items = items[p & 1];
             q.pass = p;
+            prof_begin(prof_main_, s_, kKDirect);
             direct_search(g_, jobs, nj, ctr, pairs, cap, q, kDirectRounds, kDirectWork, s_);
+            prof_end(prof_main_, s_, kKDirect);
         };
         fill_u32(direct_buf_, 0u, zero, s_);
+        prof_begin(prof_main_, s_, kKAnchors);
         direct_anchors(g_, jobs, nj, ctr, pairs, cap, bs_[0].by_label, bs_[0].label_off, bs_[1].by_label, bs_[1].label_off, batch_arcs_, s_);
+        prof_end(prof_main_, s_, kKAnchors);
         const uint32_t behind = others + (n - k - nj);  // steps not in this launch
         const uint32_t small = n + others <= lanes_.size() ? kDirectTailFew : kDirectTail;
         std::vector<char> handed(nj, 0);
@@ -1830,7 +1835,9 @@ std::string Engine::run_phase(uint32_t ph, uint64_t edges) {
     uint32_t nsteps = 0, tries = 0;
     for (const auto& qs : qs_)
         if (qs->planned && qs->matchable) nsteps += qs->q.m;
-    if (opt_.direct_steps && opt_.chain_levels && !opt_.graph_chains && !trace_ && !prof_mask_ && lanes_[0].ring_words >= kDirectRingWords) {
+    // a profile without the direct family is of the other kernels: they then run every step
+    const bool profiled = prof_mask_ && !(prof_mask_ >> kKDirect & 1u);
+    if (opt_.direct_steps && opt_.chain_levels && !opt_.graph_chains && !trace_ && !profiled && lanes_[0].ring_words >= kDirectRingWords) {
         direct_seq_++;
         if (direct_stale_ || direct_rank_at_ <= direct_seq_) {
             std::string err = direct_stale_ ? direct_tables() : direct_rank();

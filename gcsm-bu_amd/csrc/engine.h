@@ -230,7 +230,8 @@ class Engine {
 
     // Kernel families timed with HIP events on the engine's stream when profiling is enabled.
     enum KernelFamily : uint32_t { kKExtendCount = 0, kKExtendWrite, kKCpEnumerate, kKLocalIndex, kKBatchBuild, kKApply, kKCpPrepare,
-                                   kKAnchors, kKLevelCount, kKLevelWrite, kKLevelPrepare, kKLocalCheck, kKMergeInsert, kKFamilies };
+                                   kKAnchors, kKLevelCount, kKLevelWrite, kKLevelPrepare, kKLocalCheck, kKMergeInsert, kKDirect,
+                                   kKFamilies };
     struct KernelStat {
         uint64_t launches = 0;
         double ms = 0;

@@ -119,3 +119,39 @@ def test_a_step_that_fails_is_left_out_for_a_while(lib, tmp_path):  # noqa: F811
             s.restore()
     once = [1] * 9 + [2] * 3  # tried in the first phase, left out of eight, tried again
     assert failed == once + [2 + k for k in once]
+
+
+@pytest.mark.parametrize("leaves", [20, 100])  # searched in one pass, handed on
+def test_profile_sees_the_direct_search(lib, tmp_path, leaves):  # noqa: F811
+    """Family 13 times the search passes and counts their algorithmic bytes (every row's list once, however often the
+    row is handed on, and 4 per vertex found); a mask without it shows all steps in the other families."""
+    labels = [0] + [1] * leaves + [2, 2]
+    write_graph(tmp_path / "data.graph", labels, [(0, v, 0) for v in range(1, leaves + 2)])
+    (tmp_path / "update.stream").write_text(f"e 0 {leaves + 2} 0\n")
+    write_graph(tmp_path / "q.graph", [0, 2, 1, 1], [(0, 1, 0), (0, 2, 0), (0, 3, 0)], "t # 0\n")
+    with lib.Session(device=0, ring_bytes=64 << 20, cp_list_bytes=32 << 20, lanes=4) as s:
+        s.load_graph(str(tmp_path / "data.graph"))
+        q = s.add_query(tmp_path / "q.graph")
+        s.open_updates(str(tmp_path / "update.stream"), 1)
+        s.build()
+        s.plan(q)
+        s.snapshot()
+        got = {}
+        for mask in (1 << 13, 1 << 8 | 1 << 9, 0):
+            s.profile_enable(mask)
+            tried = s.direct_counts()["tried"]
+            got[mask] = s.apply_batch(0)[0][0], s.direct_counts()["tried"] - tried
+            if mask:
+                launches = {f: s.profile_read(f) for f in range(14)}
+                if mask >> 13:
+                    assert all((n > 0) == (f == 13) for f, (n, _, _) in launches.items())
+                    assert launches[13][1] > 0
+                    c = s.direct_counts()
+                    assert c["finished"] == c["tried"] == 3 and (c["handed_on"] > 0) == (leaves == 100)
+                    assert launches[13][2] == 4 * (leaves + leaves + leaves * leaves + leaves * (leaves - 1))
+                else:
+                    assert launches[13][0] == 0 and launches[8][0] + launches[9][0] > 0
+            s.restore()
+        assert got[1 << 13] == got[0] and got[0][1] == 3
+        assert got[1 << 8 | 1 << 9] == (got[0][0], 0)
+        assert got[0][0][0] == leaves * (leaves - 1)
