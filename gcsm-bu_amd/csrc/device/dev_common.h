@@ -98,8 +98,8 @@ struct StepDesc {
 
 // A pointer that was read from memory (a job table, LDS) as one to global memory.  The compiler takes it for
 // a generic one otherwise, and flat accesses count as LDS accesses too: every wait for one of them
-// also waits for the other kind.  Kernel arguments need no help.  (Round trips with the multi-step
-// kernels' pointers: large skewed graph 57.0 -> 54.3 ms, 263K-vertex stream 7.07 -> 6.77 ms.)
+// also waits for the other kind.  Kernel arguments need no help.  (Round trips without and with it,
+// in turn on one card: large skewed graph 45.9, 44.6 ms; 64 queries 42.0, 40.9; 400K-vertex stream 7.38, 7.25.)
 template <typename T>
 __device__ __forceinline__ T* as_global(T* p) {
     return (T*)((__attribute__((address_space(1))) T*)reinterpret_cast<uint64_t>(p));  // a cast of the pointer itself would be folded away

@@ -601,9 +601,9 @@ __global__ void __launch_bounds__(kWaves * 64) k_extend(DevGraph g, StepDesc d, 
 // left after the last pass) is given up: nothing of it is counted, and the host runs it with its local
 // index and levels.  The search is bound by the latency of its rounds (about 10 us each: row lookups, a
 // list element, the bitmap, binary searches); what it saves is the launches, gaps and host waits of the
-// other path, about 30 launches of 3 to 20 us per group of lanes.  Round trips: 32 queries, 1,024-edge
-// batches 5.2 -> 0.77 ms, 2K to 64K edges 46 -> 10.1 ms; one query on the 10K-vertex graph 1.20 -> 0.71 ms;
-// 64 queries, 65,536 edges 58.5 -> 48.3 ms.
+// other path, about 30 launches of 3 to 20 us per group of lanes.  Round trips without and with direct
+// steps: 32 queries, 1,024-edge batches 4.7, 0.91 ms, 2K to 64K edges 45.5, 10.0 ms; 64 queries, 65,536 edges
+// 58.4, 45.9 ms.
 constexpr uint32_t kDirectPoll = 8;     // rounds between looks at the step's state
 constexpr uint32_t kDirectTask = 16;    // items per task
 constexpr uint32_t kDirectPiece = 512;  // candidates of one row per item

@@ -77,13 +77,15 @@ constexpr uint32_t kMaxLanes = 64;
 // Direct steps (kernels.h).  A step is tried when its query edge is expected to have at most kDirectPairs
 // anchors in the batch and its search kDirectTry candidates; where one group of lanes would do for all
 // steps, when all of them together are expected to test at most kDirectFew (else a try that fails costs
-// more than it saves: 20 steps 2.9 -> 3.1 ms).  Measured per round trip against kDirectTry: 32 queries,
-// 1K to 64K edges 16.0 ms at 3e3, 14.1 at 1e4, 10.5 at 5e4, 10.2 at 2e5 (46 without direct steps); 64
-// queries, 64K edges 59.0, 55.5, 48.6, 48.1 (58.5 without).
+// more than it saves: 20 steps 2.9 -> 3.1 ms).  Measured per round trip against kDirectTry, with steps that
+// fail left out (kDirectPause): 32 queries, 2K to 64K edges 14.8 ms at 3e3, 12.0 at 1e4, 10.0 at 5e4 and 2e5
+// (45.5 without direct steps); 64 queries, 64K edges 57.7, 54.5, 49.1, 45.9 (58.4 without).
 constexpr uint32_t kDirectPairs = 2048;
 constexpr double kDirectTry = 2e5;
 constexpr double kDirectFew = 3e4;
-// Phases that a step is left out for after it failed, at first and at most.
+// Phases that a step is left out for after it failed, at first and at most: a failed try costs its passes and
+// their waits (64 queries, on another card: 268 of 1,154 tries a round trip failed, 43.9 ms; left out 40.0), a step
+// left out needlessly only its share of a group.
 constexpr uint32_t kDirectPause = 8, kDirectPauseMax = 1024;
 // Rounds of a wave per task and pass (8: 0.87 ms for 32 queries and 1,024 edges, 16: 0.77, 24: 0.78),
 // candidates after which a step is given up, passes, tasks that a further pass is worth when the steps left
